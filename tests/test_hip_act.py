@@ -144,3 +144,50 @@ def test_rmsnorm_matches_reference_engine_goldens(hip, engine_golden):
         d80 = hip.alloc(rows * (cols // 32) * 36)
         hip.rmsnorm_prepare_dev(dx, 0, dw, float(engine_golden[f"rms/{c}/eps"][0]), rows, cols, dxn, 0, d80, 0, None, 0)
         assert np.array_equal(bits(hip.download(dxn, np.zeros_like(x))), bits(engine_golden[f"rms/{c}/o"])), c
+
+
+def _hard_sum_rows(cols, rng):
+    """rows on which the order and the ties of rmsnorm's double sum show: small integers, magnitudes all over, powers of two
+    (binade edges), an outlier, terms near half a unit of the sum, infinities and NaN, and a row whose small terms are all
+    lost in order but not when they are added among themselves (the parallel sum has to notice and add in order)"""
+    n = rng.standard_normal(cols).astype(np.float32)
+    rows = [np.trunc(4 * n), np.ldexp(n, rng.integers(-40, 40, cols)), np.ldexp(np.float32(1), rng.integers(0, 6, cols))]
+    r = n.copy()
+    r[cols // 2] = 3e4
+    rows.append(r)
+    r = np.ldexp(n, -26)
+    r[: cols // 3] = 0.0
+    r[cols // 3] = 1.0
+    rows.append(r)
+    for bad in (np.inf, -np.inf, np.nan):
+        r = n.copy()
+        r[cols // 3] = bad
+        rows.append(r)
+    r, left = np.full(cols, 2.0 ** -28, np.float32), 1.0 - 2.0 ** -53   # 2^-56 a term, half a unit is 2^-54
+    for i in range(min(cols, 16)):
+        v = np.float32(np.sqrt(left))
+        while float(v) ** 2 > left:
+            v = np.nextafter(v, np.float32(0))
+        r[i] = v
+        left -= float(v) ** 2
+    rows.append(r)
+    return np.stack([np.asarray(v, np.float32) for v in rows])
+
+
+@pytest.mark.parametrize("cols", [32, 480, 512, 544, 2048, 8192, 8224, 16384])
+def test_rmsnorm_sum_order(hip, orc, cols):
+    """the in-order double sum at the wave and pass edges of the parallel kernel; in place (xn = x) too"""
+    rng = np.random.default_rng(cols + 7)
+    x = _hard_sum_rows(cols, rng)
+    want = orc.rmsnorm(x, None, 1e-6)
+    rows = x.shape[0]
+    dx = hip.upload(x)
+    d80 = hip.alloc(rows * (cols // 32) * 36)
+    hip.rmsnorm_prepare_dev(dx, 0, None, 1e-6, rows, cols, dx, 0, d80, 0, None, 0)
+    got = hip.download(dx, np.zeros_like(x))
+    for i in range(rows):
+        same = (bits(got[i]) == bits(want[i])) | (np.isnan(got[i]) & np.isnan(want[i]))
+        assert same.all(), (cols, i, got[i][~same][:4], want[i][~same][:4])
+    finite = [i for i in range(rows) if np.isfinite(want[i]).all()]
+    g80 = hip.download(d80, np.zeros((rows, (cols // 32) * 36), np.uint8))
+    assert np.array_equal(g80[finite], blocks(orc, want[finite], "q80"))
