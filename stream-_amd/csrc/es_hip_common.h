@@ -58,7 +58,11 @@ struct MvLaunch {
     size_t lds;
     bool seg_loop = false;   // some row of the launch needs more than `waves` block groups (each wave takes several)
 };
-hipError_t mv_launch(const MvLaunch &L, const MvJob *jobs, int njobs, const MvJob &single, int order, hipStream_t s);
+// jobs: the launch's job table on the device, or null: the njobs <= MV_INLINE jobs at hjobs travel with the launch itself
+// (one grid row per job, its record read from the kernel's arguments), so a small batch needs no table, no upload and no
+// read of one before its first load. Launches of mixed pass widths (nt 0) take a table.
+constexpr int MV_INLINE = 4;
+hipError_t mv_launch(const MvLaunch &L, const MvJob *jobs, int njobs, const MvJob *hjobs, int order, hipStream_t s);
 
 // Batched 32-wide form (Q4_0 / Q5_0, es_hip_mv.hip): rows [r0, r1) against activations [t0, t0 + ta) of na, one lane per
 // (row, activation); ta is a power of two <= 64 and a workgroup of 4 waves covers 4 * 64 / ta rows.

@@ -20,6 +20,8 @@
 // 1443-1469 (AVX2 Q4_0/Q5_0/Q4_K/Q6_K), 1344-1368 and src/es_q2k.c:127-190 (Q2_K), 1120-1175 and 1370-1394 (Q3_K, Q5_K).
 #include "es_hip_common.h"
 
+#include <type_traits>
+
 
 // units (one block position of one row each) whose raw loads a wave issues before using any of them; a power of two
 #ifndef ESQ_UNITS
@@ -534,6 +536,7 @@ __device__ __forceinline__ void mv_body(const MvJob &J, int order) {
     const int tile = blockIdx.x - J.tile0;
     const int ra0 = J.r0 + tile * J.rows_per_wg;
     const int rend = min(ra0 + J.rows_per_wg, J.r1);
+    if (ra0 >= rend) return;   // uniform over the workgroup
     const uint8_t *const dummy = J.W + (size_t)J.r0 * J.row_bytes;   // a valid block for lanes with nothing to load
 
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
@@ -566,7 +569,7 @@ __device__ __forceinline__ void mv_body(const MvJob &J, int order) {
     // the first unit batch's weight loads go out before the activation loads, so their latencies overlap (Q4_K at one
     // activation per pass; elsewhere keeping these registers live across the activation loads cost more than it saved)
     constexpr bool PRE = NT == 1 && F == ES_HIP_Q4_K;
-    bool pre = PRE && ra0 < rend;
+    bool pre = PRE;
     if (pre) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
@@ -692,16 +695,47 @@ __device__ __forceinline__ void mv_body(const MvJob &J, int order) {
                         s = cmode == CH_LANES ? ldg<float>(J.lanes + lane_at) : ldg<float>(J.y + (size_t)(t0 + t) * J.ystride + ra + rl);
                 }
                 int bb = 0;
-                for (; bb + 8 <= nbk; bb += 8) {
-                    float ta[8], tb[8];
+                if constexpr (W32 && NT == 1) {   // rows of many blocks: the next eight terms' reads in flight under the chain
+                    const int full = nbk & ~7;    // (every read unconditional, the last group's repeated: a branch would wait
+                    if (full) {                   // for them all)
+                        float ta[8], tb[8], ua[8], ub[8];
+                        auto fetch = [&](int b0, float (&fa)[8], float (&fb)[8]) {
 #pragma unroll
-                    for (int q = 0; q < 8; q++) { ta[q] = e[(bb + q) * NT * CW + oa]; tb[q] = e[(bb + q) * NT * CW + ob]; }
-                    if (cmode == CH_MULADD) {
+                            for (int q = 0; q < 8; q++) { fa[q] = e[(b0 + q) * CW + oa]; fb[q] = e[(b0 + q) * CW + ob]; }
+                        };
+                        auto add = [&](const float (&fa)[8], const float (&fb)[8]) {
+                            if (cmode == CH_MULADD) {
 #pragma unroll
-                        for (int q = 0; q < 8; q++) s = s + ta[q] * tb[q];   // -ffp-contract=off: two roundings
-                    } else {
+                                for (int q = 0; q < 8; q++) s = s + fa[q] * fb[q];
+                            } else {
 #pragma unroll
-                        for (int q = 0; q < 8; q++) s = __builtin_fmaf(ta[q], tb[q], s);
+                                for (int q = 0; q < 8; q++) s = __builtin_fmaf(fa[q], fb[q], s);
+                            }
+                        };
+                        fetch(0, ta, tb);
+                        for (; bb + 16 <= full; bb += 16) {
+                            fetch(bb + 8, ua, ub);
+                            add(ta, tb);
+                            fetch(min(bb + 16, full - 8), ta, tb);
+                            add(ua, ub);
+                        }
+                        if (bb < full) {
+                            add(ta, tb);
+                            bb += 8;
+                        }
+                    }
+                } else {
+                    for (; bb + 8 <= nbk; bb += 8) {
+                        float ta[8], tb[8];
+#pragma unroll
+                        for (int q = 0; q < 8; q++) { ta[q] = e[(bb + q) * NT * CW + oa]; tb[q] = e[(bb + q) * NT * CW + ob]; }
+                        if (cmode == CH_MULADD) {
+#pragma unroll
+                            for (int q = 0; q < 8; q++) s = s + ta[q] * tb[q];   // -ffp-contract=off: two roundings
+                        } else {
+#pragma unroll
+                            for (int q = 0; q < 8; q++) s = __builtin_fmaf(ta[q], tb[q], s);
+                        }
                     }
                 }
                 for (; bb < nbk; bb++) {
@@ -726,24 +760,48 @@ __device__ __forceinline__ void mv_body(const MvJob &J, int order) {
     }
 }
 
+// The kernels' arguments, as one block (their first and only parameter, at offset 0 of the argument segment).
+struct MvArgs {
+    const MvJob *jobs;   // the launch's job table, or null: grid row i runs j[i], tiles numbered from 0
+    int njobs, order;
+    MvJob j[MV_INLINE];
+};
+// this workgroup's job. In-argument jobs are read at the grid row's offset of the argument segment, in the round trip that
+// brings the arguments themselves (a select among the four records loaded them all: 0.6 us a launch).
+__device__ __forceinline__ MvJob mv_job(const MvArgs &A) {
+    static_assert(sizeof(MvJob) % 4 == 0 && offsetof(MvArgs, j) % 4 == 0, "jobs are read as dwords");
+    constexpr int N = sizeof(MvJob) / 4;
+    uint32_t v[N];
+    if (A.jobs) {
+        const MvJob J = load_tile_job(A.jobs, A.njobs, blockIdx.x);
+        __builtin_memcpy(v, &J, sizeof J);
+    } else {
+        typedef const __attribute__((address_space(4))) uint32_t *ArgPtr;
+        const ArgPtr src = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(MvArgs, j) / 4 + blockIdx.y * N;
+#pragma unroll
+        for (int i = 0; i < N; i++) v[i] = src[i];
+    }
+    // scalar registers on both paths: the compiler otherwise merges the two records in vector registers (17 to 28 more of
+    // them, which cost the multi-activation bodies a wave per SIMD)
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)v[i]);
+    return __builtin_bit_cast(MvJob, v);
+}
+
 template <int F, int NT, int W, bool SEGLOOP>
-__global__ __launch_bounds__(WAVE * W, ESQ_MIN_WAVES) void mv_kernel(const MvJob *__restrict__ jobs, int njobs, MvJob single,
-                                                                     int order) {
-    MvJob J;
-    if (jobs) J = load_tile_job(jobs, njobs, blockIdx.x);
-    else J = single;
-    mv_body<F, NT, W, SEGLOOP>(J, order);
+__global__ __launch_bounds__(WAVE * W, ESQ_MIN_WAVES) void mv_kernel(MvArgs A) {
+    const MvJob J = mv_job(A);
+    mv_body<F, NT, W, SEGLOOP>(J, A.order);
 }
 
 // A launch whose jobs take different activations per pass (J.nt: 1, 2 or 4), e.g. an MoE layer's experts at 1 to 8
 // tokens each: every job runs the body compiled for its own pass width (a single expert's token no longer runs in a
 // four-wide pass with its fewer loads in flight).
+// Always from the table: its launches are long job lists, and its registers have no room for a second source of the job
+// (config 5's layer 139 -> 144 us with mv_job).
 template <int F, int W, bool SEGLOOP>
-__global__ __launch_bounds__(WAVE * W, ESQ_MIN_WAVES) void mv_kernel_mixed(const MvJob *__restrict__ jobs, int njobs,
-                                                                           MvJob single, int order) {
-    MvJob J;
-    if (jobs) J = load_tile_job(jobs, njobs, blockIdx.x);
-    else J = single;
+__global__ __launch_bounds__(WAVE * W, ESQ_MIN_WAVES) void mv_kernel_mixed(const MvJob *__restrict__ jobs, int njobs, int order) {
+    const MvJob J = load_tile_job(jobs, njobs, blockIdx.x);
     switch (J.nt) {
     case 1: mv_body<F, 1, W, SEGLOOP, units_mixed<F, 1>()>(J, order); break;
     case 2: mv_body<F, 2, W, SEGLOOP, units_mixed<F, 2>()>(J, order); break;
@@ -758,7 +816,7 @@ __global__ __launch_bounds__(WAVE * W, ESQ_MIN_WAVES) void mv_kernel_mixed(const
 
 namespace esq {
 
-using MvFn = void (*)(const MvJob *, int, MvJob, int);
+using MvFn = void (*)(MvArgs);
 
 // Only the (NT, W) pairs the planner uses are instantiated.
 template <int F, int NT> static MvFn pick_w(int w, bool seg_loop) {
@@ -768,12 +826,14 @@ template <int F, int NT> static MvFn pick_w(int w, bool seg_loop) {
     }
     return nullptr;
 }
+using MvMixedFn = void (*)(const MvJob *, int, int);
+template <int F> static MvMixedFn pick_mixed(int w, bool seg_loop) {   // per-job pass widths
+    if (w == 4) return seg_loop ? nullptr : mv_kernel_mixed<F, 4, false>;
+    if (w == 8) return seg_loop ? mv_kernel_mixed<F, 8, true> : mv_kernel_mixed<F, 8, false>;
+    return nullptr;
+}
 template <int F> static MvFn pick_nt(int nt, int w, bool seg_loop) {
     switch (nt) {
-    case 0:   // per-job pass widths
-        if (w == 4) return seg_loop ? nullptr : mv_kernel_mixed<F, 4, false>;
-        if (w == 8) return seg_loop ? mv_kernel_mixed<F, 8, true> : mv_kernel_mixed<F, 8, false>;
-        return nullptr;
     case 1: return pick_w<F, 1>(w, seg_loop);
     case 2: return pick_w<F, 2>(w, seg_loop);
     case 4: return pick_w<F, 4>(w, seg_loop);
@@ -781,25 +841,48 @@ template <int F> static MvFn pick_nt(int nt, int w, bool seg_loop) {
     return nullptr;
 }
 
-hipError_t mv_launch(const MvLaunch &L, const MvJob *jobs, int njobs, const MvJob &single, int order, hipStream_t s) {
-    MvFn fn = nullptr;
-    switch (L.type) {
-    case ES_HIP_Q4_0: fn = pick_nt<ES_HIP_Q4_0>(L.nt, L.waves, L.seg_loop); break;
-    case ES_HIP_Q5_0: fn = pick_nt<ES_HIP_Q5_0>(L.nt, L.waves, L.seg_loop); break;
-    case ES_HIP_Q8_0: fn = pick_nt<ES_HIP_Q8_0>(L.nt, L.waves, L.seg_loop); break;
-    case ES_HIP_Q2_K: fn = pick_nt<ES_HIP_Q2_K>(L.nt, L.waves, L.seg_loop); break;
-    case ES_HIP_Q3_K: fn = pick_nt<ES_HIP_Q3_K>(L.nt, L.waves, L.seg_loop); break;
-    case ES_HIP_Q4_K: fn = pick_nt<ES_HIP_Q4_K>(L.nt, L.waves, L.seg_loop); break;
-    case ES_HIP_Q5_K: fn = pick_nt<ES_HIP_Q5_K>(L.nt, L.waves, L.seg_loop); break;
-    case ES_HIP_Q6_K: fn = pick_nt<ES_HIP_Q6_K>(L.nt, L.waves, L.seg_loop); break;
+hipError_t mv_launch(const MvLaunch &L, const MvJob *jobs, int njobs, const MvJob *hjobs, int order, hipStream_t s) {
+    if (!jobs && (njobs < 1 || njobs > MV_INLINE)) return hipErrorInvalidValue;
+    MvArgs A{jobs, njobs, order, {}};
+    dim3 grid(L.grid);
+    if (!jobs) {
+        int most = 0;   // tiles of the longest job; a shorter one's workgroups past its rows have nothing to do
+        for (int i = 0; i < njobs; i++) {
+            A.j[i] = hjobs[i];
+            A.j[i].tile0 = 0;
+            const int tiles = (hjobs[i].r1 - hjobs[i].r0 + hjobs[i].rows_per_wg - 1) / hjobs[i].rows_per_wg;
+            most = tiles > most ? tiles : most;
+        }
+        grid = dim3(most, njobs);
     }
-    if (!fn) return hipErrorInvalidValue;
+    MvFn fn = nullptr;
+    MvMixedFn mixed = nullptr;
+    auto pick = [&](auto type) {
+        constexpr int F = decltype(type)::value;
+        if (L.nt) fn = pick_nt<F>(L.nt, L.waves, L.seg_loop);
+        else mixed = pick_mixed<F>(L.waves, L.seg_loop);
+    };
+    switch (L.type) {
+    case ES_HIP_Q4_0: pick(std::integral_constant<int, ES_HIP_Q4_0>{}); break;
+    case ES_HIP_Q5_0: pick(std::integral_constant<int, ES_HIP_Q5_0>{}); break;
+    case ES_HIP_Q8_0: pick(std::integral_constant<int, ES_HIP_Q8_0>{}); break;
+    case ES_HIP_Q2_K: pick(std::integral_constant<int, ES_HIP_Q2_K>{}); break;
+    case ES_HIP_Q3_K: pick(std::integral_constant<int, ES_HIP_Q3_K>{}); break;
+    case ES_HIP_Q4_K: pick(std::integral_constant<int, ES_HIP_Q4_K>{}); break;
+    case ES_HIP_Q5_K: pick(std::integral_constant<int, ES_HIP_Q5_K>{}); break;
+    case ES_HIP_Q6_K: pick(std::integral_constant<int, ES_HIP_Q6_K>{}); break;
+    }
+    if ((!fn && !mixed) || (mixed && !jobs)) return hipErrorInvalidValue;
     if (L.lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           static_cast<int>(L.lds));
+        hipError_t e = hipFuncSetAttribute(fn ? reinterpret_cast<const void *>(fn) : reinterpret_cast<const void *>(mixed),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(L.lds));
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(fn, dim3(L.grid), dim3(WAVE * L.waves), L.lds, s, jobs, njobs, single, order);
+    if (mixed) {
+        hipLaunchKernelGGL(mixed, grid, dim3(WAVE * L.waves), L.lds, s, jobs, njobs, order);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(fn, grid, dim3(WAVE * L.waves), L.lds, s, A);
     return hipGetLastError();
 }
 

@@ -116,6 +116,10 @@ constexpr size_t CHAIN_MAX = 256;           // rows per chain batch at most
 constexpr size_t MIN_WG_BLOCKS = 512;       // blocks per workgroup at least: a workgroup's set-up (job lookup, gathered
                                             // activation loads) is a chain of dependent loads that small launches (an
                                             // MoE layer's experts at a few tokens each) would otherwise repeat per 24 rows
+constexpr size_t SMALL_WG = 512;            // ... and down to half of that while a launch has fewer workgroups than this: one
+                                            // or two matrices at a time leave CUs idle otherwise (Q4_K, one activation, in a
+                                            // graph: 2048 x 2048 5.5 us at 512 blocks, 4.3 at 256 and below; 2048 x 8192 7.1
+                                            // and 6.0; 8192 x 2048 twice 8.1 and 7.6; Q6_K 2048 x 8192 9.3 and 7.3)
 
 struct Group {
     MvLaunch L{};
@@ -205,7 +209,8 @@ int plan_groups(const std::vector<Req> &reqs, std::vector<Group> &out) {
     }
     // workgroups of about total/TARGET_WG blocks each, each wave making at least MIN_ITERS row passes, so one launch keeps
     // every CU busy whether it holds one matrix or a hundred
-    const size_t wg_blocks = std::max<size_t>(MIN_WG_BLOCKS, total_blocks / TARGET_WG);
+    const size_t small = std::min(MIN_WG_BLOCKS, std::max(MIN_WG_BLOCKS / 2, total_blocks / SMALL_WG));
+    const size_t wg_blocks = std::max<size_t>(small, total_blocks / TARGET_WG);
     for (auto &kv : by_kind) {
         FmtInfo f;
         fmt_info(kv.first.first, f);
@@ -240,7 +245,10 @@ int plan_groups(const std::vector<Req> &reqs, std::vector<Group> &out) {
             if (per_row > LDS_MAX) return fail(ES_HIP_EINVAL, "type %u cols %d: a row needs %zu bytes of LDS", q->type, q->cols, per_row);
             int chain_cap = (int)std::min<size_t>(CHAIN_MAX, std::max<size_t>(1, LDS_TARGET / per_row));
             if (chain_cap >= rstep) chain_cap -= chain_cap % rstep;
-            int rpw = (int)std::max<size_t>((size_t)MIN_ITERS * rstep, (wg_blocks + nbk - 1) / nbk);
+            // (a 32-element row over every wave of the workgroup: its chain terms are most of the work, and a workgroup's LDS
+            // holds those of a few rows; Q8_0 2048 x 8192: 13.5 us at four passes, 9.9 at two, 15.7 at one)
+            const int iters = w32 && seg >= waves ? MIN_ITERS / 2 : MIN_ITERS;
+            int rpw = (int)std::max<size_t>((size_t)iters * rstep, (wg_blocks + nbk - 1) / nbk);
             rpw = std::min(rpw, (rows + rstep - 1) / rstep * rstep);
             rpw = (rpw + rstep - 1) / rstep * rstep;
             const int chain = std::min(chain_cap, rpw);
@@ -278,8 +286,8 @@ int plan_groups(const std::vector<Req> &reqs, std::vector<Group> &out) {
     return ES_HIP_OK;
 }
 
-int launch_single(const Group &g, hipStream_t s, int order = -1) {
-    hipError_t e = esq::mv_launch(g.L, nullptr, 1, g.jobs[0], order >= 0 ? order : g_order.load(), s);
+int launch_single(const Group &g, hipStream_t s) {   // a launch's one job, by value
+    hipError_t e = esq::mv_launch(g.L, nullptr, 1, g.jobs.data(), g_order.load(), s);
     return e == hipSuccess ? ES_HIP_OK : hip_fail(e, "kernel launch");
 }
 
@@ -1023,6 +1031,16 @@ std::vector<uint8_t> table_image(const Batch &bt) {
     return img;
 }
 
+// a decode launch whose jobs travel as its arguments
+bool mv_inline(const Group &g) { return g.jobs.size() <= (size_t)esq::MV_INLINE && g.L.nt != 0; }
+// no launch of the batch reads anything but its arguments
+bool table_free(const Batch &bt) {
+    if (!bt.mm.empty() || !bt.mqg.empty() || !bt.mbg.empty() || !bt.mkg.empty() || !bt.pkg.empty()) return false;
+    for (const Group &g : bt.mv)
+        if (!mv_inline(g)) return false;
+    return true;
+}
+
 // launches in stream order: pre-passes, decode kernels, matrix-core kernel. tables: the uploaded image, or null to pass
 // single jobs by value.
 int launch_batch(const Batch &bt, const uint8_t *tables, int order, hipStream_t s) {
@@ -1041,7 +1059,9 @@ int launch_batch(const Batch &bt, const uint8_t *tables, int order, hipStream_t 
     for (size_t i = 0; i < bt.mv.size(); i++) {
         const Group &g = bt.mv[i];
         const MvJob *dj = tables ? reinterpret_cast<const MvJob *>(tables + bt.mv_off[i]) : nullptr;
-        if ((e = esq::mv_launch(g.L, dj, (int)g.jobs.size(), g.jobs[0], order, s)) != hipSuccess) return hip_fail(e, "kernel launch");
+        const int nj = (int)g.jobs.size();
+        if (mv_inline(g)) dj = nullptr;   // the jobs go with the launch
+        if ((e = esq::mv_launch(g.L, dj, nj, g.jobs.data(), order, s)) != hipSuccess) return hip_fail(e, "kernel launch");
     }
     for (const MmGroup &g : bt.mmg) {
         const esq::MmJob *dj = tables ? reinterpret_cast<const esq::MmJob *>(tables + g.off) : nullptr;
@@ -1365,7 +1385,10 @@ int run_launch(const std::vector<Req> &reqs, hipStream_t s, int order) {   // or
     }
     Batch bt;
     if (int e = plan_batch(reqs, bt)) return e;
-    if (bt.mv.empty() && bt.mm.empty() && bt.mqg.empty() && bt.mbg.empty() && bt.mkg.empty() && bt.pkg.empty()) return ES_HIP_OK;
+    if (table_free(bt)) {   // nothing staged, no scratch
+        g_table_pending = true;   // the caller's wait follows
+        return launch_batch(bt, nullptr, order >= 0 ? order : g_order.load(), s);
+    }
     if (int e = settle()) return e;
     if (keep_and_launch(reqs, bt, s, order, rc)) {
         g_table_pending = true;
@@ -1479,7 +1502,7 @@ int es_hip_synchronize(void) {
 }
 
 // ---- products on device memory ----------------------------------------------------------------------------------------
-// Plan and launch a batch in stream order: a single decode job by value; anything else (several jobs per launch,
+// Plan and launch a batch in stream order: decode launches of a few jobs by value; anything else (long job lists,
 // pre-passes) with a stream-ordered allocation for the job tables and the pre-pass workspace, freed in stream order. The
 // tables are copied from pageable memory, which the copy has consumed when it returns.
 static int run_async(const std::vector<Req> &reqs, hipStream_t s, int order = -1) {
@@ -1490,9 +1513,7 @@ static int run_async(const std::vector<Req> &reqs, hipStream_t s, int order = -1
     if (cached_launch(reqs, s, order, rc)) return rc;
     Batch bt;
     if (int e = plan_batch(reqs, bt)) return e;
-    if (bt.mm.empty() && bt.mqg.empty() && bt.mbg.empty() && bt.mkg.empty() && bt.pkg.empty() && bt.mv.size() <= 1 &&
-        (bt.mv.empty() || bt.mv[0].jobs.size() == 1))
-        return bt.mv.empty() ? ES_HIP_OK : launch_single(bt.mv[0], s, order);
+    if (table_free(bt)) return launch_batch(bt, nullptr, order >= 0 ? order : g_order.load(), s);
     if (keep_and_launch(reqs, bt, s, order, rc)) return rc;
     void *dev = nullptr;
     const size_t ws_at = align256(bt.table_bytes);
@@ -2576,7 +2597,7 @@ int moe_ctx_layer(es_hip_moe_ctx *c, int N, const void *x, size_t xstride, float
     const int order = g_order.load();
     auto run = [&](const MoeLaunch &M, uint32_t type, void *jobs, esq::PrepJob *prep) -> int {
         if (M.F.kind == esq::MOE_FAM_MV) {
-            e = esq::mv_launch(M.L, static_cast<const MvJob *>(jobs), M.njobs, M.F.mv, order, s);
+            e = esq::mv_launch(M.L, static_cast<const MvJob *>(jobs), M.njobs, &M.F.mv, order, s);
             return e == hipSuccess ? ES_HIP_OK : hip_fail(e, "MoE decode-kernel launch");
         }
         if (M.F.kind == esq::MOE_FAM_MX) {
