@@ -285,8 +285,8 @@ int es_hip_set_batched32_min(int n);
 /* Of those, products with at least n activations run on the batched matrix-core kernel (one int8 MFMA per block forms the
  * eight AVX2 lane sums of 4 rows x 32 activations; default 2); the others on the one-lane-per-output kernel. */
 int es_hip_set_batched32_mfma_min(int n);
-/* Q6_K products with at least n activations (and an even number of superblocks per row) run on the Q6_K matrix-core
- * kernel (default 16). */
+/* Q6_K products with at least n activations run on a Q6_K matrix-core kernel (default 16, which also stands for the
+ * automatic choice: from 5 activations on the kernel with one wave per superblock). */
 int es_hip_set_q6k_mfma_min_batch(int n);
 /* Q2_K products with at least n activations run on the Q2_K LDS-staged matrix-core kernel (default 2); below that, or
  * with it off, the small-batch kernel (es_hip_set_small_batch_min) or the vector kernel. */
@@ -323,10 +323,11 @@ int es_hip_set_moe_gated(int on);
  * 16 rows x 32 activations (no pre-pass); with 0, the one that reads them from a pre-pass layout. Results are identical
  * on both. Returns the previous setting. */
 int es_hip_set_batched32_direct(int on);
-/* A Q6_K product on the matrix cores that is alone in its launch, has one tile of activations (at most 64) and short
- * rows (at most 5 superblocks at 64 activations, 11 at 32, 22 at 16) runs, with on != 0 (the default), as a persistent
- * launch: one workgroup per CU copies the activations into LDS once and streams its row tiles back to back. Results
- * are identical either way. Returns the previous setting. */
+/* With on != 0 (the default) a Q6_K product on the matrix cores runs on the kernel with one wave per superblock where that is
+ * the faster one (few rows, short batches), and a product that is alone in its launch, has one tile of activations (at most
+ * 64), at least two row tiles per CU and short rows (at most 5 superblocks at 64 activations, 11 at 32, 22 at 16) as a
+ * persistent launch of the tiled kernel: one workgroup per CU copies the activations into LDS once and streams its row
+ * tiles back to back. With 0 every product runs on the tiled kernel, one workgroup per tile. Results are identical. */
 int es_hip_set_q6k_persistent(int on);
 /* Q4_K and Q3_K products that take the direct-activation kernel and have an even number (at least 2) of superblocks per
  * row, with no gathered activations, run, with on != 0, in one persistent launch per format, each workgroup computing a

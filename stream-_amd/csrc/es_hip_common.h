@@ -131,6 +131,7 @@ constexpr int MX_TOK = 32, MX_ROWS = ESQ_MX_ROWS, MX_NBK = 16;
 // the Q6_K matrix-core kernel's persistent form for single products (es_hip_mm6.hip): on (default) or off; returns the
 // previous setting
 int mm6_set_persistent(int on);
+int mm6_persistent_blocks(int bn);   // superblocks per row it takes at most at bn (16, 32 or 64) activations
 int mx_nbk_max(int nbk);
 // The gated form (a Q2_K expert's gate and up products with the SwiGLU and the Q8_K requantization of h fused in): per
 // job, W and W2 the gate's and up's rows, y the first h row's Q8_K blocks (bytes), r0 and r1 multiples of 256
@@ -146,6 +147,11 @@ constexpr int MBX_TOK = 32, MBX_ROWS = 32, MBX_NBK = 128, MBX_WAVES = 8;
 int mbx_nbk_max(int nbk);
 hipError_t mbx_launch(int type, bool gather, int nbk_max, const MkJob *jobs, int njobs, const MkJob &single, int grid,
                       int order, hipStream_t s);
+// Q6_K batches with one wave per superblock (es_hip_m6w.hip): the same jobs without a gather, workgroups of nw <= M6W_WAVES
+// waves over rows_per_wg groups of 16 rows x 16 wn activations (wn 1, 2 or 4; all activation tiles of a row chunk on one XCD:
+// 8 * ceil(chunks / 8) * ntok_tiles ids per job, tile0 a multiple of 8). keep: every job has at most nw superblocks per row.
+constexpr int M6W_WAVES = 8;
+hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob &single, int grid, int order, hipStream_t s);
 // gather: some job of the launch reads its activation rows through arow (a separate kernel build; the others need not);
 // tok: activations per workgroup tile, MK_TOK or 64 (ntok_tiles and the tile numbering then count tiles of 64)
 hipError_t mk_launch(int type, bool gather, int tok, const MkJob *jobs, int njobs, const MkJob &single, int grid, int order,
@@ -385,6 +391,36 @@ __device__ __forceinline__ uint32_t pk_mul_u16(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b));
 }
 
+// Q6_K operands of the matrix-core kernels. Two signed byte planes of four codes (one per byte, 0..63) times the group's
+// scale: v = q * sc = 256 hi + lo, formed in 16-bit lanes as v + 128 = 256 hi + (lo + 128). sc2: q6_scale2.
+__device__ __forceinline__ uint32_t q6_scale2(uint32_t scales, int byte) {   // one signed scale byte in both 16-bit halves
+    const uint32_t s = (uint32_t)((int)(scales << (24 - 8 * byte)) >> 24);
+    return __builtin_amdgcn_perm(s, s, 0x01000100u);
+}
+__device__ __forceinline__ void q6_planes(uint32_t q, uint32_t sc2, uint32_t &hi, uint32_t &lo) {
+    const u16x2 s = __builtin_bit_cast(u16x2, sc2), r = {128, 128};
+    const uint32_t me = __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, q & 0x00ff00ffu) * s + r));          // even bytes
+    const uint32_t mo = __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, (q >> 8) & 0x00ff00ffu) * s + r));   // odd bytes
+    hi = __builtin_amdgcn_perm(mo, me, 0x07030501u);
+    lo = __builtin_amdgcn_perm(mo, me, 0x06020400u) ^ 0x80808080u;
+}
+// -32 sc of eight groups (their scale bytes in w0, w1) as halves, for lane groups 0 and 1 (k positions 0..7 and 8..15 of
+// mfma_f32_16x16x32_f16 meet the bsums); the others zero. 0x7800 | u is 32768 + 32 u with u = sc + 128; 36864 minus it is
+// -32 sc, exact. Every partial sum of -32 sc * bsum is a multiple of 32 below 2^29: exact in f32.
+__device__ __forceinline__ v8h q6_corr(uint32_t w0, uint32_t w1, int lg) {
+    v8h c = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (lg >= 2) return c;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const uint32_t k0 = (2 * e) & 3;
+        const uint32_t pr = __builtin_amdgcn_perm(0x78787878u, (e < 2 ? w0 : w1) ^ 0x80808080u, k0 | 0x0400u | (k0 + 1) << 16 | 0x04000000u);
+        const h2 v = __builtin_bit_cast(h2, 0x78807880u) - __builtin_bit_cast(h2, pr);
+        c[2 * e] = v[0];
+        c[2 * e + 1] = v[1];
+    }
+    return c;
+}
+
 // The job of workgroup bid in a launch whose jobs hold consecutive tile ranges from tile0 (the last job with
 // tile0 <= bid). When the jobs are of equal size (an MoE layer's experts, copies of one matrix) the proportional guess
 // is that job: the guessed job itself and the next job's tile0 are independent loads, so the job arrives in the same
@@ -410,6 +446,17 @@ template <typename JobT> __device__ __forceinline__ JobT load_tile_job(const Job
         if (jobs[mid].tile0 <= bid) lo = mid; else hi = mid - 1;
     }
     return jobs[lo];
+}
+
+// A job record in scalar registers: merged from a table and a kernel argument it otherwise lands in vector registers.
+template <typename JobT> __device__ __forceinline__ JobT uniform_job(const JobT &J) {
+    static_assert(sizeof(JobT) % 4 == 0, "jobs are moved as dwords");
+    constexpr int N = sizeof(JobT) / 4;
+    uint32_t v[N];
+    __builtin_memcpy(v, &J, sizeof J);
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)v[i]);
+    return __builtin_bit_cast(JobT, v);
 }
 
 // One wave's 64 x 16 bytes from global memory straight into LDS: lane l's 16 bytes at base + off land at lds + 16*l

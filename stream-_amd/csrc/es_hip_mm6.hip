@@ -3,12 +3,9 @@
 // activation and superblock, tot = sum sc * q_u * x - 32 * sum_g sc_g * bsums_g with q_u the unsigned 6-bit code, then
 // s += (y.d * d) * tot (src/es_quant.c:1602-1640).
 //
-// The products q_u * sc (up to 63 * 128 in size) do not fit int8. With sc_u = sc + 128 = 16h + l and q_u = 8a + b (h, l
-// in 0..15, a, b in 0..7):  q_u * sc = q_u * sc_u - 128 q_u = 128 (a h - q_u) + 16 b h + 8 a l + b l,
-// four int8 planes (a h - q_u in -63..105, the others in 0..105) through the matrix cores, recombined exactly in int32:
-//   sum q_u * sc * x = 128 D(ah - q_u) + 16 D(bh) + 8 D(al) + D(bl).
-// corr = sum_g sc_g * bsums_g goes through one f16 MFMA (scales and bsums are exact halves and every partial sum stays
-// below 2^24: exact).
+// The products q_u * sc (-8064..8001) do not fit int8: two signed byte planes carry them exactly, q_u * sc = 256 hi + lo, so
+//   sum q_u * sc * x = 256 D(hi) + D(lo);
+// -32 corr, corr = sum_g sc_g * bsums_g, goes through one f16 MFMA (q6_planes, q6_corr, es_hip_common.h).
 //
 // Weights: a 210-byte superblock starts 2-byte aligned. Each row's superblock is read with 16-byte loads at 2-byte aligned
 // addresses (the hardware's unaligned global access) and a 2-byte load of d, and written to LDS as an aligned 208-byte
@@ -214,9 +211,9 @@ __global__ __launch_bounds__(64 * RW * TW) void mm_q6k_kernel(const MmJob *__res
         Bt B[2];
         load_b(0, B[0]);
 
-        // ---- A operands: per slice ks the four planes, and the scales as halves for corr
-        const uint32_t u[4] = {scw.x ^ 0x80808080u, scw.y ^ 0x80808080u, scw.z ^ 0x80808080u, scw.w ^ 0x80808080u};   // sc + 128
-        v4i p1[4], p2[4], p3[4], p4[4];
+        // ---- A operands: per slice ks the two planes, and -32 times the scales as halves for corr
+        const uint32_t scv[4] = {scw.x, scw.y, scw.z, scw.w};
+        v4i hi[4], lo[4];
         // the qh dwords shifted by this lane's field pair once (2 qo bits): field 2 qn + qo of each byte then sits at bits
         // 4 qn .. 4 qn + 1, so slice ks takes it with one shift (qn = 0) or none (qn = 1)
         const uint32_t qs0[4] = {qh0.x >> (2 * qo), qh0.y >> (2 * qo), qh0.z >> (2 * qo), qh0.w >> (2 * qo)};
@@ -224,57 +221,34 @@ __global__ __launch_bounds__(64 * RW * TW) void mm_q6k_kernel(const MmJob *__res
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
             const int n = ks >> 1, qn = ks & 1;
-            const uint32_t lsc = __builtin_amdgcn_perm(0, u[ks] & 0x0f0f0f0fu, sel);          // l, in both halves
-            const uint32_t hsc = __builtin_amdgcn_perm(0, (u[ks] >> 4) & 0x0f0f0f0fu, sel);   // h
+            const uint32_t sc2 = q6_scale2(scv[ks], lg);
             const uint4 qlv = n ? ql1 : ql0;
             const uint32_t qlw[4] = {qlv.x, qlv.y, qlv.z, qlv.w};
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const uint32_t nib = qn ? (qlw[i] >> 4) & 0x0f0f0f0fu : qlw[i] & 0x0f0f0f0fu;
                 const uint32_t qsw = n ? qs1[i] : qs0[i];
-                const uint32_t qu = nib | ((qn ? qsw : qsw << 4) & 0x30303030u);   // 6-bit codes, one per byte
-                const uint32_t a = (qu >> 3) & 0x07070707u, bb = qu & 0x07070707u;
-                // a h - q_u per byte: (a h + 128 - q_u) stays in 65..233, so no borrow crosses a byte
-                p1[ks][i] = (int)(((pk_mul_u16(a, hsc) | 0x80808080u) - qu) ^ 0x80808080u);
-                p2[ks][i] = (int)pk_mul_u16(a, lsc);
-                p3[ks][i] = (int)pk_mul_u16(bb, hsc);
-                p4[ks][i] = (int)pk_mul_u16(bb, lsc);
+                uint32_t h, l;
+                q6_planes(nib | ((qn ? qsw : qsw << 4) & 0x30303030u), sc2, h, l);
+                hi[ks][i] = (int)h;
+                lo[ks][i] = (int)l;
             }
         }
-        // corr operand (halves): lanes 0..15 carry sc_0..7, lanes 16..31 sc_8..15 (k positions meet bsums 0..7 / 8..15);
-        // lanes 32..63 zero. Each half is built as 1024 + sc_u (byte under the exponent of 1024), then 1152 subtracted.
-        v8h acorr;
-        {
-            const uint32_t w0 = lg == 0 ? u[0] : u[2], w1 = lg == 0 ? u[1] : u[3];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t k0 = (2 * e) & 3;
-                const uint32_t pr = __builtin_amdgcn_perm(0x64646464u, e < 2 ? w0 : w1,
-                                                          k0 | 0x0400u | (k0 + 1) << 16 | 0x04000000u);
-                const h2 v = __builtin_bit_cast(h2, pr) + __builtin_bit_cast(h2, 0xe480e480u);   // - 1152
-                acorr[2 * e] = v[0];
-                acorr[2 * e + 1] = v[1];
-            }
-            if (lg >= 2) acorr = v8h{0, 0, 0, 0, 0, 0, 0, 0};
-        }
+        const v8h acorr = q6_corr(lg == 0 ? scv[0] : scv[2], lg == 0 ? scv[1] : scv[3], lg);
 
-        v4i d1[2], d2[2], d3[2], d4[2];
+        v4i dh[2], dl[2];
         v4f dc[2];
         float tdv[2];
         auto mma = [&](int c, const Bt &Bc) {
             const int w = c & 1;
             tdv[w] = Bc.td;
             dc[w] = __builtin_amdgcn_mfma_f32_16x16x32_f16(acorr, Bc.m, v4f{0, 0, 0, 0}, 0, 0, 0);
-            d1[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(p1[0], Bc.x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
-            d2[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(p2[0], Bc.x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
-            d3[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(p3[0], Bc.x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
-            d4[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(p4[0], Bc.x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
+            dh[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi[0], Bc.x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
+            dl[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo[0], Bc.x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
             for (int ks = 1; ks < 4; ks++) {
-                d1[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(p1[ks], Bc.x[ks], d1[w], 0, 0, 0);
-                d2[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(p2[ks], Bc.x[ks], d2[w], 0, 0, 0);
-                d3[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(p3[ks], Bc.x[ks], d3[w], 0, 0, 0);
-                d4[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(p4[ks], Bc.x[ks], d4[w], 0, 0, 0);
+                dh[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi[ks], Bc.x[ks], dh[w], 0, 0, 0);
+                dl[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo[ks], Bc.x[ks], dl[w], 0, 0, 0);
             }
         };
         // fp32 epilogue of superblock b for tile c, per (row, activation), in the reference's order
@@ -282,14 +256,14 @@ __global__ __launch_bounds__(64 * RW * TW) void mm_q6k_kernel(const MmJob *__res
             const int w = c & 1;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int tot = d4[w][i] + 8 * d2[w][i] + 16 * d3[w][i] + 128 * d1[w][i] - 32 * (int)dc[w][i];
+                const int tot = ((dh[w][i] << 8) + dl[w][i]) + (int)dc[w][i];
                 const float f = tdv[w] * dv[i];
                 if constexpr (CONTRACT) s[c][i] = __builtin_fmaf(f, static_cast<float>(tot), s[c][i]);
                 else s[c][i] = s[c][i] + f * static_cast<float>(tot);
             }
         };
         // one scheduling group per tile: tile c+1's LDS reads, tile c's matrix work and tile c-1's epilogue, interleaved as
-        // 1 MFMA : 2 VALU (: 1 LDS read)
+        // 1 MFMA : 3 VALU (: 1 LDS read)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int c = 0; c < WN; c++) {
@@ -297,9 +271,9 @@ __global__ __launch_bounds__(64 * RW * TW) void mm_q6k_kernel(const MmJob *__res
             mma(c, B[c & 1]);
             if (c) epi(c - 1);
 #pragma unroll
-            for (int k = 0; k < 17; k++) {
+            for (int k = 0; k < 9; k++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
-                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);   // VALU
+                __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);   // VALU
                 if (k < 6) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -367,6 +341,9 @@ static hipError_t mm6_launch_cfg(const MmJob *jobs, int njobs, const MmJob &sing
     return hipGetLastError();
 }
 
+int mm6_persistent_blocks(int bn) {
+    return bn == 64 ? Mm6Geom<8, 1, 4>::NBKP : bn == 32 ? Mm6Geom<8, 1, 2>::NBKP : Mm6Geom<8, 1, 1>::NBKP;
+}
 int mm6_set_persistent(int on) { return g_mm6_persistent.exchange(on ? 1 : 0); }
 
 // Q6_K workgroup tiles: 128 rows x 16, 32 or 64 activations on 8 waves (16 rows x all the activations each)

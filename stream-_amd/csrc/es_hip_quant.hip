@@ -341,6 +341,8 @@ struct MkGroup {   // one direct-activation matrix-core launch: products of one 
     bool b32 = false; // ... or with nbkm, the 32-wide kernel reading Q8_0 rows (es_hip_mbx.hip)
     int tok = esq::MK_TOK;   // the direct kernel's activations per tile
     bool gated = false;      // with nbkm: the gated expert kernel (gate and up of a Q2_K expert, h as Q8_K blocks)
+    int m6_wn = 0, m6_nw = 0;   // > 0: the Q6_K kernel with one wave per superblock (es_hip_m6w.hip), activation tiles, waves
+    bool m6_keep = false;
     int grid = 0;
     std::vector<esq::MkJob> jobs;
     size_t off = 0;
@@ -676,6 +678,60 @@ bool pk_schedule_form(PkGroup &g, int cus) {
     return true;
 }
 
+// Waves per workgroup of the Q6_K kernel with one wave per superblock: a row's superblocks over at most 8 waves, as evenly
+// as their number allows.
+int m6w_waves(int nbk) {
+    const int rounds = (nbk + esq::M6W_WAVES - 1) / esq::M6W_WAVES;
+    return (nbk + rounds - 1) / rounds;
+}
+// Activations per workgroup, in tiles of 16: up to 64 (a superblock is unpacked once per workgroup), 32 where a wave takes
+// several superblocks (their activation operands are loaded ahead, which at 64 does not fit the registers), fewer while a
+// product has less than a workgroup per CU.
+int m6w_tiles(int rows, int na, int nbk, int cus) {
+    int wn = nbk > esq::M6W_WAVES ? 2 : 4;
+    while (wn > 1 && 8 * wn >= na) wn /= 2;
+    while (wn > 1 && (long)((rows + 15) / 16) * ((na + 16 * wn - 1) / (16 * wn)) < cus) wn /= 2;
+    return wn;
+}
+// Which Q6_K batches take that kernel (no gather, 32-bit offsets): of the default g_mm6_min = 16 (the automatic choice) those
+// of 5 activations or more, else those of g_mm6_min, where it is the faster of the matrix-core kernels. The tiled kernel
+// (es_hip_mm6.hip) runs a tile's superblocks one after another, 2.4 us each, a set of 256 tiles of 128 rows x 64 activations
+// at a time (2 us more each), behind a pre-pass (6 us); this one takes about 1.4 ns per superblock of 16 rows x 16 wn
+// activations, 2.3 with several superblocks per wave, and 5 us. Measured (us, this kernel / tiled): 2048 x 8192 at 64, 128 and
+// 512 activations 24 / 79, 41 / 78, 141 / 79; 8192 x 2048 13 / 26, 18 / 26, 50 / 48; 4096 x 4096 21 / 44, 37 / 43, 129 / 47;
+// against the decode kernel's passes of 4 at 8 activations 8192 x 2048 9.3 / 14.1, 151936 x 1024 57 / 66 (2048 x 8192 16.6 /
+// 15.2), and slower at 4 (8.9 / 8.6). A product of one activation tile and many row tiles whose activations fit the LDS
+// keeps the tiled kernel's persistent form (151936 x 1024 at 16 and 64: 57 / 43, 61 / 58).
+std::atomic<int> g_m6w_on{1};
+bool m6w_eligible(const Req &q) {
+    const int set = g_mm6_min.load(), mn = set == 16 ? 5 : set;
+    if (!g_m6w_on.load() || q.type != ES_HIP_Q6_K || mn <= 0 || q.na < mn || q.na > 2048 || q.arow || q.ints || q.r1 <= q.r0) return false;
+    const int nbk = q.cols / 256, rows = q.r1 - q.r0, cus = device().cus;
+    const size_t stride = q.astride ? q.astride : (size_t)nbk * 292;
+    if ((size_t)q.na * stride >= ((size_t)1 << 32) - 65536 || (size_t)q.r1 * nbk * 210 >= ((size_t)1 << 32)) return false;
+    if (q.na < 16) return true;
+    const int rt = (rows + 127) / 128, bn = q.na <= 16 ? 16 : q.na <= 32 ? 32 : 64;
+    if (q.na <= 64 && rt >= 2 * cus && nbk <= esq::mm6_persistent_blocks(bn)) return false;
+    const int wn = m6w_tiles(rows, q.na, nbk, cus);
+    const double units = (double)((rows + 15) / 16) * ((q.na + 16 * wn - 1) / (16 * wn)) * nbk;
+    const long sets = ((long)rt * ((q.na + 63) / 64) + cus - 1) / cus;
+    return 5.0 + units * (nbk > esq::M6W_WAVES ? 2.3e-3 : 1.4e-3) < 6.0 + (2.0 + 2.4 * nbk) * sets;
+}
+// Row groups per workgroup and the tile numbering: about one resident set of workgroups (16 waves per CU) for the launch.
+void m6w_tiling(MkGroup &g, int cus) {
+    long units = 0;
+    for (const esq::MkJob &j : g.jobs) units += (long)((j.r1 - j.r0 + 15) / 16) * j.ntok_tiles;
+    const long slots = (long)cus * std::max(1, 8 / g.m6_nw);
+    const int per = (int)std::max<long>(1, (units + slots - 1) / slots);
+    g.grid = 0;
+    for (esq::MkJob &j : g.jobs) {
+        j.rows_per_wg = per;
+        j.tile0 = g.grid;
+        const int chunks = ((j.r1 - j.r0 + 15) / 16 + per - 1) / per;
+        g.grid += 8 * ((chunks + 7) / 8) * j.ntok_tiles;
+    }
+}
+
 bool mb_eligible(const Req &q) {
     const int mn = g_mb_min.load();
     return (q.type == ES_HIP_Q4_0 || q.type == ES_HIP_Q5_0 || q.type == ES_HIP_Q8_0) && mn > 0 && q.na >= mn && !q.ints &&
@@ -854,7 +910,7 @@ int plan_batch(const std::vector<Req> &reqs, Batch &bt, bool allow_pk = true) {
             const int tok = mk_tok(q);
             MkGroup *g = nullptr;
             for (MkGroup &x : bt.mkg)
-                if (!x.b32 && x.type == (int)q.type && x.gather == (q.arow != nullptr) && x.nbkm == 0 && x.tok == tok) g = &x;
+                if (!x.b32 && !x.m6_wn && x.type == (int)q.type && x.gather == (q.arow != nullptr) && x.nbkm == 0 && x.tok == tok) g = &x;
             if (!g) {
                 bt.mkg.push_back(MkGroup{(int)q.type, q.arow != nullptr});
                 g = &bt.mkg.back();
@@ -877,6 +933,33 @@ int plan_batch(const std::vector<Req> &reqs, Batch &bt, bool allow_pk = true) {
             const int row_tiles = (q.r1 - q.r0 + esq::MK_ROWS - 1) / esq::MK_ROWS;
             g->grid += 8 * ((row_tiles + 7) / 8) * j.ntok_tiles;
             g->jobs.push_back(j);
+            continue;
+        }
+        if (m6w_eligible(q)) {
+            const int wn = m6w_tiles(q.r1 - q.r0, q.na, nbk, device().cus), nw = m6w_waves(nbk);
+            MkGroup *g = nullptr;
+            for (MkGroup &x : bt.mkg)
+                if (x.m6_wn == wn && x.m6_nw == nw && x.m6_keep == (nbk <= nw)) g = &x;
+            if (!g) {
+                bt.mkg.push_back(MkGroup{(int)q.type, false});
+                g = &bt.mkg.back();
+                g->m6_wn = wn;
+                g->m6_nw = nw;
+                g->m6_keep = nbk <= nw;
+            }
+            esq::MkJob j{};
+            j.W = static_cast<const uint8_t *>(q.W);
+            j.act = static_cast<const uint8_t *>(q.act);
+            j.y = q.y;
+            j.astride = q.astride ? q.astride : (uint64_t)nbk * f.ab;
+            j.ystride = q.ystride;
+            j.row_bytes = (uint64_t)nbk * f.bb;
+            j.r0 = q.r0;
+            j.r1 = q.r1;
+            j.cols = q.cols;
+            j.na = q.na;
+            j.ntok_tiles = (q.na + 16 * wn - 1) / (16 * wn);
+            g->jobs.push_back(j);   // (tiles numbered once the launch's jobs are known, m6w_tiling)
             continue;
         }
         if (!mm_eligible(q)) {
@@ -944,8 +1027,10 @@ int plan_batch(const std::vector<Req> &reqs, Batch &bt, bool allow_pk = true) {
         g->grid += 8 * ((row_tiles + 7) / 8) * j.ntok_tiles;
         g->jobs.push_back(j);
     }
-    for (MkGroup &g : bt.mkg)
+    for (MkGroup &g : bt.mkg) {
         if (g.b32) mbx_tiles(g, device().cus);
+        if (g.m6_wn) m6w_tiling(g, device().cus);
+    }
     for (PkGroup &g : bt.pkg)
         if (!pk_schedule(g, device().cus)) return plan_batch(reqs, bt, false);   // too many tiles for one launch
     // a pre-pass numbers its 16-byte items with 32-bit indices
@@ -1034,11 +1119,16 @@ std::vector<uint8_t> table_image(const Batch &bt) {
 // a decode launch whose jobs travel as its arguments
 bool mv_inline(const Group &g) { return g.jobs.size() <= (size_t)esq::MV_INLINE && g.L.nt != 0; }
 // no launch of the batch reads anything but its arguments
-bool table_free(const Batch &bt) {
-    if (!bt.mm.empty() || !bt.mqg.empty() || !bt.mbg.empty() || !bt.mkg.empty() || !bt.pkg.empty()) return false;
+bool table_free(const Batch &bt) {   // single jobs go by value, the persistent direct kernel always reads tables
+    if (!bt.pkg.empty()) return false;
     for (const Group &g : bt.mv)
         if (!mv_inline(g)) return false;
-    return true;
+    auto single = [](const auto &groups) {
+        for (const auto &g : groups)
+            if (g.jobs.size() != 1) return false;
+        return true;
+    };
+    return single(bt.mmg) && single(bt.mqg) && single(bt.mbg) && single(bt.mkg);
 }
 
 // launches in stream order: pre-passes, decode kernels, matrix-core kernel. tables: the uploaded image, or null to pass
@@ -1079,7 +1169,8 @@ int launch_batch(const Batch &bt, const uint8_t *tables, int order, hipStream_t 
     }
     for (const MkGroup &g : bt.mkg) {
         const esq::MkJob *dj = tables ? reinterpret_cast<const esq::MkJob *>(tables + g.off) : nullptr;
-        if ((e = g.b32    ? esq::mbx_launch(g.type, g.gather, g.nbkm, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)
+        if ((e = g.m6_wn ? esq::m6w_launch(g.m6_wn, g.m6_nw, g.m6_keep, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)
+                 : g.b32  ? esq::mbx_launch(g.type, g.gather, g.nbkm, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)
                  : g.nbkm && g.gated ? esq::mxg_launch(g.gather, g.nbkm, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)
                  : g.nbkm ? esq::mx_launch(g.type, g.gather, g.nbkm, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)
                           : esq::mk_launch(g.type, g.gather, g.tok, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)) !=
@@ -1385,7 +1476,7 @@ int run_launch(const std::vector<Req> &reqs, hipStream_t s, int order) {   // or
     }
     Batch bt;
     if (int e = plan_batch(reqs, bt)) return e;
-    if (table_free(bt)) {   // nothing staged, no scratch
+    if (table_free(bt) && !bt.ws_bytes) {   // nothing staged, no scratch
         g_table_pending = true;   // the caller's wait follows
         return launch_batch(bt, nullptr, order >= 0 ? order : g_order.load(), s);
     }
@@ -1502,8 +1593,8 @@ int es_hip_synchronize(void) {
 }
 
 // ---- products on device memory ----------------------------------------------------------------------------------------
-// Plan and launch a batch in stream order: decode launches of a few jobs by value; anything else (long job lists,
-// pre-passes) with a stream-ordered allocation for the job tables and the pre-pass workspace, freed in stream order. The
+// Plan and launch a batch in stream order: decode launches of a few jobs and other launches of one by value (with a
+// stream-ordered allocation for their pre-pass workspace, if any); anything else (long job lists) with a stream-ordered allocation for the job tables and the pre-pass workspace, freed in stream order. The
 // tables are copied from pageable memory, which the copy has consumed when it returns.
 static int run_async(const std::vector<Req> &reqs, hipStream_t s, int order = -1) {
     if (has_long(reqs))
@@ -1513,17 +1604,20 @@ static int run_async(const std::vector<Req> &reqs, hipStream_t s, int order = -1
     if (cached_launch(reqs, s, order, rc)) return rc;
     Batch bt;
     if (int e = plan_batch(reqs, bt)) return e;
-    if (table_free(bt)) return launch_batch(bt, nullptr, order >= 0 ? order : g_order.load(), s);
-    if (keep_and_launch(reqs, bt, s, order, rc)) return rc;
+    const bool by_value = table_free(bt);
+    if (by_value && !bt.ws_bytes) return launch_batch(bt, nullptr, order >= 0 ? order : g_order.load(), s);
+    if (!by_value && keep_and_launch(reqs, bt, s, order, rc)) return rc;
     void *dev = nullptr;
-    const size_t ws_at = align256(bt.table_bytes);
+    const size_t ws_at = by_value ? 0 : align256(bt.table_bytes);
     hipError_t e = hipMallocAsync(&dev, std::max<size_t>(ws_at + bt.ws_bytes, 256), s);
     if (e != hipSuccess) return hip_fail(e, "hipMallocAsync (tables and workspace)");
     bind(bt, static_cast<uint8_t *>(dev) + ws_at);
-    const std::vector<uint8_t> img = table_image(bt);
-    if (!img.empty() && (e = hipMemcpyAsync(dev, img.data(), img.size(), hipMemcpyHostToDevice, s)) != hipSuccess)
-        rc = hip_fail(e, "job table upload");
-    if (!rc) rc = launch_batch(bt, static_cast<const uint8_t *>(dev), order >= 0 ? order : g_order.load(), s);
+    if (!by_value) {
+        const std::vector<uint8_t> img = table_image(bt);
+        if (!img.empty() && (e = hipMemcpyAsync(dev, img.data(), img.size(), hipMemcpyHostToDevice, s)) != hipSuccess)
+            rc = hip_fail(e, "job table upload");
+    }
+    if (!rc) rc = launch_batch(bt, by_value ? nullptr : static_cast<const uint8_t *>(dev), order >= 0 ? order : g_order.load(), s);
     e = hipFreeAsync(dev, s);
     if (rc) return rc;
     return e == hipSuccess ? ES_HIP_OK : hip_fail(e, "hipFreeAsync");
@@ -1603,7 +1697,10 @@ int es_hip_matvec_multi_dev_noalloc(uint32_t type, const void *W, int cols, int 
     if (int rc = plan_batch(reqs, bt)) return rc;
     if (bt.mm.empty() && bt.mqg.empty() && bt.mbg.empty() && bt.mkg.empty() && bt.pkg.empty())
         return bt.mv.empty() ? ES_HIP_OK : launch_single(bt.mv[0], s);
-    const size_t ws_at = align256(bt.table_bytes), need = ws_at + bt.ws_bytes;
+    size_t need = align256(bt.table_bytes) + bt.ws_bytes;
+    const size_t ws_at = align256(bt.table_bytes);
+    if (type == ES_HIP_Q6_K && na >= 16)   // the limit holds whichever Q6_K kernel serves the call: the tiled one's pre-pass planes
+        need = std::max(need, align256((size_t)(cols / 256) * ((na + 63) / 64 * 64) * 256) + align256((size_t)(cols / 256) * ((na + 63) / 64 * 64) * 36));
     if (need > NOALLOC_SCRATCH)
         return fail(ES_HIP_EINVAL, "this product needs %zu bytes of job tables and workspace, more than the %zu bytes of the "
                                    "no-allocation scratch (use es_hip_matvec_multi_dev)", need, NOALLOC_SCRATCH);
@@ -1759,7 +1856,11 @@ int es_hip_set_direct_persistent(int on) {
 int es_hip_set_q2k_expert_max_batch(int n) { g_cfg_gen.fetch_add(1); return g_mx_max.exchange(n); }
 int es_hip_set_moe_gated(int on) { g_cfg_gen.fetch_add(1); return g_moe_gated.exchange(on != 0 ? 1 : 0); }
 int es_hip_set_batched32_direct(int on) { g_cfg_gen.fetch_add(1); return g_mbx_on.exchange(on ? 1 : 0); }
-int es_hip_set_q6k_persistent(int on) { g_cfg_gen.fetch_add(1); return esq::mm6_set_persistent(on); }
+int es_hip_set_q6k_persistent(int on) {
+    g_cfg_gen.fetch_add(1);
+    g_m6w_on.store(on ? 1 : 0);
+    return esq::mm6_set_persistent(on);
+}
 int es_hip_set_direct_mfma_tok64(int on) { g_cfg_gen.fetch_add(1); return g_mk_tok64.exchange(on ? 1 : 0); }
 
 double es_hip_plan_time_ms(es_hip_plan *p, int warmup, int iters, void *stream) {
