@@ -9,6 +9,7 @@
 // float and in double; expf follows glibc's method bit for bit (es_hip_expf.h).
 #include "es_hip_common.h"
 #include "es_hip_expf.h"
+#include "es_hip_q8k.h"
 #include "es_hip_seqsum.h"
 
 namespace esq {
@@ -35,9 +36,6 @@ __device__ __forceinline__ void store_per(float *p, const float (&v)[PER]) {
     *reinterpret_cast<f32x4_a4 *>(p) = f32x4_a4{v[0], v[1], v[2], v[3]};
     *reinterpret_cast<f32x4_a4 *>(p + 4) = f32x4_a4{v[4], v[5], v[6], v[7]};
 }
-__device__ __forceinline__ uint32_t pack_i8(int a, int b, int c, int d) {
-    return (uint32_t)(a & 0xff) | (uint32_t)(b & 0xff) << 8 | (uint32_t)(c & 0xff) << 16 | (uint32_t)d << 24;
-}
 
 // Eight consecutive elements e .. e + 7 of a row per thread: the kernels here are bound by issuing vector instructions where
 // every element forms its block's scale (three IEEE divisions each) and the workgroup synchronises per block: SwiGLU of
@@ -46,10 +44,7 @@ __device__ __forceinline__ uint32_t pack_i8(int a, int b, int c, int d) {
 // Q8_K block, so a block's scale is formed once per eight elements, its maximum and sums are lane moves and nothing
 // synchronises the workgroup. Lanes without elements (have false) are whole blocks; they take part in the lane moves.
 __device__ __forceinline__ void quant_per(const float (&v)[PER], bool have, int e, const QuantOut &o) {
-    float a = __builtin_fabsf(v[0]);   // a maximum is exact in any order
-#pragma unroll
-    for (int k = 1; k < PER; k++) a = __builtin_fmaxf(a, __builtin_fabsf(v[k]));
-    a = group_max<4>(a);
+    const float a = amax_quad(v);
     if (o.q80 && have) {   // quantize_q80: d = amax / 127, id = 1 / d (0 when d is 0), q = (int)(v * id +- 0.5)
         const float d = a / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
         int q[PER];
@@ -63,27 +58,18 @@ __device__ __forceinline__ void quant_per(const float (&v)[PER], bool have, int 
         *reinterpret_cast<uint32_t *>(blk + 8 + (e & 31)) = pack_i8(q[4], q[5], q[6], q[7]);
         if ((e & 31) == 0) *reinterpret_cast<float *>(blk) = d;
     }
-    if (o.q8k) {   // es_quantize_q8_K: id = 127 / amax, q = lrintf(v * id) clamped to +-127, d = amax / 127, bsums
-        a = __builtin_fmaxf(a, dpp_movf<0x141>(a));   // row_half_mirror, row_mirror: the other quads of the 16 lanes
-        a = __builtin_fmaxf(a, dpp_movf<0x140>(a));
-        const float amax = __builtin_fmaxf(a, __shfl_xor(a, 16));
-        int q[PER] = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (amax != 0.0f) {   // a zero block is all zeros (d, qs and bsums)
-            const float id = 127.0f / amax;
-#pragma unroll
-            for (int k = 0; k < PER; k++) {
-                const int t = static_cast<int>(__builtin_rintf(v[k] * id));   // lrintf: round to nearest even
-                q[k] = t > 127 ? 127 : t < -127 ? -127 : t;
-            }
-        }
-        const int s = group_sum<2>(q[0] + q[1] + q[2] + q[3] + q[4] + q[5] + q[6] + q[7]);   // sums of 16 consecutive qs
+    if (o.q8k) {
+        float d;
+        uint32_t lo, hi;
+        int bsum;
+        q8k_from8(v, a, d, lo, hi, bsum);
         if (have) {
             const int i = e & 255;
             uint8_t *blk = o.q8k + (size_t)(e >> 8) * 292;
-            *reinterpret_cast<uint32_t *>(blk + 4 + i) = pack_i8(q[0], q[1], q[2], q[3]);
-            *reinterpret_cast<uint32_t *>(blk + 8 + i) = pack_i8(q[4], q[5], q[6], q[7]);
-            if ((i & 15) == 0) reinterpret_cast<int16_t *>(blk + 260)[i >> 4] = static_cast<int16_t>(s);
-            if (i == 0) *reinterpret_cast<float *>(blk) = amax != 0.0f ? amax / 127.0f : 0.0f;
+            *reinterpret_cast<uint32_t *>(blk + 4 + i) = lo;
+            *reinterpret_cast<uint32_t *>(blk + 8 + i) = hi;
+            if ((i & 15) == 0) reinterpret_cast<int16_t *>(blk + 260)[i >> 4] = static_cast<int16_t>(bsum);
+            if (i == 0) *reinterpret_cast<float *>(blk) = d;
         }
     }
 }

@@ -240,7 +240,7 @@ hipError_t dequant_launch(uint32_t type, const void *src, float *dst, long n, hi
 hipError_t fdot_launch(uint32_t type, const void *W, size_t rb, int r0, int r1, int cols, const float *x, size_t xstride,
                        int na, float *y, size_t ystride, hipStream_t s);
 hipError_t route_softmax_launch(const float *logits, uint64_t ls, int ntok, int ne, int k, int norm_topk, int *sel, float *w,
-                                int kmax, hipStream_t s);
+                                int kmax, int *sel2, float *w2, hipStream_t s);
 
 // Device-routed MoE (es_hip_moe.hip): moe_n's grouping (src/es_engine.c:871-888) and the job tables of one layer's
 // gate/up and down launches built on the device from a routing in device memory, so a layer needs no host round trip.
@@ -284,6 +284,26 @@ struct MoeDevArgs {
     uint8_t *gu_ws, *dn_ws;          // MM: the experts' planes, packed in slot order (256-byte aligned)
 };
 hipError_t moe_group_build_launch(const MoeDevArgs &a, const MoeFamily &gu, const MoeFamily &dn, hipStream_t s);
+
+// Device-routed layers of a few tokens as (token, choice) pairs (es_hip_mv.hip): gate and up of every pair in one launch (mv:
+// the decode kernel's template job of one activation, pair p's rows into bgu), then SwiGLU, down and combine in
+// another, rt rows of a token per workgroup (mv.row_bytes: the down rows'). At most MOE_PAIR_K choices per token, a K-quant down.
+constexpr int MOE_PAIR_K = 16;
+struct MoePairs {
+    MvJob mv;
+    const int *sel;         // [ntok][k] experts (others than 0 .. n_exp - 1 contribute nothing)
+    const float *w;         // [ntok][k]
+    const uint8_t *const *gate, *const *up, *const *down;
+    const uint8_t *x;
+    uint64_t xstride;
+    float *bgu;             // [pair][2 ff]
+    float *out;
+    uint64_t ostride;
+    int k, n_exp, ff, n, rt, order;
+};
+hipError_t moe_pairs_gu_launch(const MoePairs &a, const MvLaunch &L, int pairs, hipStream_t s);
+size_t moe_pairs_down_lds(int k, int ff, int rt);
+hipError_t moe_pairs_down_launch(int type, const MoePairs &a, int ntok, hipStream_t s);
 
 constexpr int ACT_RMS_MAX_COLS = 16384;   // rmsnorm rows' squares are staged whole in LDS (128 KB of doubles)
 // Activation preparation (es_hip_act.hip): rows of fp32 values (plain, rmsnorm-ed, or the SwiGLU of gate|up rows) into

@@ -179,8 +179,11 @@ __device__ __forceinline__ float wave_fmax(float v) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// sel2 / w2 (optional, rows of k): the routing once more, for a caller who asked for it (two device copies behind the kernel
+// cost more than the kernel itself).
 __global__ __launch_bounds__(64) void route_softmax(const float *__restrict__ logits, uint64_t ls, int ne, int k, int norm_topk,
-                                                    int *__restrict__ sel, float *__restrict__ w, int kmax) {
+                                                    int *__restrict__ sel, float *__restrict__ w, int kmax, int *__restrict__ sel2,
+                                                    float *__restrict__ w2) {
     __shared__ __align__(16) float p[ROUTE_MAX_EXPERTS];
     __shared__ uint64_t tab[32];
     __shared__ float total;
@@ -268,7 +271,10 @@ __global__ __launch_bounds__(64) void route_softmax(const float *__restrict__ lo
             wsum += bv;   // w[j] = r[best]; wsum += w[j] (:802-803)
             if (l == j) { wj = bv; sj = be; }
         }
-        if (l < k) sel[(size_t)t * kmax + l] = sj;
+        if (l < k) {
+            sel[(size_t)t * kmax + l] = sj;
+            if (sel2) sel2[(size_t)t * k + l] = sj;
+        }
     } else {
         lds_sync();
         for (int j = 0; j < k; j++) {   // the reference's scan (:794-804), on one lane
@@ -280,6 +286,7 @@ __global__ __launch_bounds__(64) void route_softmax(const float *__restrict__ lo
                     if (!used && (be < 0 || p[e] > p[be])) be = e;
                 }
                 sel[(size_t)t * kmax + j] = be;
+                if (sel2) sel2[(size_t)t * k + j] = be;
                 wsum += p[be];
                 total = p[be];
             }
@@ -290,13 +297,17 @@ __global__ __launch_bounds__(64) void route_softmax(const float *__restrict__ lo
     }
     if (l == 0) total = norm_topk ? (wsum > 6.103515625e-5f ? wsum : 6.103515625e-5f) : 1.0f;   // :832
     lds_sync();
-    if (l < k) w[(size_t)t * kmax + l] = norm_topk ? wj / total : wj;
+    if (l < k) {
+        const float v = norm_topk ? wj / total : wj;
+        w[(size_t)t * kmax + l] = v;
+        if (w2) w2[(size_t)t * k + l] = v;
+    }
 }
 
 hipError_t route_softmax_launch(const float *logits, uint64_t ls, int ntok, int ne, int k, int norm_topk, int *sel, float *w,
-                                int kmax, hipStream_t s) {
+                                int kmax, int *sel2, float *w2, hipStream_t s) {
     if (ntok <= 0) return hipSuccess;
-    hipLaunchKernelGGL(route_softmax, dim3(ntok), dim3(64), 0, s, logits, ls, ne, k, norm_topk, sel, w, kmax);
+    hipLaunchKernelGGL(route_softmax, dim3(ntok), dim3(64), 0, s, logits, ls, ne, k, norm_topk, sel, w, kmax, sel2, w2);
     return hipGetLastError();
 }
 

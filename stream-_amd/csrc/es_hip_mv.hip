@@ -19,6 +19,8 @@
 // Reference kernels restated (integer parts and float order): src/es_quant.c:1013-1117 (scalar mv_*), 1252-1343 and
 // 1443-1469 (AVX2 Q4_0/Q5_0/Q4_K/Q6_K), 1344-1368 and src/es_q2k.c:127-190 (Q2_K), 1120-1175 and 1370-1394 (Q3_K, Q5_K).
 #include "es_hip_common.h"
+#include "es_hip_expf.h"
+#include "es_hip_q8k.h"
 
 #include <type_traits>
 
@@ -60,6 +62,23 @@ struct Term2 { float a, b; };
 
 enum { CH_FMA = 0, CH_MULADD = 1, CH_LANES = 2 };
 
+// An activation block as the lanes read it: a Q8_K (or Q8_0) block in global memory, or a Q8_K block in LDS laid out as qs at
+// 0, bsums at 256, d at 288, LACT_BYTES apart (16-byte aligned reads).
+struct GAct {
+    const uint8_t *a;
+    __device__ __forceinline__ operator const uint8_t *() const { return a; }
+    __device__ __forceinline__ float d() const { return ldg<float>(a); }
+    template <typename T> __device__ __forceinline__ T qs(int off) const { return ldg<T>(a + 4 + off); }
+    template <typename T> __device__ __forceinline__ T bs(int off) const { return ldg<T>(a + 260 + off); }
+};
+constexpr int LACT_BYTES = 304;
+struct LAct {
+    const uint8_t *a;
+    __device__ __forceinline__ float d() const { return *reinterpret_cast<const float *>(a + 288); }
+    template <typename T> __device__ __forceinline__ T qs(int off) const { return *reinterpret_cast<const T *>(a + off); }
+    template <typename T> __device__ __forceinline__ T bs(int off) const { return *reinterpret_cast<const T *>(a + 256 + off); }
+};
+
 // ---------------------------------------------------------------------------------------------------------------------
 // Per-format lane work: Raw (the bytes one lane loads), Wt (unpacked), Act (activation slice), Ints (integer partials)
 
@@ -73,15 +92,15 @@ template <> struct Lane<ES_HIP_Q4_K> {
     struct Wt { uint32_t lo[8], hi[8]; int sc0, sc1, mn0, mn1; float d, dmin; };
     struct Ints { int dot, aux; };
 
-    static __device__ __forceinline__ void load_act(const uint8_t *a, int k, Act &x) {
-        x.d = ldg<float>(a);
+    template <typename A> static __device__ __forceinline__ void load_act(const A &a, int k, Act &x) {
+        x.d = a.d();
 #pragma unroll
         for (int v = 0; v < 2; v++) {
-            const uint4 l = ldg<uint4>(a + 4 + 64 * k + 16 * v), h = ldg<uint4>(a + 4 + 64 * k + 32 + 16 * v);
+            const uint4 l = a.template qs<uint4>(64 * k + 16 * v), h = a.template qs<uint4>(64 * k + 32 + 16 * v);
             x.lo[4 * v] = l.x; x.lo[4 * v + 1] = l.y; x.lo[4 * v + 2] = l.z; x.lo[4 * v + 3] = l.w;
             x.hi[4 * v] = h.x; x.hi[4 * v + 1] = h.y; x.hi[4 * v + 2] = h.z; x.hi[4 * v + 3] = h.w;
         }
-        const uint2 b = ldg<uint2>(a + 260 + 8 * k);   // bsums 4k .. 4k+3, the last 8 bytes of the record for k = 3
+        const uint2 b = a.template bs<uint2>(8 * k);   // bsums 4k .. 4k+3, the last 8 bytes of the record for k = 3
         x.bs0 = static_cast<int16_t>(b.x) + static_cast<int16_t>(b.x >> 16);
         x.bs1 = static_cast<int16_t>(b.y) + static_cast<int16_t>(b.y >> 16);
     }
@@ -170,14 +189,14 @@ template <> struct Lane<ES_HIP_Q6_K> {
     struct Ints { int dot, aux; };
 
     static __device__ __forceinline__ int grp(int k, int m) { return 8 * (k >> 1) + 2 * (k & 1) + (m & 1) + 4 * (m >> 1); }
-    static __device__ __forceinline__ void load_act(const uint8_t *a, int k, Act &x) {
-        x.d = ldg<float>(a);
+    template <typename A> static __device__ __forceinline__ void load_act(const A &a, int k, Act &x) {
+        x.d = a.d();
 #pragma unroll
         for (int m = 0; m < 4; m++) {
             const int g = grp(k, m);
-            const uint4 v = ldg<uint4>(a + 4 + 16 * g);
+            const uint4 v = a.template qs<uint4>(16 * g);
             x.y[m][0] = v.x; x.y[m][1] = v.y; x.y[m][2] = v.z; x.y[m][3] = v.w;
-            x.bs[m] = ldg<int16_t>(a + 260 + 2 * g);
+            x.bs[m] = a.template bs<int16_t>(2 * g);
         }
     }
     static __device__ __forceinline__ void zero_act(Act &x) {
@@ -254,15 +273,15 @@ template <> struct Lane<ES_HIP_Q3_K> {
     struct Wt { uint32_t c[4][4]; int sc[4]; float d; };
     struct Ints { int dot, aux; };
 
-    static __device__ __forceinline__ void load_act(const uint8_t *a, int k, Act &x) {
+    template <typename A> static __device__ __forceinline__ void load_act(const A &a, int k, Act &x) {
         const int n = k >> 1, half = k & 1;
-        x.d = ldg<float>(a);
+        x.d = a.d();
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int g = 8 * n + 2 * j + half;
-            const uint4 v = ldg<uint4>(a + 4 + 16 * g);
+            const uint4 v = a.template qs<uint4>(16 * g);
             x.y[j][0] = v.x; x.y[j][1] = v.y; x.y[j][2] = v.z; x.y[j][3] = v.w;
-            x.bs[j] = ldg<int16_t>(a + 260 + 2 * g);
+            x.bs[j] = a.template bs<int16_t>(2 * g);
         }
     }
     static __device__ __forceinline__ void zero_act(Act &x) {
@@ -345,15 +364,15 @@ template <> struct Lane<ES_HIP_Q2_K> {
     struct Wt { uint32_t q[4]; int scl[4], mn[4]; float d, dmin; };
     struct Ints { int dot, aux; };
 
-    static __device__ __forceinline__ void load_act(const uint8_t *a, int k, Act &x) {
+    template <typename A> static __device__ __forceinline__ void load_act(const A &a, int k, Act &x) {
         const int h = k >> 1, part = k & 1;
-        x.d = ldg<float>(a);
+        x.d = a.d();
 #pragma unroll
         for (int s = 0; s < 4; s++) {
             const int g = 8 * h + 2 * s + part;
-            const uint4 v = ldg<uint4>(a + 4 + 16 * g);
+            const uint4 v = a.template qs<uint4>(16 * g);
             x.y[s][0] = v.x; x.y[s][1] = v.y; x.y[s][2] = v.z; x.y[s][3] = v.w;
-            x.bs[s] = ldg<int16_t>(a + 260 + 2 * g);
+            x.bs[s] = a.template bs<int16_t>(2 * g);
         }
     }
     static __device__ __forceinline__ void zero_act(Act &x) {
@@ -586,7 +605,7 @@ __device__ __forceinline__ void mv_body(const MvJob &J, int order) {
             for (int t = 0; t < NT; t++) {
                 if (live && t < nt) {
                     const int q = J.arow ? ldg<int>(J.arow + t0 + t) : t0 + t;
-                    L::load_act(J.act + (size_t)q * J.astride + (size_t)b * AB, k, act[t]);
+                    L::load_act(GAct{J.act + (size_t)q * J.astride + (size_t)b * AB}, k, act[t]);
                 }
                 else L::zero_act(act[t]);
             }
@@ -809,6 +828,126 @@ __global__ __launch_bounds__(WAVE * W, ESQ_MIN_WAVES) void mv_kernel_mixed(const
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------------------
+// Routed pairs: an MoE layer of a few tokens, whose (token, choice) pairs mostly name different experts. Every pair is a
+// product of its own against the expert its choice names, so the layer needs no grouping and no job tables: the gate and up
+// products of all pairs in one launch, and in a second one the SwiGLU, the requantization, the down products and the
+// weighted combine, a workgroup taking some rows of one token for all of its choices. Config 5's experts at one token: the
+// grouping (6.6 us), SwiGLU (2.9), down (9.4) and combine (2.9) launches became one of 11.6 us, the layer 33.9 -> 23.7 us. With
+// the SwiGLU in a launch of its own it took the same at one token and 3 us more at four. It is bound by its chain of
+// dependent steps (choice, expert's address, weights; h; products; chains; combine).
+
+template <int F, int W>
+__global__ __launch_bounds__(WAVE * W) void mv_pairs(MoePairs A) {
+    const int p = blockIdx.z, e = A.sel[p];
+    if (e < 0 || e >= A.n_exp) return;   // (contributes nothing, as in the grouping)
+    MvJob J = A.mv;
+    J.W = blockIdx.y ? A.up[e] : A.gate[e];
+    J.act = A.x + (size_t)(p / A.k) * A.xstride;
+    J.y = A.bgu + (size_t)p * 2 * A.ff + (size_t)blockIdx.y * A.ff;
+    mv_body<F, 1, W, false>(uniform_job(J), A.order);
+}
+
+// Rows [r0, r0 + rt) of token blockIdx.y: wave w takes the choices w, w + 8, ..., 16 blocks of the choice's rows at a time (four
+// lanes a block, as in mv_body), two such groups of raw loads in flight; the first ones go out before the activations are
+// formed. The workgroup forms its token's h = SwiGLU(gate, up) as Q8_K blocks in LDS itself: every workgroup of a token
+// repeats that (about 2 us of vector work at 8 choices of 768), so rt grows with the tokens and the launch stays about one
+// workgroup per CU. Float orders as in swiglu_q8k, mv_body and moe_combine.
+template <int F>
+__global__ __launch_bounds__(512) void moe_down_pairs(MoePairs A) {
+    using L = Lane<F>;
+    constexpr int LPB = Fmt<F>::LPB, BB = Fmt<F>::BB, SLOTS = WAVE / LPB, U = 2;
+    extern __shared__ __align__(16) uint8_t sm[];
+    __shared__ uint64_t tab[32];
+    __shared__ float wl[MOE_PAIR_K];
+    const int t = blockIdx.y, rt = A.rt, r0 = blockIdx.x * rt, nbk = A.ff / 256, units = rt * nbk, kc = A.k;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, slot = lane / LPB, k = lane % LPB;
+    const bool contract = A.order == ES_HIP_ORDER_X86_CONTRACT;
+    uint8_t *const acts = sm;                                                                       // [choice][block]
+    Term2 *const term = reinterpret_cast<Term2 *>(sm + (size_t)kc * nbk * LACT_BYTES);     // [choice][row][block]
+    float *const ye = reinterpret_cast<float *>(term + (size_t)kc * units);                         // [choice][row]
+
+    typename L::Raw raw[U];
+    auto expert = [&](int j) { const int e = A.sel[t * kc + j]; return e >= 0 && e < A.n_exp ? e : -1; };
+    auto load = [&](const uint8_t *W, int u0) {   // units u0 + slot, u0 + SLOTS + slot (clamped; past the last is not used)
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            const int u = min(u0 + SLOTS * i + slot, units - 1), row = u / nbk, b = u - row * nbk;
+            L::load_raw(W + (size_t)min(r0 + row, A.n - 1) * A.mv.row_bytes + (size_t)b * BB, k, raw[i]);
+        }
+    };
+    int e0 = wave < kc ? expert(wave) : -1;
+    if (e0 >= 0) load(A.down[e0], 0);
+    if (tid < kc) wl[tid] = expert(tid) >= 0 ? A.w[t * kc + tid] : 0.0f;
+    {
+        static constexpr uint64_t T[32] = ESQ_EXPF_TABLE;
+        if (tid < 32) tab[tid] = T[tid];
+        lds_sync();
+        const int per = nbk * 32, total = kc * per;   // 8 elements a thread, 32 lanes a block
+        for (int it = tid; it - (tid & 63) < total; it += 512) {
+            const int i = min(it, total - 1), j = i / per, e = (i - j * per) * 8;
+            const float *g = A.bgu + (size_t)(t * kc + j) * 2 * A.ff + e;
+            float v[8], u[8];
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const float4 a = ldg<float4>(g + 4 * q), b = ldg<float4>(g + A.ff + 4 * q);
+                v[4 * q] = a.x; v[4 * q + 1] = a.y; v[4 * q + 2] = a.z; v[4 * q + 3] = a.w;
+                u[4 * q] = b.x; u[4 * q + 1] = b.y; u[4 * q + 2] = b.z; u[4 * q + 3] = b.w;
+            }
+#pragma unroll
+            for (int q = 0; q < 8; q++) v[q] = v[q] / (1.0f + esq_expf_tab(-v[q], tab)) * u[q];
+            float d;
+            uint32_t lo, hi;
+            int bsum;
+            q8k_from8(v, d, lo, hi, bsum);
+            if (it < total) {
+                uint8_t *blk = acts + (size_t)(i >> 5) * LACT_BYTES;
+                const int at = e & 255;
+                *reinterpret_cast<uint2 *>(blk + at) = make_uint2(lo, hi);
+                if ((at & 15) == 0) *reinterpret_cast<int16_t *>(blk + 256 + (at >> 3)) = static_cast<int16_t>(bsum);
+                if (at == 0) *reinterpret_cast<float *>(blk + 288) = d;
+            }
+        }
+    }
+    lds_sync();
+    for (int j = wave; j < kc; j += 8) {
+        const int e = j == wave ? e0 : expert(j);
+        if (e < 0) {
+            for (int u = lane; u < units; u += WAVE) term[(size_t)j * units + u] = Term2{0.0f, 0.0f};
+            continue;
+        }
+        const uint8_t *W = A.down[e];
+        for (int u0 = 0; u0 < units; u0 += U * SLOTS) {
+            if (j != wave || u0) load(W, u0);
+#pragma unroll
+            for (int i = 0; i < U; i++) {
+                const int u = min(u0 + SLOTS * i + slot, units - 1), b = u % nbk;
+                typename L::Act x;
+                L::load_act(LAct{acts + (size_t)(j * nbk + b) * LACT_BYTES}, k, x);
+                typename L::Wt w;
+                L::unpack(raw[i], k, w);
+                typename L::Ints v = L::ints(w, x);
+                v.dot = group_sum<LPB>(v.dot);
+                v.aux = group_sum<LPB>(v.aux);
+                if (k == 0 && u0 + SLOTS * i + slot < units) term[(size_t)j * units + u] = L::term(w, x, v, contract);
+            }
+        }
+    }
+    lds_sync();
+    for (int i = tid; i < kc * rt; i += 512) {   // the reference's sum over a row's blocks, per choice
+        const Term2 *e = term + (size_t)i * nbk;
+        float s = 0.0f;
+        for (int b = 0; b < nbk; b++) s = contract ? __builtin_fmaf(e[b].a, e[b].b, s) : s + e[b].a * e[b].b;
+        ye[i] = s;
+    }
+    lds_sync();
+    if (tid < rt && r0 + tid < A.n) {   // the choices in order
+        float s = 0.0f;
+        for (int j = 0; j < kc; j++) s = s + wl[j] * ye[j * rt + tid];
+        stg<float>(A.out + (size_t)t * A.ostride + r0 + tid, s);
+    }
+}
+
 }  // namespace esq
 
 // ---------------------------------------------------------------------------------------------------------------------
@@ -884,6 +1023,55 @@ hipError_t mv_launch(const MvLaunch &L, const MvJob *jobs, int njobs, const MvJo
     }
     hipLaunchKernelGGL(fn, grid, dim3(WAVE * L.waves), L.lds, s, A);
     return hipGetLastError();
+}
+
+template <int F> static hipError_t pairs_gu(const MoePairs &A, const MvLaunch &L, int pairs, hipStream_t s) {
+    const auto fn = L.waves == 4 ? mv_pairs<F, 4> : mv_pairs<F, 8>;
+    if (L.lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           static_cast<int>(L.lds));
+        if (e != hipSuccess) return e;
+    }
+    const int tiles = (A.mv.r1 - A.mv.r0 + A.mv.rows_per_wg - 1) / A.mv.rows_per_wg;
+    hipLaunchKernelGGL(fn, dim3(tiles, 2, pairs), dim3(WAVE * L.waves), L.lds, s, A);
+    return hipGetLastError();
+}
+hipError_t moe_pairs_gu_launch(const MoePairs &A, const MvLaunch &L, int pairs, hipStream_t s) {
+    if (L.seg_loop || (L.waves != 4 && L.waves != 8)) return hipErrorInvalidValue;
+    switch (L.type) {
+    case ES_HIP_Q4_0: return pairs_gu<ES_HIP_Q4_0>(A, L, pairs, s);
+    case ES_HIP_Q5_0: return pairs_gu<ES_HIP_Q5_0>(A, L, pairs, s);
+    case ES_HIP_Q8_0: return pairs_gu<ES_HIP_Q8_0>(A, L, pairs, s);
+    case ES_HIP_Q2_K: return pairs_gu<ES_HIP_Q2_K>(A, L, pairs, s);
+    case ES_HIP_Q3_K: return pairs_gu<ES_HIP_Q3_K>(A, L, pairs, s);
+    case ES_HIP_Q4_K: return pairs_gu<ES_HIP_Q4_K>(A, L, pairs, s);
+    case ES_HIP_Q5_K: return pairs_gu<ES_HIP_Q5_K>(A, L, pairs, s);
+    case ES_HIP_Q6_K: return pairs_gu<ES_HIP_Q6_K>(A, L, pairs, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+size_t moe_pairs_down_lds(int k, int ff, int rt) {
+    const size_t nbk = ff / 256;
+    return k * nbk * LACT_BYTES + (size_t)k * rt * nbk * sizeof(Term2) + (size_t)k * rt * sizeof(float);
+}
+template <int F> static hipError_t pairs_down(const MoePairs &A, int ntok, hipStream_t s) {
+    const auto fn = moe_down_pairs<F>;
+    const size_t lds = moe_pairs_down_lds(A.k, A.ff, A.rt);
+    if (lds > 60 * 1024) return hipErrorInvalidValue;   // (the caller chooses rt)
+    hipLaunchKernelGGL(fn, dim3((A.n + A.rt - 1) / A.rt, ntok), dim3(512), lds, s, A);
+    return hipGetLastError();
+}
+hipError_t moe_pairs_down_launch(int type, const MoePairs &A, int ntok, hipStream_t s) {
+    if (A.k < 1 || A.k > MOE_PAIR_K || A.ff % 256 || A.rt < 1 || A.rt > 512) return hipErrorInvalidValue;
+    switch (type) {
+    case ES_HIP_Q2_K: return pairs_down<ES_HIP_Q2_K>(A, ntok, s);
+    case ES_HIP_Q3_K: return pairs_down<ES_HIP_Q3_K>(A, ntok, s);
+    case ES_HIP_Q4_K: return pairs_down<ES_HIP_Q4_K>(A, ntok, s);
+    case ES_HIP_Q5_K: return pairs_down<ES_HIP_Q5_K>(A, ntok, s);
+    case ES_HIP_Q6_K: return pairs_down<ES_HIP_Q6_K>(A, ntok, s);
+    }
+    return hipErrorInvalidValue;
 }
 
 // ---------------------------------------------------------------------------------------------------------------------

@@ -2643,8 +2643,23 @@ void es_hip_moe_ctx_destroy(es_hip_moe_ctx *c) {
 
 namespace {
 
-// one layer from a routing already in the context's sel / w (device), in stream order
-int moe_ctx_layer(es_hip_moe_ctx *c, int N, const void *x, size_t xstride, float *out, size_t ostride, hipStream_t s) {
+// The pair form of a layer (es_hip_mv.hip): the products of R choices, each on its own, without grouping and job tables. It
+// saves about 15 us of launches and reads an expert chosen c times c times (the repeats at about 10 TB/s, from the L2 and the
+// Infinity Cache), so it is taken while the repeats of a random routing stay under 128 MB. Measured per layer (us, grouped /
+// pairs): 128 experts of 3.06 MB, top 8: 1 token 33.9 / 23.7, 4 46.8 / 35.3, 8 63.2 / 49.9, 16 (141 MB) 86.5 / 76.3, 32 (440
+// MB) 110 / 130; 64 of 2.06 MB (Q2_K), top 8: 28.0 / 19.7, 44.8 / 31.3, 58.4 / 44.0 (at 16 its grouped form runs on the
+// expert-sized kernel); 16 of 1.8 MB, top 4: 25.3 / 16.3, 31.3 / 20.0, 36.1 / 23.9, 43.8 / 32.9.
+bool moe_pairs_ok(const es_hip_moe_ctx *c, int N, size_t expert_bytes) {
+    const int R = N * c->k;
+    if (!c->h_q8k || c->k > esq::MOE_PAIR_K || R > 256) return false;
+    double unused = c->n_exp;
+    for (int t = 0; t < N; t++) unused *= 1.0 - (double)c->k / c->n_exp;
+    return (R - (c->n_exp - unused)) * (double)expert_bytes <= 128e6;
+}
+
+// one layer from a routing in device memory, in stream order
+int moe_ctx_layer(es_hip_moe_ctx *c, int N, const int *sel, const float *w, const void *x, size_t xstride, float *out, size_t ostride,
+                  hipStream_t s) {
     const int R = N * c->k, umax = std::min(c->n_exp, R), n = c->n, ff = c->ff;
     FmtInfo fg, fd;
     fmt_info(c->gt, fg);
@@ -2666,9 +2681,47 @@ int moe_ctx_layer(es_hip_moe_ctx *c, int N, const void *x, size_t xstride, float
     if (int rc = moe_family(c, c->dt, n, ff, umax, 1, R, expect, N, c->w_down0, c->ha, nullptr, c->hstride, c->bye, (uint64_t)n,
                             c->dn_ws, D))
         return rc;
+    if (G.F.kind == esq::MOE_FAM_MV && D.F.kind == esq::MOE_FAM_MV &&
+        moe_pairs_ok(c, N, 2 * (size_t)ff * (n / fg.be) * fg.bb + (size_t)n * (ff / fd.be) * fd.bb)) {
+        MoeLaunch P;   // the gate/up launch sized for products of one activation
+        if (int rc = moe_family(c, c->gt, ff, n, R, 2, R, 1.0, 1, c->w_gate0, static_cast<const uint8_t *>(x), nullptr, xs, c->bgu,
+                                2 * (uint64_t)ff, nullptr, P))
+            return rc;
+        if (P.F.kind == esq::MOE_FAM_MV && !P.L.seg_loop) {
+            esq::MoePairs a{};
+            a.mv = P.F.mv;
+            a.mv.arow = nullptr;
+            a.mv.na = a.mv.nt = 1;
+            a.mv.tile0 = 0;
+            a.sel = sel;
+            a.w = w;
+            a.gate = c->dgate;
+            a.up = c->dup;
+            a.down = c->ddown;
+            a.x = static_cast<const uint8_t *>(x);
+            a.xstride = xs;
+            a.bgu = c->bgu;
+            a.out = out;
+            a.ostride = ostride ? ostride : (uint64_t)n;
+            a.k = c->k;
+            a.n_exp = c->n_exp;
+            a.ff = ff;
+            a.n = n;
+            a.order = g_order.load();
+            // rows per workgroup: about one workgroup per CU, a multiple of 8 in 8 .. 128 that fits 48 KB of LDS
+            a.rt = std::min(128, std::max(8, (int)((long)n * N / device().cus) / 8 * 8));
+            while (a.rt > 8 && esq::moe_pairs_down_lds(a.k, ff, a.rt) > 48 * 1024) a.rt -= 8;
+            if (esq::moe_pairs_down_lds(a.k, ff, a.rt) <= 48 * 1024) {
+                hipError_t e = esq::moe_pairs_gu_launch(a, P.L, R, s);
+                a.mv.row_bytes = (uint64_t)(ff / fd.be) * fd.bb;
+                if (e == hipSuccess) e = esq::moe_pairs_down_launch((int)c->dt, a, N, s);
+                return e == hipSuccess ? ES_HIP_OK : hip_fail(e, "MoE pair launch");
+            }
+        }
+    }
     esq::MoeDevArgs a{};
-    a.sel = c->sel;
-    a.w = c->w;
+    a.sel = sel;
+    a.w = w;
     a.ntok = N;
     a.k = c->k;
     a.n_exp = c->n_exp;
@@ -2752,15 +2805,18 @@ int es_hip_moe_ctx_run_logits(es_hip_moe_ctx *c, int N, const float *logits, siz
     if (N == 0) return ES_HIP_OK;
     if (!logits) return fail(ES_HIP_EINVAL, "null logits");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // (outputs at an odd alignment, which the kernel cannot store to, are copied)
+    int *sel2 = reinterpret_cast<uintptr_t>(sel_out) & 3 ? nullptr : sel_out;
+    float *w2 = reinterpret_cast<uintptr_t>(w_out) & 3 ? nullptr : w_out;
     hipError_t e = esq::route_softmax_launch(logits, lstride ? lstride : (uint64_t)c->n_exp, N, c->n_exp, c->k, norm_topk,
-                                             c->sel, c->w, c->k, s);
+                                             c->sel, c->w, c->k, sel2, w2, s);
     if (e != hipSuccess) return hip_fail(e, "routing launch");
     const size_t pairs = (size_t)N * c->k;
-    if (sel_out && (e = hipMemcpyAsync(sel_out, c->sel, pairs * sizeof(int), hipMemcpyDeviceToDevice, s)) != hipSuccess)
+    if (sel_out != sel2 && (e = hipMemcpyAsync(sel_out, c->sel, pairs * sizeof(int), hipMemcpyDeviceToDevice, s)) != hipSuccess)
         return hip_fail(e, "routing copy");
-    if (w_out && (e = hipMemcpyAsync(w_out, c->w, pairs * sizeof(float), hipMemcpyDeviceToDevice, s)) != hipSuccess)
+    if (w_out != w2 && (e = hipMemcpyAsync(w_out, c->w, pairs * sizeof(float), hipMemcpyDeviceToDevice, s)) != hipSuccess)
         return hip_fail(e, "routing copy");
-    return moe_ctx_layer(c, N, x, xstride, out, ostride, s);
+    return moe_ctx_layer(c, N, c->sel, c->w, x, xstride, out, ostride, s);
 }
 
 int es_hip_moe_ctx_run(es_hip_moe_ctx *c, int N, const int *sel, const float *w, const void *x, size_t xstride, float *out,
@@ -2773,10 +2829,16 @@ int es_hip_moe_ctx_run(es_hip_moe_ctx *c, int N, const int *sel, const float *w,
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t pairs = (size_t)N * c->k;
     hipError_t e;
-    if ((e = hipMemcpyAsync(c->sel, sel, pairs * sizeof(int), hipMemcpyDeviceToDevice, s)) != hipSuccess ||
-        (e = hipMemcpyAsync(c->w, w, pairs * sizeof(float), hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_fail(e, "routing copy");
-    return moe_ctx_layer(c, N, x, xstride, out, ostride, s);
+    // the layer's kernels read the caller's routing in stream order; only at an odd alignment, which they cannot, a copy of it
+    if (reinterpret_cast<uintptr_t>(sel) & 3) {
+        if ((e = hipMemcpyAsync(c->sel, sel, pairs * sizeof(int), hipMemcpyDeviceToDevice, s)) != hipSuccess) return hip_fail(e, "routing copy");
+        sel = c->sel;
+    }
+    if (reinterpret_cast<uintptr_t>(w) & 3) {
+        if ((e = hipMemcpyAsync(c->w, w, pairs * sizeof(float), hipMemcpyDeviceToDevice, s)) != hipSuccess) return hip_fail(e, "routing copy");
+        w = c->w;
+    }
+    return moe_ctx_layer(c, N, sel, w, x, xstride, out, ostride, s);
 }
 
 }  // extern "C"
@@ -2902,7 +2964,7 @@ int es_hip_route_softmax_dev(const float *logits, size_t lstride, int ntok, int 
     if (ntok > 1 && lstride < (size_t)n_exp) return fail(ES_HIP_EINVAL, "logit stride %zu < %d", lstride, n_exp);
     if ((reinterpret_cast<uintptr_t>(logits) | reinterpret_cast<uintptr_t>(sel) | reinterpret_cast<uintptr_t>(w)) & 3)
         return fail(ES_HIP_EINVAL, "logits, sel and w must be 4-byte aligned");
-    hipError_t e = esq::route_softmax_launch(logits, lstride, ntok, n_exp, k, norm_topk, sel, w, kmax,
+    hipError_t e = esq::route_softmax_launch(logits, lstride, ntok, n_exp, k, norm_topk, sel, w, kmax, nullptr, nullptr,
                                              static_cast<hipStream_t>(stream));
     return e == hipSuccess ? ES_HIP_OK : hip_fail(e, "routing launch");
 }
