@@ -299,8 +299,7 @@ int es_hip_set_direct_mfma_min_batch(int n);
 /* The direct-activation kernel's minimum tile count per product (default 128; twice that for rows longer than 4096):
  * below it a product has too few workgroups to fill the device. Returns the previous value. */
 int es_hip_set_direct_mfma_min_tiles(int n);
-/* Q5_K products with at least n activations (default 8) run on the direct-activation matrix-core kernel (a third int8
- * plane for the fifth bit); below it, or with it off (n <= 0), on the vector kernel. Results are identical on both. Returns
+/* Q5_K products with at least n activations (default 8) run on the direct-activation matrix-core kernel; below it, or with it off (n <= 0), on the vector kernel. Results are identical on both. Returns
  * the previous value. */
 int es_hip_set_q5k_mfma_min_batch(int n);
 /* Q3_K products with at least n activations (default 8) run on the direct-activation matrix-core kernel (two int8 planes of
@@ -329,16 +328,16 @@ int es_hip_set_batched32_direct(int on);
  * persistent launch of the tiled kernel: one workgroup per CU copies the activations into LDS once and streams its row
  * tiles back to back. With 0 every product runs on the tiled kernel, one workgroup per tile. Results are identical. */
 int es_hip_set_q6k_persistent(int on);
-/* Q4_K and Q3_K products that take the direct-activation kernel and have an even number (at least 2) of superblocks per
- * row, with no gathered activations, run, with on != 0, in one persistent launch per format, each workgroup computing a
+/* Q4_K, Q5_K and Q3_K products that take the direct-activation kernel and have an even number (at least 2) of superblocks
+ * per row, with no gathered activations, run, with on != 0, in one persistent launch per format, each workgroup computing a
  * host-scheduled list of tiles with its loads running ahead across tile boundaries, in one of two forms: two workgroups
- * per CU (tiles of 64 rows x 128 or 64 activations), or, for Q4_K, one workgroup of 8 waves per CU (tiles of 64 rows x
- * 128 activations; four waves stage the activations and the unpacked weights in LDS for the four that run the matrix
- * cores). on = 1 (the default) picks the second form for Q4_K launches of at least 4 tiles of 128 activations per CU
- * (config 2's three prefill products in one launch), the first otherwise; on = 2 takes the second for every Q4_K
- * launch, on = 3 the first for every launch. Q4_K products of this kind take the persistent launch at any tile count
- * (config 2's 2048 x 8192 down product shares the launch with gate and up). Results are identical in every form.
- * Returns the previous setting. */
+ * per CU (Q4_K, Q3_K; tiles of 64 rows x 128 or 64 activations), or, for Q4_K and Q5_K, one workgroup of 8 waves per CU
+ * (every tile of 64 rows x 128, or x 64, activations; four waves stage the activations and the unpacked weights in LDS for
+ * the four that run the matrix cores). on = 1 (the default) picks the second form for Q5_K, and for Q4_K launches of at
+ * most one tile or at least four tiles of 128 activations per CU, the first otherwise; on = 2 takes the second for every
+ * Q4_K launch, on = 3 the first for every launch (Q5_K: one workgroup per tile). Q4_K products of this kind take the
+ * persistent launch at any tile count (config 2's 2048 x 8192 down product shares the launch with gate and up). Results
+ * are identical in every form. Returns the previous setting. */
 int es_hip_set_direct_persistent(int on);
 /* Q5_K and Q3_K products on the direct-activation kernel that would have fewer than 256 tiles of 64 rows x 128
  * activations run, with on != 0 (the default) and at least 64 activations, in tiles of 64 activations (twice the

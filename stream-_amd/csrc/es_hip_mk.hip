@@ -40,8 +40,8 @@
 // D: lane l, register i holds D[4*(l/16)+i][l%16]) are those of the device, checked by the parity tests.
 //
 // Q5_K (src/es_quant.c:1153-1175): Q4_K's layout plus qh[32] after the scales, bit 2c (2c + 1) of qh[l] the fifth bit of
-// element l of sub-block 2c (2c + 1), so q = q4 + 16 q5. A third int8 plane q5 * sc (<= 63) goes through the matrix cores
-// and dot = D_lo + 8 D_hi + 16 D_q5, exact. Its epilogue is the reference's scalar mv_q5_K (the x86 build has no AVX2
+// element l of sub-block 2c (2c + 1). q * sc (<= 1953) goes through the matrix cores as two int8 planes,
+// q * sc = 256 hi + lo, so dot = 256 D_hi + D_lo, exact (three planes before, 13 MFMAs a tile instead of 9). Its epilogue is the reference's scalar mv_q5_K (the x86 build has no AVX2
 // Q5_K kernel and no FMA in it): s += y.d * (d * dot - dmin * mins) with every product and sum rounded, in every order.
 //
 // Q3_K (src/es_quant.c:1120-1150, 1369-1395): 110-byte superblocks hmask[32] | qs[64] | scales[12] | d, 2-byte aligned,
@@ -114,50 +114,57 @@ template <int F> struct BOps {   // one row tile's B operands for one superblock
     v4h mn;
     float d, dm;
 };
-template <> struct BOps<ES_HIP_Q5_K> {
-    v4i lo[4], hi[4], q5[4];
-    v4h mn;
-    float d, dm;
-};
 template <> struct BOps<ES_HIP_Q3_K> {   // dm unused (0)
     v4i lo[4], hi[4];
     float d, dm;
 };
 
-// scale_min_k4 (src/es_quant.c:75-83) byte-parallel: the two int8 planes of the four slices (three for Q5_K) and the
-// mins operand
+// scale_min_k4 (src/es_quant.c:75-83) byte-parallel: the two int8 planes of the four slices and the mins operand
 template <int F> __device__ __forceinline__ void build_b(const WRaw<F> &w, int lg, BOps<F> &B) {
     const uint4 h = w.h;
     const uint32_t sc0 = h.y & 0x3f3f3f3fu, sc1 = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
     const uint32_t mn0 = h.z & 0x3f3f3f3fu, mn1 = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
     // v_perm_b32 selectors putting byte 2*(lg >> 1) (sel0) or 2*(lg >> 1) + 1 (sel1) into both 16-bit halves
     const uint32_t sel0 = 0x0c000c00u + (uint32_t)(2 * (lg >> 1)) * 0x00010001u, sel1 = sel0 + 0x00010001u;
-    const uint32_t l0 = sc0 & 0x07070707u, h0 = (sc0 >> 3) & 0x07070707u;
-    const uint32_t l1 = sc1 & 0x07070707u, h1 = (sc1 >> 3) & 0x07070707u;
-    const uint32_t slw[4] = {__builtin_amdgcn_perm(0, l0, sel0), __builtin_amdgcn_perm(0, l0, sel1),
-                             __builtin_amdgcn_perm(0, l1, sel0), __builtin_amdgcn_perm(0, l1, sel1)};
-    const uint32_t shw[4] = {__builtin_amdgcn_perm(0, h0, sel0), __builtin_amdgcn_perm(0, h0, sel1),
-                             __builtin_amdgcn_perm(0, h1, sel0), __builtin_amdgcn_perm(0, h1, sel1)};
     const uint32_t qa[2][4] = {{w.q0.x, w.q0.y, w.q0.z, w.q0.w}, {w.q1.x, w.q1.y, w.q1.z, w.q1.w}};
-#pragma unroll
-    for (int s = 0; s < 4; s++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t v = qa[s >> 1][i];
-            const uint32_t nib = (s & 1) ? (v >> 4) & 0x0f0f0f0fu : v & 0x0f0f0f0fu;
-            B.lo[s][i] = (int)pk_mul_u16(nib, slw[s]);   // byte * scale <= 105: no carry between bytes
-            B.hi[s][i] = (int)pk_mul_u16(nib, shw[s]);
-        }
-    if constexpr (F == ES_HIP_Q5_K) {   // slice s takes sub-block j = 2 (lg >> 1) + 4 (s >> 1) + (s & 1): bit j of its qh bytes
+    if constexpr (F == ES_HIP_Q5_K) {   // q * sc <= 1953 as 256 hi + lo, lo signed: v + 128 in 16-bit lanes (even, odd bytes)
         const uint32_t scw[4] = {__builtin_amdgcn_perm(0, sc0, sel0), __builtin_amdgcn_perm(0, sc0, sel1),
                                  __builtin_amdgcn_perm(0, sc1, sel0), __builtin_amdgcn_perm(0, sc1, sel1)};
-        const uint32_t hw[4] = {w.qh.x, w.qh.y, w.qh.z, w.qh.w};
+        // slice s takes sub-block j = 2 (lg >> 1) + 4 (s >> 1) + (s & 1): bit j of its qh bytes, shifted by the lane's part once
+        const uint32_t j2 = 2u * (uint32_t)(lg >> 1);
+        const uint32_t hw[4] = {w.qh.x >> j2, w.qh.y >> j2, w.qh.z >> j2, w.qh.w >> j2};
+        const u16x2 r128 = {128, 128};
 #pragma unroll
         for (int s = 0; s < 4; s++) {
-            const uint32_t j = 2 * (lg >> 1) + 4 * (s >> 1) + (s & 1);
+            const int j = 4 * (s >> 1) + (s & 1);
+            const u16x2 sc = __builtin_bit_cast(u16x2, scw[s]);
 #pragma unroll
-            for (int i = 0; i < 4; i++) B.q5[s][i] = (int)pk_mul_u16((hw[i] >> j) & 0x01010101u, scw[s]);   // <= 63
+            for (int i = 0; i < 4; i++) {
+                const uint32_t v = qa[s >> 1][i], n = (s & 1) ? v >> 4 : v;          // codes' low bits in every byte's low nibble
+                const uint32_t h5 = j <= 4 ? hw[i] << (4 - j) : hw[i] >> (j - 4);    // their fifth bits at bit 4
+                const uint32_t q = (n & 0x0f0f0f0fu) | (h5 & 0x10101010u);
+                const uint32_t e = __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, q & 0x00ff00ffu) * sc + r128));
+                const uint32_t o = __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, (q >> 8) & 0x00ff00ffu) * sc + r128));
+                B.hi[s][i] = (int)__builtin_amdgcn_perm(o, e, 0x07030501u);
+                B.lo[s][i] = (int)(__builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u);
+            }
         }
+    } else {
+        const uint32_t l0 = sc0 & 0x07070707u, h0 = (sc0 >> 3) & 0x07070707u;
+        const uint32_t l1 = sc1 & 0x07070707u, h1 = (sc1 >> 3) & 0x07070707u;
+        const uint32_t slw[4] = {__builtin_amdgcn_perm(0, l0, sel0), __builtin_amdgcn_perm(0, l0, sel1),
+                                 __builtin_amdgcn_perm(0, l1, sel0), __builtin_amdgcn_perm(0, l1, sel1)};
+        const uint32_t shw[4] = {__builtin_amdgcn_perm(0, h0, sel0), __builtin_amdgcn_perm(0, h0, sel1),
+                                 __builtin_amdgcn_perm(0, h1, sel0), __builtin_amdgcn_perm(0, h1, sel1)};
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t v = qa[s >> 1][i];
+                const uint32_t nib = (s & 1) ? (v >> 4) & 0x0f0f0f0fu : v & 0x0f0f0f0fu;
+                B.lo[s][i] = (int)pk_mul_u16(nib, slw[s]);   // byte * scale <= 105: no carry between bytes
+                B.hi[s][i] = (int)pk_mul_u16(nib, shw[s]);
+            }
     }
     // mins operand: k positions 4lg .. 4lg+3 meet bsums 4lg .. 4lg+3, i.e. sub-blocks 2lg and 2lg+1, each twice. Each half
     // is built as 1024 + m (byte m under the exponent of 1024) and 1024 subtracted exactly.
@@ -212,7 +219,6 @@ template <int F> __device__ __forceinline__ void b_ready(const BOps<F> &B) {
 #pragma unroll
     for (int s = 0; s < 4; s++) {
         asm volatile("" ::"v"(B.lo[s]), "v"(B.hi[s]));
-        if constexpr (F == ES_HIP_Q5_K) asm volatile("" ::"v"(B.q5[s]));
     }
     if constexpr (F != ES_HIP_Q3_K) asm volatile("" ::"v"(B.mn));
     asm volatile("" ::"v"(B.d), "v"(B.dm));
@@ -228,10 +234,6 @@ template <int F> struct MAcc {   // the matrix-core results of one 16 x 16 tile 
     v4i lo, hi;
     v4f mn;
 };
-template <> struct MAcc<ES_HIP_Q5_K> {
-    v4i lo, hi, q5;
-    v4f mn;
-};
 template <> struct MAcc<ES_HIP_Q3_K> {
     v4i lo, hi;
 };
@@ -245,12 +247,10 @@ template <int F> struct Pend {   // a tile's results waiting for their epilogue,
 template <int F> __device__ __forceinline__ void mma(const AOps &a, const BOps<F> &B, MAcc<F> &m) {
     m.lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a.x[0], B.lo[0], v4i{0, 0, 0, 0}, 0, 0, 0);
     m.hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a.x[0], B.hi[0], v4i{0, 0, 0, 0}, 0, 0, 0);
-    if constexpr (F == ES_HIP_Q5_K) m.q5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a.x[0], B.q5[0], v4i{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
     for (int s = 1; s < 4; s++) {
         m.lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a.x[s], B.lo[s], m.lo, 0, 0, 0);
         m.hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a.x[s], B.hi[s], m.hi, 0, 0, 0);
-        if constexpr (F == ES_HIP_Q5_K) m.q5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a.x[s], B.q5[s], m.q5, 0, 0, 0);
     }
     if constexpr (F != ES_HIP_Q3_K) m.mn = __builtin_amdgcn_mfma_f32_16x16x16f16(a.bs, B.mn, v4f{0, 0, 0, 0}, 0, 0, 0);
 }
@@ -259,13 +259,12 @@ template <int F, bool CONTRACT>
 __device__ __forceinline__ void epilogue(const MAcc<F> &m, float d, float dm, const v4f &yd, v4f &s) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        int dot = m.lo[i] + 8 * m.hi[i];
+        const int dot = m.lo[i] + (F == ES_HIP_Q5_K ? 256 : 8) * m.hi[i];
         if constexpr (F == ES_HIP_Q3_K) {   // s += (y.d * d) * tot
             const float a = yd[i] * d;
             if constexpr (CONTRACT) s[i] = __builtin_fmaf(a, static_cast<float>(dot), s[i]);
             else s[i] = s[i] + a * static_cast<float>(dot);
         } else {
-            if constexpr (F == ES_HIP_Q5_K) dot += 16 * m.q5[i];
             const float q = dm * m.mn[i];   // the mins are exact integers in the f32 accumulator
             if constexpr (CONTRACT)
                 s[i] = __builtin_fmaf(yd[i], __builtin_fmaf(d, static_cast<float>(dot), -q), s[i]);
@@ -275,7 +274,7 @@ __device__ __forceinline__ void epilogue(const MAcc<F> &m, float d, float dm, co
     }
 }
 
-// One tile step: 9 MFMAs (13 for Q5_K, 8 for Q3_K) interleaved with the step's vector work (the previous tile's epilogue) and the
+// One tile step: 9 MFMAs (8 for Q3_K) interleaved with the step's vector work (the previous tile's epilogue) and the
 // next tile's LDS reads: 1 MFMA : 3 VALU : 1 LDS read.
 template <int NMFMA> __device__ __forceinline__ void step_schedule() {
 #pragma unroll
@@ -474,7 +473,7 @@ __global__ __launch_bounds__(64 * MK_WAVES, MK_WG_PER_CU) void mk_kernel(const M
             p1.yd = A[tt & 1].yd;
             p1.d = B.d;
             p1.dm = B.dm;
-            step_schedule<F == ES_HIP_Q5_K ? 13 : F == ES_HIP_Q3_K ? 8 : 9>();
+            step_schedule<F == ES_HIP_Q3_K ? 8 : 9>();
             __builtin_amdgcn_sched_barrier(0);
         }
         wait_vmcnt<NW>();   // this wave's copies of superblock b + 1 (the weights of b + 2 may still be in flight)
@@ -693,7 +692,7 @@ __device__ __forceinline__ void pk_body(const PkTile *__restrict__ tiles, int k0
             p1.yd = A[tt & 1].yd;
             p1.d = B.d;
             p1.dm = B.dm;
-            step_schedule<F == ES_HIP_Q5_K ? 13 : F == ES_HIP_Q3_K ? 8 : 9>();
+            step_schedule<F == ES_HIP_Q3_K ? 8 : 9>();
             __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (t64) {
@@ -795,11 +794,11 @@ __global__ __launch_bounds__(256, 2) void pk_kernel(const PkTile *__restrict__ t
     else pk_body<F, CONTRACT, false>(tiles, k0, nt, smem);
 }
 
-// ---- the wave-specialised persistent form (Q4_K) ------------------------------------------------------------------------
-// One workgroup of 8 waves per CU runs a host-scheduled list of tiles (64 rows x 128 activations) as a stream of items
+// ---- the wave-specialised persistent form (Q4_K, Q5_K) ------------------------------------------------------------------------
+// One workgroup of 8 waves per CU runs a host-scheduled list of tiles (64 rows x T = 128 or 64 activations) as a stream of items
 // (tile, superblock), as pk_body does, but splits each item's work by kind over the waves of a SIMD:
-//   waves 0-3 (matrix waves): wave m reads the B operands of rows 16m .. 16m+15 from LDS and runs the item's 8 tile steps
-//     (72 MFMAs and the float epilogue of the tiles two steps back) and the tile's stores, as pk_body does;
+//   waves 0-3 (matrix waves): wave m reads the B operands of rows 16m .. 16m+15 from LDS and runs the item's T / 16 tile steps
+//     (9 MFMAs each and the float epilogue of the tiles two steps back) and the tile's stores, as pk_body does;
 //   waves 4-7 (staging waves): wave 4 + u loads a quarter of the item's activations (values, scales, bsums) and the
 //     weights of rows 16u .. 16u+15 into registers three items ahead, and one item ahead writes them into LDS: the values
 //     swizzled as in mk_kernel, the bsums converted to halves, the weights unpacked into the B operands (build_b).
@@ -807,9 +806,9 @@ __global__ __launch_bounds__(256, 2) void pk_kernel(const PkTile *__restrict__ t
 // load is an ordinary (compiler-counted) buffer load into registers, so no wait drains loads issued after the ones it
 // needs. LDS: two activation slots and two B-operand slots (item i in slots i & 1) and the tile records; one barrier per
 // item: at barrier i, item i's slots are complete and item i - 1's are free.
-struct WsGeom {
-    using SL = MkSlot<128>;
-    static constexpr uint32_t ACT = SL::BYTES;            // an activation slot (the 128-activation layout of mk_kernel)
+template <int T> struct WsGeom {
+    using SL = MkSlot<T>;
+    static constexpr uint32_t ACT = SL::BYTES;            // an activation slot (mk_kernel's layout for T activations)
     static constexpr uint32_t PLT = 9 * 1024;             // one row tile's B operands: 9 chunks of 16 bytes per lane
     static constexpr uint32_t PLS = 4 * PLT;              // a B-operand slot: 4 row tiles
     static constexpr uint32_t PL0 = 2 * ACT, REC0 = PL0 + 2 * PLS;
@@ -844,11 +843,12 @@ __device__ __forceinline__ WsRec ws_rec(uint32_t rec0, int k) {
 }
 
 // the matrix waves (m = 0 .. 3)
-template <int F, bool CONTRACT>
+template <int F, int T, bool CONTRACT>
 __device__ __forceinline__ void ws_matrix(uint8_t *smem, int nt, int nitems, int m) {
-    using G = WsGeom;
-    using SL = MkSlot<128>;
-    constexpr bool FUSED = CONTRACT;
+    using G = WsGeom<T>;
+    using SL = MkSlot<T>;
+    constexpr bool FUSED = CONTRACT && F != ES_HIP_Q5_K;
+    constexpr int NT = T / 16;
     const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
     const uint32_t smem0 = lds_addr(smem);
     uint32_t xo[4];
@@ -857,16 +857,16 @@ __device__ __forceinline__ void ws_matrix(uint8_t *smem, int nt, int nitems, int
         const int nat = 4 * (lg >> 1) + 8 * (s >> 1) + 2 * (s & 1) + (lg & 1);
         xo[s] = SL::QS + lr * TROW + 16 * (nat ^ lr);
     }
-    const uint32_t bso = SL::BS + lg * (128 * 8) + lr * 8, ydo = SL::D + 16 * lg;
+    const uint32_t bso = SL::BS + lg * (T * 8) + lr * 8, ydo = SL::D + 16 * lg;
     auto aload = [&](const uint32_t (&xa)[4], uint32_t ba, uint32_t ya, int tt, AOps &A) {
 #pragma unroll
         for (int s = 0; s < 4; s++) A.x[s] = lds_ld<v4i>(xa[s] + 16 * TROW * tt);
         A.bs = lds_ld<v4h>(ba + 128 * tt);
         A.yd = lds_ld<v4f>(ya + 64 * tt);
     };
-    v4f acc[8];
+    v4f acc[NT];
 #pragma unroll
-    for (int t = 0; t < 8; t++) acc[t] = v4f{0, 0, 0, 0};
+    for (int t = 0; t < NT; t++) acc[t] = v4f{0, 0, 0, 0};
     Pend<F> p0, p1;
     p0.m = MAcc<F>{};
     p0.yd = v4f{0, 0, 0, 0};
@@ -874,8 +874,8 @@ __device__ __forceinline__ void ws_matrix(uint8_t *smem, int nt, int nitems, int
     p1 = p0;
     const Pend<F> pzero = p0;
     auto flush = [&](const WsRec &r) {   // as pk_body's: the pending epilogues, the stores, the accumulators cleared
-        epilogue<F, FUSED>(p0.m, p0.d, p0.dm, p0.yd, acc[6]);
-        epilogue<F, FUSED>(p1.m, p1.d, p1.dm, p1.yd, acc[7]);
+        epilogue<F, FUSED>(p0.m, p0.d, p0.dm, p0.yd, acc[NT - 2]);
+        epilogue<F, FUSED>(p1.m, p1.d, p1.dm, p1.yd, acc[NT - 1]);
         p0 = pzero;
         p1 = pzero;
         const int row = 16 * m + lr;
@@ -883,7 +883,7 @@ __device__ __forceinline__ void ws_matrix(uint8_t *smem, int nt, int nitems, int
         const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)r.y, (short)0, (int)yrange, 0x00020000);
         uint32_t yoff = row < r.rows ? (uint32_t)(4 * lg) * r.ystride4 + 4u * (uint32_t)row : 0x80000000u;
 #pragma unroll
-        for (int tt = 0; tt < 8; tt++)
+        for (int tt = 0; tt < NT; tt++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const float v = acc[tt][i];
@@ -891,7 +891,7 @@ __device__ __forceinline__ void ws_matrix(uint8_t *smem, int nt, int nitems, int
                 yoff += i < 3 ? r.ystride4 : 13 * r.ystride4;
             }
 #pragma unroll
-        for (int t = 0; t < 8; t++) acc[t] = v4f{0, 0, 0, 0};
+        for (int t = 0; t < NT; t++) acc[t] = v4f{0, 0, 0, 0};
     };
     int k = 0, j = 0;
     WsRec rc = ws_rec(smem0 + G::REC0, 0);
@@ -917,11 +917,11 @@ __device__ __forceinline__ void ws_matrix(uint8_t *smem, int nt, int nitems, int
         aload(xa, ba, ya, 0, A[0]);
         __builtin_amdgcn_sched_barrier(0);   // every operand of the item's first step requested before its first MFMA
 #pragma unroll
-        for (int tt = 0; tt < 8; tt++) {
-            if (tt + 1 < 8) aload(xa, ba, ya, tt + 1, A[(tt + 1) & 1]);
+        for (int tt = 0; tt < NT; tt++) {
+            if (tt + 1 < NT) aload(xa, ba, ya, tt + 1, A[(tt + 1) & 1]);
             MAcc<F> cur;
             mma<F>(A[tt & 1], B, cur);
-            epilogue<F, FUSED>(p0.m, p0.d, p0.dm, p0.yd, acc[(tt + 6) % 8]);
+            epilogue<F, FUSED>(p0.m, p0.d, p0.dm, p0.yd, acc[(tt + NT - 2) % NT]);
             p0 = p1;
             p1.m = cur;
             p1.yd = A[tt & 1].yd;
@@ -938,21 +938,22 @@ __device__ __forceinline__ void ws_matrix(uint8_t *smem, int nt, int nitems, int
 }
 
 // the staging waves (u = 0 .. 3)
-template <int F>
+template <int F, int T>
 __device__ __forceinline__ void ws_stage(uint8_t *smem, int nt, int nitems, int u) {
-    using G = WsGeom;
-    using SL = MkSlot<128>;
+    using G = WsGeom<T>;
+    using SL = MkSlot<T>;
+    constexpr int TW = T / 4, NC = TW / 4;   // activations a wave stages, value chunks per lane
     using FM = MkFmt<F>;
     const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
     const uint32_t smem0 = lds_addr(smem);
-    struct Set {   // one item's loads: 8 value chunks (activations 32u + 4c + lane/16), the scale (activation 32u + lane %
-                   // 32), 8 bsums (activation 32u + lane/2, half lane & 1), the weights' header and two qs chunks
-        u32x4 q[8], bs, h, q0, q1;
+    struct Set {   // one item's loads: NC value chunks (activations TW u + 4c + lane/16), the scale (activation TW u + lane %
+                   // TW), 8 bsums (activation TW u + (lane/2) % TW, half lane & 1), the weights' header, two qs chunks, qh
+        u32x4 q[NC], bs, h, q0, q1, qh;
         uint32_t d;
     };
     struct LTile {   // the load stream's tile: buffer resources and per-lane offsets
         __amdgpu_buffer_rsrc_t ar, wr;
-        uint32_t q[8], bs, d, wo;
+        uint32_t q[NC], bs, d, wo;
         int nbk;
     };
     auto ltile = [&](int k) {
@@ -962,9 +963,9 @@ __device__ __forceinline__ void ws_stage(uint8_t *smem, int nt, int nitems, int 
         t.wr = __builtin_amdgcn_make_buffer_rsrc((void *)r.w, (short)0, (int)0xffffffffu, 0x00020000);
         auto act_off = [&](int a) { return (uint32_t)min(r.tok0 + a, r.na - 1) * r.astride; };
 #pragma unroll
-        for (int c = 0; c < 8; c++) t.q[c] = act_off(32 * u + 4 * c + (lane >> 4)) + 4 + 16 * (lane & 15);
-        t.bs = act_off(32 * u + (lane >> 1)) + 260 + 16 * (lane & 1);
-        t.d = act_off(32 * u + (lane & 31));
+        for (int c = 0; c < NC; c++) t.q[c] = act_off(TW * u + 4 * c + (lane >> 4)) + 4 + 16 * (lane & 15);
+        t.bs = act_off(TW * u + (lane >> 1) % TW) + 260 + 16 * (lane & 1);
+        t.d = act_off(TW * u + lane % TW);
         t.wo = (uint32_t)min(16 * u + lr, r.rows - 1) * r.row_bytes;
         t.nbk = r.nbk;
         return t;
@@ -981,18 +982,20 @@ __device__ __forceinline__ void ws_stage(uint8_t *smem, int nt, int nitems, int 
         S.h = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(t.wr, (int)t.wo, sw, 0));
         S.q0 = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(t.wr, (int)(t.wo + FM::QS + 16 * lg), sw, 0));
         S.q1 = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(t.wr, (int)(t.wo + FM::QS + 64 + 16 * lg), sw, 0));
+        if constexpr (F == ES_HIP_Q5_K)
+            S.qh = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(t.wr, (int)(t.wo + FM::QH + 16 * (lg & 1)), sw, 0));
     };
-    // LDS destinations within a slot: value chunk c of activation a = 32u + 4c + lane/16 at row a, position
-    // (lane % 16) ^ (a & 15); the scale at D + 4a (lanes 32-63 repeat lanes 0-31); the bsums' halves as mk_kernel lays
+    // LDS destinations within a slot: value chunk c of activation a = TW u + 4c + lane/16 at row a, position
+    // (lane % 16) ^ (a & 15); the scale at D + 4a (lanes past TW repeat the first ones); the bsums' halves as mk_kernel lays
     // them out ([lg][activation][4]); this row tile's B operands at chunk c, 16 bytes per lane
-    uint32_t qd[8];
+    uint32_t qd[NC];
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const int a = 32 * u + 4 * c + (lane >> 4);
+    for (int c = 0; c < NC; c++) {
+        const int a = TW * u + 4 * c + (lane >> 4);
         qd[c] = SL::QS + (uint32_t)a * TROW + 16u * (uint32_t)((lane & 15) ^ (a & 15));
     }
-    const uint32_t dd = SL::D + 4u * (uint32_t)(32 * u + (lane & 31));
-    const uint32_t bd = SL::BS + (uint32_t)(2 * (lane & 1)) * (128 * 8) + (uint32_t)(32 * u + (lane >> 1)) * 8;
+    const uint32_t dd = SL::D + 4u * (uint32_t)(TW * u + lane % TW);
+    const uint32_t bd = SL::BS + (uint32_t)(2 * (lane & 1)) * (T * 8) + (uint32_t)(TW * u + (lane >> 1) % TW) * 8;
     const uint32_t pd = G::PL0 + (uint32_t)u * G::PLT + 16u * (uint32_t)lane;
     auto put_value = [&](const Set &S, int slot, int c) {
         *reinterpret_cast<u32x4 *>(smem + (uint32_t)slot * G::ACT + qd[c]) = S.q[c];
@@ -1008,13 +1011,14 @@ __device__ __forceinline__ void ws_stage(uint8_t *smem, int nt, int nitems, int 
             hv[c] = (uint32_t)__builtin_bit_cast(uint16_t, e0) | (uint32_t)__builtin_bit_cast(uint16_t, e1) << 16;
         }
         *reinterpret_cast<uint2 *>(ab + bd) = make_uint2(hv[0], hv[1]);
-        *reinterpret_cast<uint2 *>(ab + bd + 128 * 8) = make_uint2(hv[2], hv[3]);
+        *reinterpret_cast<uint2 *>(ab + bd + T * 8) = make_uint2(hv[2], hv[3]);
     };
     auto put_operands = [&](const Set &S, int slot) {
         WRaw<F> wr;
         wr.h = make_uint4(S.h.x, S.h.y, S.h.z, S.h.w);
         wr.q0 = make_uint4(S.q0.x, S.q0.y, S.q0.z, S.q0.w);
         wr.q1 = make_uint4(S.q1.x, S.q1.y, S.q1.z, S.q1.w);
+        if constexpr (F == ES_HIP_Q5_K) wr.qh = make_uint4(S.qh.x, S.qh.y, S.qh.z, S.qh.w);
         BOps<F> B;
         build_b<F>(wr, lg, B);
         uint8_t *pb = smem + pd + (uint32_t)slot * G::PLS;
@@ -1040,7 +1044,7 @@ __device__ __forceinline__ void ws_stage(uint8_t *smem, int nt, int nitems, int 
     };
     auto issue = [&](Set &S) {
 #pragma unroll
-        for (int c = 0; c < 8; c++) S.q[c] = ld_value(lt, lj, c);
+        for (int c = 0; c < NC; c++) S.q[c] = ld_value(lt, lj, c);
         ld_scales(lt, lj, S);
         ld_weights(lt, lj, S);
         advance();
@@ -1050,7 +1054,7 @@ __device__ __forceinline__ void ws_stage(uint8_t *smem, int nt, int nitems, int 
     issue(S1);
     issue(S2);
 #pragma unroll
-    for (int c = 0; c < 8; c++) put_value(S0, 0, c);
+    for (int c = 0; c < NC; c++) put_value(S0, 0, c);
     put_scales(S0, 0);
     put_operands(S0, 0);
     // item i: the loads of item i + 3 into the set item i used, interleaved with the writes of item i + 1 into slots
@@ -1060,7 +1064,7 @@ __device__ __forceinline__ void ws_stage(uint8_t *smem, int nt, int nitems, int 
         lds_sync();
         const int sl = (i + 1) & 1;
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
+        for (int c = 0; c < NC; c++) {
             Sl.q[c] = ld_value(lt, lj, c);
             __builtin_amdgcn_sched_barrier(0);
             put_value(Sp, sl, c);
@@ -1085,9 +1089,9 @@ __device__ __forceinline__ void ws_stage(uint8_t *smem, int nt, int nitems, int 
     if (i < nitems) period(S1, S2, i++);
 }
 
-template <int F, bool CONTRACT>
+template <int F, int T, bool CONTRACT>
 __global__ __launch_bounds__(512, 1) void ws_kernel(const PkTile *__restrict__ tiles, const int *__restrict__ wgptr) {
-    using G = WsGeom;
+    using G = WsGeom<T>;
     __shared__ __align__(16) uint8_t smem[G::BYTES];
     const int k0 = wgptr[blockIdx.x], nt = wgptr[blockIdx.x + 1] - k0;
     if (nt <= 0) return;
@@ -1098,8 +1102,8 @@ __global__ __launch_bounds__(512, 1) void ws_kernel(const PkTile *__restrict__ t
     int nitems = 0;   // every wave counts the items (tile records in LDS, read as scalars)
     for (int k = 0; k < nt; k++) nitems += ws_rec(lds_addr(smem) + G::REC0, k).nbk;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if (wave < 4) ws_matrix<F, CONTRACT>(smem, nt, nitems, wave);
-    else ws_stage<F>(smem, nt, nitems, wave - 4);
+    if (wave < 4) ws_matrix<F, T, CONTRACT>(smem, nt, nitems, wave);
+    else ws_stage<F, T>(smem, nt, nitems, wave - 4);
 }
 
 }  // namespace
@@ -1141,12 +1145,19 @@ static void pk_launch_fmt(bool contract, const PkTile *tiles, const int *wgptr, 
     else hipLaunchKernelGGL((pk_kernel<F, false>), dim3(grid), dim3(256), 0, s, tiles, wgptr, g64);
 }
 
-hipError_t ws_launch(int type, const PkTile *tiles, const int *wgptr, int grid, int order, hipStream_t s) {
-    if (type != ES_HIP_Q4_K) return hipErrorInvalidValue;
-    if (order == ES_HIP_ORDER_X86_CONTRACT)
-        hipLaunchKernelGGL((ws_kernel<ES_HIP_Q4_K, true>), dim3(grid), dim3(512), 0, s, tiles, wgptr);
-    else
-        hipLaunchKernelGGL((ws_kernel<ES_HIP_Q4_K, false>), dim3(grid), dim3(512), 0, s, tiles, wgptr);
+hipError_t ws_launch(int type, int tok, const PkTile *tiles, const int *wgptr, int grid, int order, hipStream_t s) {
+    const bool contract = order == ES_HIP_ORDER_X86_CONTRACT, t64 = tok == 64;
+    if (tok != 64 && tok != 128) return hipErrorInvalidValue;
+    if (type == ES_HIP_Q4_K) {
+        const auto k = t64 ? (contract ? ws_kernel<ES_HIP_Q4_K, 64, true> : ws_kernel<ES_HIP_Q4_K, 64, false>)
+                           : (contract ? ws_kernel<ES_HIP_Q4_K, 128, true> : ws_kernel<ES_HIP_Q4_K, 128, false>);
+        hipLaunchKernelGGL(k, dim3(grid), dim3(512), 0, s, tiles, wgptr);
+    } else if (type == ES_HIP_Q5_K) {   // never fused
+        const auto k = t64 ? ws_kernel<ES_HIP_Q5_K, 64, false> : ws_kernel<ES_HIP_Q5_K, 128, false>;
+        hipLaunchKernelGGL(k, dim3(grid), dim3(512), 0, s, tiles, wgptr);
+    } else {
+        return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 

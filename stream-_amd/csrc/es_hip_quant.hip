@@ -362,7 +362,8 @@ struct PkGroup {
     std::vector<esq::PkTile> tiles;   // in workgroup order
     std::vector<int> wgptr;           // grid + 1 entries: workgroup g takes tiles[wgptr[g] .. wgptr[g + 1])
     int grid = 0, g64 = 0;            // workgroups [0, g64) take the 64-wide tiles
-    bool ws = false;                  // the wave-specialised form (Q4_K): one workgroup per CU, 128-wide tiles only
+    bool ws = false;                  // the wave-specialised form (Q4_K, Q5_K): one workgroup per CU, tiles of ws_tok activations
+    int ws_tok = 128;
     size_t off = 0;                   // byte offset of the tiles in the device image; wgptr follows them
 };
 
@@ -478,13 +479,14 @@ bool mk_eligible(const Req &q) {
 std::atomic<int> g_pk_on{1};
 std::atomic<uint64_t> g_cfg_gen{0};   // bumped by every setting that changes how a batch is planned
 
-// The persistent direct kernel: Q4_K / Q3_K products that the direct kernels take (at least g_mk_min / g_mk3_min
+// The persistent direct kernel: Q4_K / Q3_K / Q5_K products that the direct kernels take (at least g_mk_min / g_mk3_min / g_mk5_min
 // activations), with an even number (>= 2) of superblocks per row and no gathered activations, every activation row
 // within 4 GiB of act and a tile's outputs (128 activations) within 2^31 bytes of its first.
 bool pk_eligible(const Req &q) {
     if (!g_pk_on.load() || q.arow || q.ints || q.r1 <= q.r0) return false;
-    if (q.type != ES_HIP_Q4_K && q.type != ES_HIP_Q3_K) return false;
-    const int mn = q.type == ES_HIP_Q3_K ? g_mk3_min.load() : g_mk_min.load(), nbk = q.cols / 256;
+    if (q.type != ES_HIP_Q4_K && q.type != ES_HIP_Q3_K && (q.type != ES_HIP_Q5_K || g_pk_on.load() == 3)) return false;
+    const int mn = q.type == ES_HIP_Q3_K ? g_mk3_min.load() : q.type == ES_HIP_Q5_K ? g_mk5_min.load() : g_mk_min.load();
+    const int nbk = q.cols / 256;
     if (mn <= 0 || q.na < mn || nbk < 2 || (nbk & 1)) return false;
     const size_t stride = q.astride ? q.astride : (size_t)nbk * 292;
     // (a tile's stores past its activations fall outside its range only when consecutive activations' outputs are at
@@ -504,17 +506,26 @@ double pk_cost(int nbk, bool t64) { return nbk * (t64 ? 0.6 : 1.0) + 1.0; }
 // each set, all tiles of a row tile go to one XCD (workgroup g runs on XCD g % 8: its L2 reads the row tile's weights
 // once), row tiles are spread over the XCDs and tiles over an XCD's workgroups longest first, each to the least loaded.
 // Returns false when some workgroup would get more than PK_MAX_TILES tiles.
-// The form of a persistent launch: the wave-specialised kernel (one workgroup per CU, 128-wide tiles) measured faster
-// on config 2's three products in one launch (1152 tiles: 75-77 us against 85-86 us), even with gate and up alone (1024
-// tiles), and slower when the tiles leave CUs idle (the down product alone, 128 tiles: 47 us against 37 us).
-bool pk_ws(const PkGroup &g, int cus) {
+// The form of a persistent launch: the wave-specialised kernel (one workgroup per CU) measured faster on config 2's three
+// products in one launch (1152 tiles of 128: 75-77 us against 85-86 us) and even with gate and up alone (1024 tiles).
+// Tiles of 64 activations while every CU gets at most one of them (a short product: at 128 wide half the CUs idle), of 128
+// while every CU gets at most one of those, and from four per CU; in between the two-workgroup form packs better (8192 x
+// 2048 twice, us, two-workgroup / 64 / 128 wide: T = 64 13.6 / 12.6 / 16.7, 128 19.6 / 20.7 / 18.0, 256 30.7 / 36.8 / 31.4;
+// 2048 x 8192: T = 64 36.3 / 31.2 / 41.3, 512 37.7 / 34.2 / 42.9, 1024 58.0 / 64.2 / 53.0; 4096 x 4096: T = 256 21.9 / 19.7 /
+// 25.0, 512 31.3 / 34.4 / 28.1). Q5_K has no two-workgroup form: against its per-tile launches (three planes, before) 8192
+// x 2048 twice T = 8 19.3 -> 13.2, 512 67.3 -> 61.7; 2048 x 8192 T = 333 45.7 -> 41.8.
+bool pk_ws(PkGroup &g, int cus) {
     const int on = g_pk_on.load();
-    if (g.type != ES_HIP_Q4_K || on == 3) return false;
-    if (on == 2) return true;
-    long tiles = 0;
-    for (const PkGroup::Prod &p : g.prods)
-        tiles += (long)((p.r1 - p.r0 + esq::MK_ROWS - 1) / esq::MK_ROWS) * ((p.na + 127) / 128);
-    return tiles >= 4L * std::max(cus, 8);
+    if (g.type == ES_HIP_Q3_K || on == 3) return false;
+    long t128 = 0, t64 = 0;
+    for (const PkGroup::Prod &p : g.prods) {
+        const long rt = (p.r1 - p.r0 + esq::MK_ROWS - 1) / esq::MK_ROWS;
+        t128 += rt * ((p.na + 127) / 128);
+        t64 += rt * ((p.na + 63) / 64);
+    }
+    cus = std::max(cus, 8);
+    g.ws_tok = t64 <= cus ? 64 : 128;
+    return on == 2 || g.type == ES_HIP_Q5_K || t64 <= cus || t128 <= cus || t128 >= 4L * cus;
 }
 
 bool pk_schedule_form(PkGroup &g, int cus);
@@ -524,7 +535,7 @@ bool pk_schedule_form(PkGroup &g, int cus);
 bool pk_schedule(PkGroup &g, int cus) {
     g.ws = pk_ws(g, cus);
     if (pk_schedule_form(g, cus)) return true;
-    if (!g.ws) return false;
+    if (!g.ws || g.type == ES_HIP_Q5_K) return false;
     g.ws = false;
     return pk_schedule_form(g, cus);
 }
@@ -541,7 +552,7 @@ bool pk_schedule_form(PkGroup &g, int cus) {
         const PkGroup::Prod &p = g.prods[pi];
         const int rts = (p.r1 - p.r0 + esq::MK_ROWS - 1) / esq::MK_ROWS;
         const bool t64 = !g.ws && (p.na <= 64 || pk_cost(p.nbk, false) > mean);
-        const int T = t64 ? 64 : 128;
+        const int T = g.ws ? g.ws_tok : t64 ? 64 : 128;
         for (int rt = 0; rt < rts; rt++)
             for (int t0 = 0; t0 < p.na; t0 += T)
                 (t64 ? v64 : v128).push_back(Tl{pi, rt, t0, std::min(T, p.na - t0), t64, pk_cost(p.nbk, t64)});
@@ -1163,7 +1174,7 @@ int launch_batch(const Batch &bt, const uint8_t *tables, int order, hipStream_t 
         if (!tables) return fail(ES_HIP_EINVAL, "the persistent kernel needs its tile tables on the device");
         const esq::PkTile *tl = reinterpret_cast<const esq::PkTile *>(tables + g.off);
         const int *wp = reinterpret_cast<const int *>(tables + g.off + align256(g.tiles.size() * sizeof(esq::PkTile)));
-        if ((e = g.ws ? esq::ws_launch(g.type, tl, wp, g.grid, order, s) : esq::pk_launch(g.type, tl, wp, g.grid, g.g64, order, s)) !=
+        if ((e = g.ws ? esq::ws_launch(g.type, g.ws_tok, tl, wp, g.grid, order, s) : esq::pk_launch(g.type, tl, wp, g.grid, g.g64, order, s)) !=
             hipSuccess)
             return hip_fail(e, "matrix-core launch");
     }
