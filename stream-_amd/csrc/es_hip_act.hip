@@ -145,7 +145,7 @@ constexpr int RMS_WAVES = 16;   // waves per workgroup at most: 8192 elements at
 // (the row stays in registers). The sum of squares is the reference's in-order one, evaluated in parallel (es_hip_seqsum.h):
 // one thread adding a row's squares in order is a chain of dependent fp64 additions of about 10 ns each, which was the
 // whole kernel (2048 columns: 21.6 us for one row, 27.8 us for 512); now the chain has 8 additions per doubling of the sum
-// (7.0 and 10.1 us).
+// (back to back in a graph 5.1 and 6.9 us).
 template <int NCH>
 __global__ __launch_bounds__(RMS_WAVES * 64) void act_prep_rms(const float *__restrict__ x, uint64_t xs, const float *__restrict__ w,
                                                                float eps, int cols, float *xn, uint64_t xns, uint8_t *q80,
@@ -158,13 +158,19 @@ __global__ __launch_bounds__(RMS_WAVES * 64) void act_prep_rms(const float *__re
     __shared__ int s_ok;
     const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
     const float *xr = x + (size_t)r * xs;
-    float v[NCH][PER];
+    float v[NCH][PER], wt[NCH][PER];
 #pragma unroll
     for (int c = 0; c < NCH; c++) {
         const int e = (c * (int)blockDim.x + tid) * PER;
 #pragma unroll
-        for (int k = 0; k < PER; k++) v[c][k] = 0.0f;
-        if (e < cols) load_per(xr + e, v[c]);
+        for (int k = 0; k < PER; k++) {
+            v[c][k] = 0.0f;
+            wt[c][k] = 1.0f;
+        }
+        if (e < cols) {
+            load_per(xr + e, v[c]);
+            if (w) load_per(w + e, wt[c]);   // (beside the row's: its latency would otherwise follow the sum's)
+        }
     }
     double sum = 0.0;   // exact: the in-order sum of everything before this pass
     bool ok = true;
@@ -189,7 +195,12 @@ __global__ __launch_bounds__(RMS_WAVES * 64) void act_prep_rms(const float *__re
         const double before = __shfl_up(incl, 1);
         lds_sync();
         double base = sum;
-        for (int i = 0; i < wv; i++) base = base + wtot[i];
+        double pre[4];   // (the first ones read together)
+#pragma unroll
+        for (int i = 0; i < 4; i++) pre[i] = wtot[min(i, nw - 1)];
+#pragma unroll
+        for (int i = 0; i < 4; i++) base = i < wv ? base + pre[i] : base;
+        for (int i = 4; i < wv; i++) base = base + wtot[i];
         const double from = lane == 0 ? base : base + before, to = base + incl;
         const bool event = !seq_is_run(from, to);
         SeqRun run = event ? SeqRun{0.0, 0.0, 4u} : seq_run(q, seq_binade(from));
@@ -225,8 +236,10 @@ __global__ __launch_bounds__(RMS_WAVES * 64) void act_prep_rms(const float *__re
         if (wv == 0) {   // the exact sum through the runs and events in order, the same on every lane; 0x800: no run
             for (int i = 0; i < nw; i++) {
                 const int n = nev[i];
+                SumEvent next = ev[i * 64];   // (one record ahead: its reads overlap this one's additions)
                 for (int k = 0; k < n; k++) {
-                    const SumEvent E = ev[i * 64 + k];
+                    const SumEvent E = next;
+                    next = ev[i * 64 + min(k + 1, 63)];
                     if (E.binade != 0x800u) sum = seq_add_run(sum, SeqRun{E.a0, E.a1, E.e}, E.binade, ok);
 #pragma unroll
                     for (int m = 0; m < PER; m++) sum = sum + E.q[m];
@@ -258,10 +271,8 @@ __global__ __launch_bounds__(RMS_WAVES * 64) void act_prep_rms(const float *__re
         const int e = (c * (int)blockDim.x + tid) * PER;
         const bool have = e < cols;
         if (have) {
-            float wt[PER] = {1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f};
-            if (w) load_per(w + e, wt);
 #pragma unroll
-            for (int k = 0; k < PER; k++) v[c][k] = v[c][k] * s * wt[k];
+            for (int k = 0; k < PER; k++) v[c][k] = v[c][k] * s * wt[c][k];
             if (xn) store_per(xn + (size_t)r * xns + e, v[c]);
         }
         quant_per(v[c], have, have ? e : 0, o);

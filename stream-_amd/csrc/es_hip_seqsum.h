@@ -50,17 +50,23 @@ template <int N> ESQ_SEQSUM_QUAL SeqRun seq_run(const double (&q)[N], uint32_t b
     return SeqRun{t0 - s0, t1 - s1, p0 | (p1 ^ 1u) << 1};
 }
 
+// b if odd, else a, by masks (a choice between two fields of a struct can become an indexed load from the stack)
+ESQ_SEQSUM_QUAL double seq_pick(bool odd, double a, double b) {
+    const uint64_t m = odd ? ~0ull : 0ull;
+    return __builtin_bit_cast(double, (__builtin_bit_cast(uint64_t, b) & m) | (__builtin_bit_cast(uint64_t, a) & ~m));
+}
+
 // x, then y
 ESQ_SEQSUM_QUAL SeqRun seq_join(const SeqRun &x, const SeqRun &y) {
     const bool o0 = x.e & 1u, o1 = !(x.e & 2u);   // x ends odd from an even, from an odd start
     const uint32_t ye0 = y.e & 1u, ye1 = (y.e >> 1 & 1u) ^ 1u;
     const uint32_t e0 = o0 ? ye1 : ye0, e1 = o1 ? ye1 : ye0;
-    return SeqRun{x.a0 + (o0 ? y.a1 : y.a0), x.a1 + (o1 ? y.a1 : y.a0), e0 | (e1 ^ 1u) << 1};
+    return SeqRun{x.a0 + seq_pick(o0, y.a0, y.a1), x.a1 + seq_pick(o1, y.a0, y.a1), e0 | (e1 ^ 1u) << 1};
 }
 
 // the sum after a run from s; b: the binade the run was formed in. ok is cleared when s was or is not in it.
 ESQ_SEQSUM_QUAL double seq_add_run(double s, const SeqRun &r, uint32_t b, bool &ok) {
-    const double t = s + (__builtin_bit_cast(uint64_t, s) & 1u ? r.a1 : r.a0);
+    const double t = s + seq_pick(__builtin_bit_cast(uint64_t, s) & 1u, r.a0, r.a1);
     ok = ok && seq_binade(s) == b && seq_binade(t) == b;
     return t;
 }
