@@ -365,8 +365,13 @@ __device__ int3 block_excl_scan3(int3 v, int3 *wsum, int3 *tot) {
 
 __device__ int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-// One workgroup: moe_n's grouping (src/es_engine.c:871-888) of the ntok * k choices, then every job of the layer's two
-// launches. Experts take slots in order of first use; an expert's rows follow its choices in (token, j) order.
+// moe_n's grouping (src/es_engine.c:871-888) of the ntok * k choices, then every job of the layer's two launches. The
+// grouping is a chain of short LDS phases that one workgroup goes through; the job records behind it (over a hundred bytes
+// each, up to three per expert) took another 2.3 us on one CU. So 2 * GROUP_PARTS workgroups each do the grouping for
+// themselves and write one launch's table (blockIdx.y), every GROUP_PARTS-th run of 16 slots of it (blockIdx.x); the first
+// alone writes the pair rows. A layer of 128 experts, 8 picks, 32 tokens (2048 x 768, Q4_K and Q6_K): 111.3 -> 107.9 us;
+// 64 experts of Q2_K, 128 tokens: 73.9 -> 73.0. One part per launch 108.8, two 108.2, four 107.9, eight 107.6, 16 107.8.
+// Experts take slots in order of first use; an expert's rows follow its choices in (token, j) order.
 // The kernel's arguments as one block (its first and only parameter, at offset 0 of the argument segment).
 struct MoeBuildArgs {
     MoeDevArgs A;
@@ -374,6 +379,8 @@ struct MoeBuildArgs {
 };
 static_assert(sizeof(MoeBuildArgs) % 4 == 0 && sizeof(MoeBuildArgs) / 4 <= MOE_GROUP_THREADS, "one dword per thread");
 static_assert(MOE_MAX_PAIRS <= (1 << 20) && ROUTE_MAX_EXPERTS <= 1024, "slot order keys fit an int");
+
+constexpr int GROUP_PARTS = 4;
 
 __global__ __launch_bounds__(MOE_GROUP_THREADS) void moe_group_build(MoeBuildArgs P) {
     __shared__ __align__(16) int first[ROUTE_MAX_EXPERTS];
@@ -389,6 +396,7 @@ __global__ __launch_bounds__(MOE_GROUP_THREADS) void moe_group_build(MoeBuildArg
     const int lane = tid & 63, wv = tid >> 6;
     constexpr int NW = MOE_GROUP_THREADS / 64;
     const uint64_t lt = (1ull << lane) - 1;
+    const bool lead = blockIdx.x == 0 && blockIdx.y == 0;
     // the first chunk's choices and weights, loaded before anything waits on them
     const int sel0 = tid < R ? P.A.sel[tid] : -1;
     const float w0_ = tid < R ? P.A.w[tid] : 0.0f;
@@ -455,7 +463,7 @@ __global__ __launch_bounds__(MOE_GROUP_THREADS) void moe_group_build(MoeBuildArg
     // per thread: earlier chunks (taken), earlier waves of the chunk (wcnt), earlier lanes of the wave (a match mask
     // from ballots over the expert id's bits)
     for (int c0 = 0; c0 < R; c0 += T) {
-        for (int i = tid; i < NW * NE; i += T) wcnt[i / NE][i % NE] = 0;
+        for (int i = lane; i < NE; i += 64) wcnt[wv][i] = 0;   // a wave writes and clears its own row only
         const int p = c0 + tid;
         const int e0 = c0 == 0 ? sel0 : p < R ? A.sel[p] : -1;
         const int e = e0 >= 0 && e0 < NE ? e0 : -1;
@@ -464,7 +472,6 @@ __global__ __launch_bounds__(MOE_GROUP_THREADS) void moe_group_build(MoeBuildArg
             const uint64_t m = __ballot(e >= 0 && ((e >> b) & 1));
             same &= ((e >> b) & 1) ? m : ~m;
         }
-        lds_sync();
         if (e >= 0 && (same & lt) == 0) wcnt[wv][e] = __popcll(same);   // the wave's first lane with e
         lds_sync();
         if (p < R) {
@@ -475,10 +482,12 @@ __global__ __launch_bounds__(MOE_GROUP_THREADS) void moe_group_build(MoeBuildArg
                 for (int i = 0; i < wv; i++) r += wcnt[i][e];
                 row = ustart[slot[e]] + taken[e] + r;
                 wt = c0 == 0 ? w0_ : A.w[p];
-                A.tok_of[row] = p / A.k;
+                if (lead) A.tok_of[row] = p / A.k;
             }
-            A.rowof[p] = row;   // an invalid expert id contributes 0 * row 0
-            A.wv[p] = wt;
+            if (lead) {
+                A.rowof[p] = row;   // an invalid expert id contributes 0 * row 0
+                A.wv[p] = wt;
+            }
         }
         lds_sync();
         if (p < R && e >= 0 && (same & lt) == 0) atomicAdd(&taken[e], __popcll(same));
@@ -523,156 +532,155 @@ __global__ __launch_bounds__(MOE_GROUP_THREADS) void moe_group_build(MoeBuildArg
     const int c = real ? cnt[uexp] : 0, s0 = real ? ustart[u] : 0;
     const uint8_t *wg_u = pg[uexp], *wu_u = pu[uexp], *wd_u = pd[uexp];
     const int ff = A.ff, n = A.n;
-    for (int prod = 0; prod < 2; prod++) {   // 0: gate/up, 1: down
-        const MoeFamily &F = prod ? sa.DN : sa.GU;
-        const int njob = prod || (F.kind == MOE_FAM_MX && F.gated) ? 1 : 2;   // gated: gate and up in one job
-        int ntok = 0, tiles = 0, items = 0, units = 0;
-        if (F.kind == MOE_FAM_MX && real) {
-            ntok = ceil_div(c, MX_TOK);
-            tiles = njob * (ntok == 1 ? F.mx_tiles : F.row_tiles8 * ntok);
-        }
-        if (F.kind == MOE_FAM_MM && real) {
-            ntok = ceil_div(c, F.bn);
-            tiles = njob * F.row_tiles8 * ntok;
-            const int per = F.pj.nbk * (int)prep_words(F.pj.kind);
-            items = ceil_div(ntok * F.bn * per, PREP_SPAN) * PREP_SPAN;
-            // the expert's planes in 256-byte units: values [nbk][na_pad][256], then meta + scales [nbk][na_pad][36]
-            units = ceil_div(F.pj.nbk * ntok * F.bn * 256, 256) + ceil_div(F.pj.nbk * ntok * F.bn * 36, 256);
-        }
-        int tot_tiles = 0, tot_items = 0, w0 = 0;
-        if (F.kind != MOE_FAM_MV) {   // uniform across the block: every thread takes part in the scan
-            const int3 sc = block_excl_scan3(make_int3(tiles, items, units), wsum, &s_tot);
-            tot_tiles = s_tot.x;
-            tot_items = s_tot.y;
-            tiles = sc.x;
-            items = sc.y;
-            w0 = sc.z;
-        }
-        const int t0 = tiles, i0 = items;
-        const uint8_t *wsrc = prod ? wd_u : wg_u;
-        if (F.kind == MOE_FAM_MV) {
-            MvJob *jobs = static_cast<MvJob *>(prod ? A.dn_jobs : A.gu_jobs);
-            const int end = njob * U * F.mv_tiles;
-            if (tid < A.umax)
-                for (int g = 0; g < njob; g++) {
-                    MvJob J = F.mv;
-                    if (real) {
-                        J.W = g ? wu_u : wsrc;
-                        if (prod) {
-                            J.act = A.ha + (size_t)s0 * A.hstride;
-                            J.arow = nullptr;
-                            J.y = A.bye + (size_t)s0 * n;
-                        } else {
-                            J.act = A.x;
-                            J.arow = A.tok_of + s0;
-                            J.y = A.bgu + (size_t)s0 * 2 * ff + (size_t)g * ff;
-                        }
-                        J.na = c;
-                        J.nt = min(J.nt, c >= 3 ? 4 : c);   // the planner's width for c activations, within the LDS sizing
-                        J.tile0 = (njob * tid + g) * F.mv_tiles;
-                    } else {   // empty: the template's valid pointers, no rows, no activations, after the last real tile
-                        J.na = 0;
-                        J.r0 = J.r1 = 0;
-                        J.tile0 = end;
-                    }
-                    jobs[njob * tid + g] = J;
-                }
-            if (tid == 0) {   // the sentinel
+    const int prod = blockIdx.y;   // 0: gate/up, 1: down
+    const bool mine = (tid >> 4) % GROUP_PARTS == (int)blockIdx.x, last = blockIdx.x == GROUP_PARTS - 1;   // last: the sentinel's
+    const MoeFamily &F = prod ? sa.DN : sa.GU;
+    const int njob = prod || (F.kind == MOE_FAM_MX && F.gated) ? 1 : 2;   // gated: gate and up in one job
+    int ntok = 0, tiles = 0, items = 0, units = 0;
+    if (F.kind == MOE_FAM_MX && real) {
+        ntok = ceil_div(c, MX_TOK);
+        tiles = njob * (ntok == 1 ? F.mx_tiles : F.row_tiles8 * ntok);
+    }
+    if (F.kind == MOE_FAM_MM && real) {
+        ntok = ceil_div(c, F.bn);
+        tiles = njob * F.row_tiles8 * ntok;
+        const int per = F.pj.nbk * (int)prep_words(F.pj.kind);
+        items = ceil_div(ntok * F.bn * per, PREP_SPAN) * PREP_SPAN;
+        // the expert's planes in 256-byte units: values [nbk][na_pad][256], then meta + scales [nbk][na_pad][36]
+        units = ceil_div(F.pj.nbk * ntok * F.bn * 256, 256) + ceil_div(F.pj.nbk * ntok * F.bn * 36, 256);
+    }
+    int tot_tiles = 0, tot_items = 0, w0 = 0;
+    if (F.kind != MOE_FAM_MV) {   // uniform across the block: every thread takes part in the scan
+        const int3 sc = block_excl_scan3(make_int3(tiles, items, units), wsum, &s_tot);
+        tot_tiles = s_tot.x;
+        tot_items = s_tot.y;
+        tiles = sc.x;
+        items = sc.y;
+        w0 = sc.z;
+    }
+    const int t0 = tiles, i0 = items;
+    const uint8_t *wsrc = prod ? wd_u : wg_u;
+    if (F.kind == MOE_FAM_MV) {
+        MvJob *jobs = static_cast<MvJob *>(prod ? A.dn_jobs : A.gu_jobs);
+        const int end = njob * U * F.mv_tiles;
+        if (tid < A.umax && mine)
+            for (int g = 0; g < njob; g++) {
                 MvJob J = F.mv;
-                J.na = 0;
-                J.r0 = J.r1 = 0;
-                J.tile0 = end;
-                jobs[njob * A.umax] = J;
-            }
-        } else if (F.kind == MOE_FAM_MX) {
-            MkJob *jobs = static_cast<MkJob *>(prod ? A.dn_jobs : A.gu_jobs);
-            if (tid < A.umax)
-                for (int g = 0; g < njob; g++) {
-                    MkJob J = F.mk;
-                    if (real) {
-                        J.W = g ? wu_u : wsrc;
-                        J.act = prod ? A.ha + (size_t)s0 * A.hstride : A.x;
-                        J.arow = prod ? nullptr : A.tok_of + s0;
-                        J.y = prod ? A.bye + (size_t)s0 * n : A.bgu + (size_t)s0 * 2 * ff + (size_t)g * ff;
-                        if (!prod && F.gated) {   // h's Q8_K blocks of the expert's first pair row
-                            J.W2 = wu_u;
-                            J.y = reinterpret_cast<float *>(A.ha + (size_t)s0 * A.hstride);
-                        }
-                        J.na = c;
-                        J.ntok_tiles = ntok;
-                        J.tile0 = t0 + g * (ntok == 1 ? F.mx_tiles : F.row_tiles8 * ntok);
-                    } else {
-                        J.na = 0;
-                        J.r0 = J.r1 = 0;
-                        J.ntok_tiles = 1;
-                        J.tile0 = tot_tiles;
-                    }
-                    jobs[njob * tid + g] = J;
-                }
-            if (tid == 0) {
-                MkJob J = F.mk;
-                J.na = 0;
-                J.r0 = J.r1 = 0;
-                J.ntok_tiles = 1;
-                J.tile0 = tot_tiles;
-                jobs[njob * A.umax] = J;
-            }
-        } else {
-            MmJob *jobs = static_cast<MmJob *>(prod ? A.dn_jobs : A.gu_jobs);
-            PrepJob *pj = prod ? A.dn_prep : A.gu_prep;
-            uint8_t *ws = prod ? A.dn_ws : A.gu_ws;
-            if (tid < A.umax) {
-                const int na_pad = ntok * F.bn;
-                uint8_t *xq = ws + (size_t)w0 * 256;
-                uint8_t *xm = xq + ((size_t)F.pj.nbk * na_pad * 256 + 255) / 256 * 256;
-                PrepJob P = F.pj;
                 if (real) {
-                    P.act = prod ? A.ha + (size_t)s0 * A.hstride : A.x;
-                    P.arow = prod ? nullptr : A.tok_of + s0;
-                    P.xq = xq;
-                    P.xm = xm;
-                    P.start = i0;
-                    P.na = c;
-                    P.na_pad = na_pad;
-                } else {
-                    P.na = P.na_pad = 0;
-                    P.start = tot_items;
-                }
-                pj[tid] = P;
-                for (int g = 0; g < njob; g++) {
-                    MmJob J = F.mm;
-                    if (real) {
-                        J.W = g ? wu_u : wsrc;
-                        J.xq = xq;
-                        J.xm = xm;
-                        J.y = prod ? A.bye + (size_t)s0 * n : A.bgu + (size_t)s0 * 2 * ff + (size_t)g * ff;
-                        J.na = c;
-                        J.na_pad = na_pad;
-                        J.ntok_tiles = ntok;
-                        J.tile0 = t0 + g * F.row_tiles8 * ntok;
+                    J.W = g ? wu_u : wsrc;
+                    if (prod) {
+                        J.act = A.ha + (size_t)s0 * A.hstride;
+                        J.arow = nullptr;
+                        J.y = A.bye + (size_t)s0 * n;
                     } else {
-                        J.na = 0;
-                        J.r0 = J.r1 = 0;
-                        J.ntok_tiles = 1;
-                        J.tile0 = tot_tiles;
+                        J.act = A.x;
+                        J.arow = A.tok_of + s0;
+                        J.y = A.bgu + (size_t)s0 * 2 * ff + (size_t)g * ff;
                     }
-                    jobs[njob * tid + g] = J;
+                    J.na = c;
+                    J.nt = min(J.nt, c >= 3 ? 4 : c);   // the planner's width for c activations, within the LDS sizing
+                    J.tile0 = (njob * tid + g) * F.mv_tiles;
+                } else {   // empty: the template's valid pointers, no rows, no activations, after the last real tile
+                    J.na = 0;
+                    J.r0 = J.r1 = 0;
+                    J.tile0 = end;
                 }
+                jobs[njob * tid + g] = J;
             }
-            if (tid == 0) {
-                PrepJob P = F.pj;
+        if (tid == 0 && last) {   // the sentinel
+            MvJob J = F.mv;
+            J.na = 0;
+            J.r0 = J.r1 = 0;
+            J.tile0 = end;
+            jobs[njob * A.umax] = J;
+        }
+    } else if (F.kind == MOE_FAM_MX) {
+        MkJob *jobs = static_cast<MkJob *>(prod ? A.dn_jobs : A.gu_jobs);
+        if (tid < A.umax && mine)
+            for (int g = 0; g < njob; g++) {
+                MkJob J = F.mk;
+                if (real) {
+                    J.W = g ? wu_u : wsrc;
+                    J.act = prod ? A.ha + (size_t)s0 * A.hstride : A.x;
+                    J.arow = prod ? nullptr : A.tok_of + s0;
+                    J.y = prod ? A.bye + (size_t)s0 * n : A.bgu + (size_t)s0 * 2 * ff + (size_t)g * ff;
+                    if (!prod && F.gated) {   // h's Q8_K blocks of the expert's first pair row
+                        J.W2 = wu_u;
+                        J.y = reinterpret_cast<float *>(A.ha + (size_t)s0 * A.hstride);
+                    }
+                    J.na = c;
+                    J.ntok_tiles = ntok;
+                    J.tile0 = t0 + g * (ntok == 1 ? F.mx_tiles : F.row_tiles8 * ntok);
+                } else {
+                    J.na = 0;
+                    J.r0 = J.r1 = 0;
+                    J.ntok_tiles = 1;
+                    J.tile0 = tot_tiles;
+                }
+                jobs[njob * tid + g] = J;
+            }
+        if (tid == 0 && last) {
+            MkJob J = F.mk;
+            J.na = 0;
+            J.r0 = J.r1 = 0;
+            J.ntok_tiles = 1;
+            J.tile0 = tot_tiles;
+            jobs[njob * A.umax] = J;
+        }
+    } else {
+        MmJob *jobs = static_cast<MmJob *>(prod ? A.dn_jobs : A.gu_jobs);
+        PrepJob *pj = prod ? A.dn_prep : A.gu_prep;
+        uint8_t *ws = prod ? A.dn_ws : A.gu_ws;
+        if (tid < A.umax && mine) {
+            const int na_pad = ntok * F.bn;
+            uint8_t *xq = ws + (size_t)w0 * 256;
+            uint8_t *xm = xq + ((size_t)F.pj.nbk * na_pad * 256 + 255) / 256 * 256;
+            PrepJob P = F.pj;
+            if (real) {
+                P.act = prod ? A.ha + (size_t)s0 * A.hstride : A.x;
+                P.arow = prod ? nullptr : A.tok_of + s0;
+                P.xq = xq;
+                P.xm = xm;
+                P.start = i0;
+                P.na = c;
+                P.na_pad = na_pad;
+            } else {
                 P.na = P.na_pad = 0;
                 P.start = tot_items;
-                pj[A.umax] = P;
+            }
+            pj[tid] = P;
+            for (int g = 0; g < njob; g++) {
                 MmJob J = F.mm;
-                J.na = 0;
-                J.r0 = J.r1 = 0;
-                J.ntok_tiles = 1;
-                J.tile0 = tot_tiles;
-                jobs[njob * A.umax] = J;
+                if (real) {
+                    J.W = g ? wu_u : wsrc;
+                    J.xq = xq;
+                    J.xm = xm;
+                    J.y = prod ? A.bye + (size_t)s0 * n : A.bgu + (size_t)s0 * 2 * ff + (size_t)g * ff;
+                    J.na = c;
+                    J.na_pad = na_pad;
+                    J.ntok_tiles = ntok;
+                    J.tile0 = t0 + g * F.row_tiles8 * ntok;
+                } else {
+                    J.na = 0;
+                    J.r0 = J.r1 = 0;
+                    J.ntok_tiles = 1;
+                    J.tile0 = tot_tiles;
+                }
+                jobs[njob * tid + g] = J;
             }
         }
-        lds_sync();
+        if (tid == 0 && last) {
+            PrepJob P = F.pj;
+            P.na = P.na_pad = 0;
+            P.start = tot_items;
+            pj[A.umax] = P;
+            MmJob J = F.mm;
+            J.na = 0;
+            J.r0 = J.r1 = 0;
+            J.ntok_tiles = 1;
+            J.tile0 = tot_tiles;
+            jobs[njob * A.umax] = J;
+        }
     }
 }
 
@@ -680,7 +688,7 @@ __global__ __launch_bounds__(MOE_GROUP_THREADS) void moe_group_build(MoeBuildArg
 
 hipError_t moe_group_build_launch(const MoeDevArgs &a, const MoeFamily &gu, const MoeFamily &dn, hipStream_t s) {
     const MoeBuildArgs P{a, gu, dn};
-    hipLaunchKernelGGL(moe_group_build, dim3(1), dim3(MOE_GROUP_THREADS), 0, s, P);
+    hipLaunchKernelGGL(moe_group_build, dim3(GROUP_PARTS, 2), dim3(MOE_GROUP_THREADS), 0, s, P);
     return hipGetLastError();
 }
 
