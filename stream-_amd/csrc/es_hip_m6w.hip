@@ -90,9 +90,8 @@ __global__ __launch_bounds__(512) void m6w_kernel(const MkJob *__restrict__ jobs
     uint32_t aoff[WN];   // the lane's activation rows (past the last repeat it; not stored)
 #pragma unroll
     for (int c = 0; c < WN; c++) aoff[c] = (uint32_t)min(tok0 + 16 * c + lr, J.na - 1) * (uint32_t)J.astride;
-    // item it: row group g0 + it / nround, superblock (it % nround) * nw + wave. Every load is unconditional (items past the last
-    // repeat it, superblocks past the row's end its last one, whose terms no chain reads): a load behind a branch makes the
-    // compiler's waits drain the queue.
+    // item it: row group g0 + it / nround, superblock (it % nround) * nw + wave. A wave past the row's end in the last round
+    // keeps its former weights and takes the row's last activation block: no chain reads its terms.
     Raw6 raw;
     B6 B[WN];
     auto load_w = [&](int it) {

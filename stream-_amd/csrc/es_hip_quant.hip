@@ -2791,6 +2791,11 @@ int moe_ctx_check(const es_hip_moe_ctx *c, int N, const void *x, const float *ou
     if (N > 1 && ostride && ostride < (size_t)c->n) return fail(ES_HIP_EINVAL, "ostride %zu < n %d", ostride, c->n);
     return ES_HIP_OK;
 }
+bool overlap(const void *a, size_t na, const void *b, size_t nb) {   // (null: nowhere)
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return p && q && p < q + nb && q < p + na;
+}
+
 // the token rows x as check_req checks a product's activations: dword-aligned rows at least one row's blocks apart
 int moe_ctx_check_x(const es_hip_moe_ctx *c, int N, const void *x, size_t xstride) {
     if (N == 0) return ES_HIP_OK;
@@ -2816,13 +2821,16 @@ int es_hip_moe_ctx_run_logits(es_hip_moe_ctx *c, int N, const float *logits, siz
     if (N == 0) return ES_HIP_OK;
     if (!logits) return fail(ES_HIP_EINVAL, "null logits");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // (outputs at an odd alignment, which the kernel cannot store to, are copied)
-    int *sel2 = reinterpret_cast<uintptr_t>(sel_out) & 3 ? nullptr : sel_out;
-    float *w2 = reinterpret_cast<uintptr_t>(w_out) & 3 ? nullptr : w_out;
-    hipError_t e = esq::route_softmax_launch(logits, lstride ? lstride : (uint64_t)c->n_exp, N, c->n_exp, c->k, norm_topk,
-                                             c->sel, c->w, c->k, sel2, w2, s);
+    // Outputs at an odd alignment, which the kernel cannot store to, are copied, and so are all where one lies over another
+    // or over the logits: other tokens' waves may still be reading those.
+    const size_t pairs = (size_t)N * c->k, ls = lstride ? lstride : (size_t)c->n_exp;
+    const size_t lbytes = ((size_t)(N - 1) * ls + c->n_exp) * sizeof(float);
+    const bool apart = !overlap(sel_out, pairs * sizeof(int), logits, lbytes) && !overlap(w_out, pairs * sizeof(float), logits, lbytes) &&
+                       !overlap(sel_out, pairs * sizeof(int), w_out, pairs * sizeof(float));
+    int *sel2 = reinterpret_cast<uintptr_t>(sel_out) & 3 || !apart ? nullptr : sel_out;
+    float *w2 = reinterpret_cast<uintptr_t>(w_out) & 3 || !apart ? nullptr : w_out;
+    hipError_t e = esq::route_softmax_launch(logits, ls, N, c->n_exp, c->k, norm_topk, c->sel, c->w, c->k, sel2, w2, s);
     if (e != hipSuccess) return hip_fail(e, "routing launch");
-    const size_t pairs = (size_t)N * c->k;
     if (sel_out != sel2 && (e = hipMemcpyAsync(sel_out, c->sel, pairs * sizeof(int), hipMemcpyDeviceToDevice, s)) != hipSuccess)
         return hip_fail(e, "routing copy");
     if (w_out != w2 && (e = hipMemcpyAsync(w_out, c->w, pairs * sizeof(float), hipMemcpyDeviceToDevice, s)) != hipSuccess)
@@ -2840,12 +2848,14 @@ int es_hip_moe_ctx_run(es_hip_moe_ctx *c, int N, const int *sel, const float *w,
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t pairs = (size_t)N * c->k;
     hipError_t e;
-    // the layer's kernels read the caller's routing in stream order; only at an odd alignment, which they cannot, a copy of it
-    if (reinterpret_cast<uintptr_t>(sel) & 3) {
+    // The layer's kernels read the caller's routing in stream order: a copy of it only at an odd alignment, which they cannot
+    // read, and under the outputs, which the pair form writes while other workgroups still read the routing.
+    const size_t obytes = ((size_t)(N - 1) * (ostride ? ostride : (size_t)c->n) + c->n) * sizeof(float);
+    if (reinterpret_cast<uintptr_t>(sel) & 3 || overlap(sel, pairs * sizeof(int), out, obytes)) {
         if ((e = hipMemcpyAsync(c->sel, sel, pairs * sizeof(int), hipMemcpyDeviceToDevice, s)) != hipSuccess) return hip_fail(e, "routing copy");
         sel = c->sel;
     }
-    if (reinterpret_cast<uintptr_t>(w) & 3) {
+    if (reinterpret_cast<uintptr_t>(w) & 3 || overlap(w, pairs * sizeof(float), out, obytes)) {
         if ((e = hipMemcpyAsync(c->w, w, pairs * sizeof(float), hipMemcpyDeviceToDevice, s)) != hipSuccess) return hip_fail(e, "routing copy");
         w = c->w;
     }

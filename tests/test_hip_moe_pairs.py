@@ -61,3 +61,26 @@ def test_pairs_repeats_and_no_expert(hipo, orc):
     sel[0] = 7                      # one expert four times
     sel[1, 2], sel[3, 0] = -1, 12   # no expert
     layer(hipo, orc, (O.Q4_K, O.Q4_K, O.Q4_K), 256, 256, 12, sel, w, 41)
+
+
+def test_routing_under_the_outputs(hipo, orc):
+    """the routing read from where the outputs go, and the routing outputs of run_logits over its own logits"""
+    types, n, ff, n_exp, N, k = (O.Q4_K, O.Q4_K, O.Q6_K), 512, 256, 24, 8, 4
+    ex = Experts(hipo, orc, types, n_exp, n, ff, 51)
+    x = orc.quantize_act(types[0], orc.gauss(52, 1.0, N * n).reshape(N, n))
+    logits = orc.gauss(53, 1.0, N * n_exp).reshape(N, n_exp)
+    sel, w, _ = orc.route_softmax(logits, k, True)
+    ref = orc.moe_ffn(types, ex.host, n, ff, x, sel, w, order=MODES[0][1], path=MODES[0][2])
+    ctx = hipo.moe_ctx(ex.args(np.zeros(1, np.int32), np.zeros((1, k), np.int32), np.zeros((1, k), np.float32)), N, k)
+    buf = np.zeros((N, n), np.float32)
+    buf[0, :N * k] = np.ascontiguousarray(sel, np.int32).view(np.float32).ravel()
+    buf[1, 1:1 + N * k] = w.ravel()
+    dx, dout = hipo.upload(x), hipo.upload(buf)
+    ctx.run(N, dout, int(dout) + 4 * (n + 1), dx, x.strides[0], dout, n)
+    assert np.array_equal(bits(hipo.download(dout, np.zeros((N, n), np.float32))), bits(ref))
+    dl, dout = hipo.upload(logits), hipo.upload(np.zeros((N, n), np.float32))
+    ctx.run_logits(N, dl, 0, True, dx, x.strides[0], dout, n, int(dl) + 4 * N * k, dl)
+    assert np.array_equal(bits(hipo.download(dout, np.zeros((N, n), np.float32))), bits(ref))
+    assert np.array_equal(bits(hipo.download(dl, np.zeros((N, k), np.float32))), bits(w))
+    assert np.array_equal(hipo.download(dl, np.zeros((N, k), np.int32), offset=4 * N * k), sel)
+    ctx.close()
