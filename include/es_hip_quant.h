@@ -286,7 +286,7 @@ int es_hip_set_batched32_min(int n);
  * eight AVX2 lane sums of 4 rows x 32 activations; default 2); the others on the one-lane-per-output kernel. */
 int es_hip_set_batched32_mfma_min(int n);
 /* Q6_K products with at least n activations run on a Q6_K matrix-core kernel (default 16, which also stands for the
- * automatic choice: from 5 activations on the kernel with one wave per superblock). */
+ * automatic choice: from 5 activations on the kernel with one wave per superblock, where it is the faster one). */
 int es_hip_set_q6k_mfma_min_batch(int n);
 /* Q2_K products with at least n activations run on the Q2_K LDS-staged matrix-core kernel (default 2); below that, or
  * with it off, the small-batch kernel (es_hip_set_small_batch_min) or the vector kernel. */

@@ -696,39 +696,80 @@ int m6w_waves(int nbk) {
     return (nbk + rounds - 1) / rounds;
 }
 // Activations per workgroup, in tiles of 16: up to 64 (a superblock is unpacked once per workgroup), 32 where a wave takes
-// several superblocks (their activation operands are loaded ahead, which at 64 does not fit the registers), fewer while a
-// product has less than a workgroup per CU.
-int m6w_tiles(int rows, int na, int nbk, int cus) {
+// several superblocks (their activation operands are loaded ahead, which at 64 does not fit the registers), fewer while the
+// launch's row groups (16 rows) come to less than a workgroup per CU.
+int m6w_tiles(long groups, int na, int nbk, int cus) {
     int wn = nbk > esq::M6W_WAVES ? 2 : 4;
     while (wn > 1 && 8 * wn >= na) wn /= 2;
-    while (wn > 1 && (long)((rows + 15) / 16) * ((na + 16 * wn - 1) / (16 * wn)) < cus) wn /= 2;
+    while (wn > 1 && groups * ((na + 16 * wn - 1) / (16 * wn)) < cus) wn /= 2;
     return wn;
 }
-// Which Q6_K batches take that kernel (no gather, 32-bit offsets): of the default g_mm6_min = 16 (the automatic choice) those
-// of 5 activations or more, else those of g_mm6_min, where it is the faster of the matrix-core kernels. The tiled kernel
-// (es_hip_mm6.hip) runs a tile's superblocks one after another, 2.4 us each, a set of 256 tiles of 128 rows x 64 activations
-// at a time (2 us more each), behind a pre-pass (6 us); this one takes about 1.4 ns per superblock of 16 rows x 16 wn
-// activations, 2.3 with several superblocks per wave, and 5 us. Measured (us, this kernel / tiled): 2048 x 8192 at 64, 128 and
-// 512 activations 24 / 79, 41 / 78, 141 / 79; 8192 x 2048 13 / 26, 18 / 26, 50 / 48; 4096 x 4096 21 / 44, 37 / 43, 129 / 47;
-// against the decode kernel's passes of 4 at 8 activations 8192 x 2048 9.3 / 14.1, 151936 x 1024 57 / 66 (2048 x 8192 16.6 /
-// 15.2), and slower at 4 (8.9 / 8.6). A product of one activation tile and many row tiles whose activations fit the LDS
-// keeps the tiled kernel's persistent form (151936 x 1024 at 16 and 64: 57 / 43, 61 / 58).
 std::atomic<int> g_m6w_on{1};
-bool m6w_eligible(const Req &q) {
+// What that kernel can take: no gather, 32-bit offsets; of the default g_mm6_min = 16 (the automatic choice) products of 5
+// activations or more, else those of g_mm6_min.
+bool m6w_capable(const Req &q) {
     const int set = g_mm6_min.load(), mn = set == 16 ? 5 : set;
-    if (!g_m6w_on.load() || q.type != ES_HIP_Q6_K || mn <= 0 || q.na < mn || q.na > 2048 || q.arow || q.ints || q.r1 <= q.r0) return false;
-    const int nbk = q.cols / 256, rows = q.r1 - q.r0, cus = device().cus;
+    if (!g_m6w_on.load() || q.type != ES_HIP_Q6_K || mn <= 0 || q.na < mn || q.na > 2048 || q.arow || q.ints || q.row_bytes || q.r1 <= q.r0)
+        return false;
+    const int nbk = q.cols / 256;
     const size_t stride = q.astride ? q.astride : (size_t)nbk * 292;
-    if ((size_t)q.na * stride >= ((size_t)1 << 32) - 65536 || (size_t)q.r1 * nbk * 210 >= ((size_t)1 << 32)) return false;
-    if (q.na < 16) return true;
-    const int rt = (rows + 127) / 128, bn = q.na <= 16 ? 16 : q.na <= 32 ? 32 : 64;
-    if (q.na <= 64 && rt >= 2 * cus && nbk <= esq::mm6_persistent_blocks(bn)) return false;
-    const int wn = m6w_tiles(rows, q.na, nbk, cus);
-    const double units = (double)((rows + 15) / 16) * ((q.na + 16 * wn - 1) / (16 * wn)) * nbk;
-    const long sets = ((long)rt * ((q.na + 63) / 64) + cus - 1) / cus;
-    return 5.0 + units * (nbk > esq::M6W_WAVES ? 2.3e-3 : 1.4e-3) < 6.0 + (2.0 + 2.4 * nbk) * sets;
+    return (size_t)q.na * stride < ((size_t)1 << 32) - 65536 && (size_t)q.r1 * nbk * 210 < ((size_t)1 << 32);
 }
-// Row groups per workgroup and the tile numbering: about one resident set of workgroups (16 waves per CU) for the launch.
+// Which of a batch's Q6_K products take it: those of 16 activations or more, and those of fewer, each where the launch of all
+// of them is the faster one. The tiled kernel (es_hip_mm6.hip) runs a tile's superblocks one after another, 2.4 us each, a set
+// of 256 tiles of 128 rows x 64 activations at a time (2 us more each), behind a pre-pass (6 us); this one takes about 1.4 ns
+// per superblock of 16 rows x 16 wn activations, 2.3 with several superblocks per wave, and 5 us. Measured (us, this kernel /
+// tiled): 2048 x 8192 at 64, 128 and 512 activations 24 / 79, 41 / 78, 141 / 79; 8192 x 2048 13 / 26, 18 / 26, 50 / 48; 4096 x
+// 4096 21 / 44, 37 / 43, 129 / 47. Against the decode kernel's passes of 4 at 8 activations 8192 x 2048 9.3 / 14.1, 151936 x 1024
+// 57 / 66 (2048 x 8192 16.6 / 15.2), and slower at 4 (8.9 / 8.6). Batches of these (us, this kernel / decode kernel): 112 x
+// 2048 x 768 at 5, 8 and 12 69 / 63, 69 / 74, 69 / 108, 32 of them at 6 22.5 / 29; 16 x 8192 x 2048 86 / 76, 86 / 87, 87 / 128, two 13.4 /
+// 17.8, 13.7 / 20.8; 16 x 2048 x 8192 104 / 77, 106 / 88, 109 / 129, two 15.8 / 17.7. So a batch that fills the device anyway takes it
+// from a mean of 7 activations, 9 with rows longer than its waves, a small one always; where products of fewer activations
+// need a decode launch beside it, it must have half of the weights (8192 x 2048 at 8 and at 1 14.0 / 19.6; an expert layer with
+// a few experts at 5 and 6 123 / 115) and rows not too long (2048 x 8192 at 8 with 512 x 2048 at 2 21.6 / 19.9). 64 x 2048 x 768 at
+// 20 and 40 against the tiled kernel 36.6 / 43.5, 44.8 / 54.8. A product of one activation tile and many row tiles whose
+// activations fit the LDS keeps the tiled kernel's persistent form (151936 x 1024 at 16 and 64: 57 / 43, 61 / 58).
+struct M6wChoice { bool few = false, many = false; long gfew = 0, gmany = 0; };   // groups: rows / 16 of either kind
+M6wChoice m6w_choose(const std::vector<Req> &reqs, int cus) {
+    M6wChoice c;
+    long sfew = 0, afew = 0, rest = 0, tiles = 0;   // superblocks below 16 (and times activations), those left to the decode kernel
+    int nbk_max = 0;
+    bool longr = false;
+    for (const Req &q : reqs) {
+        if (q.type != ES_HIP_Q6_K || q.r1 <= q.r0 || q.na <= 0) continue;
+        const long g = (q.r1 - q.r0 + 15) / 16, blocks = (long)(q.r1 - q.r0) * (q.cols / 256);
+        if (!m6w_capable(q)) {
+            if (q.na < 16) rest += blocks;
+        } else if (q.na < 16) {
+            sfew += blocks;
+            afew += blocks * q.na;
+            longr = longr || q.cols / 256 > esq::M6W_WAVES;
+            c.gfew += g;
+        } else {
+            c.gmany += g;
+            tiles += (long)((q.r1 - q.r0 + 127) / 128) * ((q.na + 63) / 64);
+            nbk_max = std::max(nbk_max, q.cols / 256);
+        }
+    }
+    double cost = 5.0;
+    for (const Req &q : reqs)
+        if (q.na >= 16 && m6w_capable(q)) {
+            const int nbk = q.cols / 256, wn = m6w_tiles(c.gmany, q.na, nbk, cus);
+            cost += (double)((q.r1 - q.r0 + 15) / 16) * ((q.na + 16 * wn - 1) / (16 * wn)) * nbk * (nbk > esq::M6W_WAVES ? 2.3e-3 : 1.4e-3);
+        }
+    c.many = cost < 6.0 + (2.0 + 2.4 * nbk_max) * ((tiles + cus - 1) / cus);
+    c.few = sfew > 0 && sfew >= rest && (afew >= (longr ? 9 : 7) * sfew || (sfew <= (longr ? 131072 : 262144) && !(rest && longr)));
+    return c;
+}
+bool m6w_eligible(const Req &q, const M6wChoice &c) {
+    if (!m6w_capable(q)) return false;
+    if (q.na < 16) return c.few;
+    const int nbk = q.cols / 256, rt = (q.r1 - q.r0 + 127) / 128, bn = q.na <= 16 ? 16 : q.na <= 32 ? 32 : 64;
+    return c.many && !(q.na <= 64 && rt >= 2 * device().cus && nbk <= esq::mm6_persistent_blocks(bn));
+}
+// Row groups per workgroup and the tile numbering: about one resident set of workgroups (16 waves per CU) for the launch, a
+// product's chunks a multiple of 8 (workgroup g runs on XCD g % 8: 112
+// products of 2048 rows in 5 chunks each left three XCDs idle, 115 us; in 8 chunks 69).
 void m6w_tiling(MkGroup &g, int cus) {
     long units = 0;
     for (const esq::MkJob &j : g.jobs) units += (long)((j.r1 - j.r0 + 15) / 16) * j.ntok_tiles;
@@ -736,10 +777,10 @@ void m6w_tiling(MkGroup &g, int cus) {
     const int per = (int)std::max<long>(1, (units + slots - 1) / slots);
     g.grid = 0;
     for (esq::MkJob &j : g.jobs) {
-        j.rows_per_wg = per;
+        const int ngroup = (j.r1 - j.r0 + 15) / 16, sets = ((ngroup + per - 1) / per + 7) / 8;
+        j.rows_per_wg = (ngroup + 8 * sets - 1) / (8 * sets);
         j.tile0 = g.grid;
-        const int chunks = ((j.r1 - j.r0 + 15) / 16 + per - 1) / per;
-        g.grid += 8 * ((chunks + 7) / 8) * j.ntok_tiles;
+        g.grid += 8 * sets * j.ntok_tiles;
     }
 }
 
@@ -793,6 +834,7 @@ void mbx_tiles(MkGroup &g, int cus) {
 
 int plan_batch(const std::vector<Req> &reqs, Batch &bt, bool allow_pk = true) {
     bt = Batch();
+    const M6wChoice m6w = m6w_choose(reqs, device().cus);
     std::vector<Req> mv;
     for (const Req &q : reqs) {
         FmtInfo f;
@@ -946,8 +988,8 @@ int plan_batch(const std::vector<Req> &reqs, Batch &bt, bool allow_pk = true) {
             g->jobs.push_back(j);
             continue;
         }
-        if (m6w_eligible(q)) {
-            const int wn = m6w_tiles(q.r1 - q.r0, q.na, nbk, device().cus), nw = m6w_waves(nbk);
+        if (m6w_eligible(q, m6w)) {
+            const int wn = m6w_tiles(q.na < 16 ? m6w.gfew : m6w.gmany, q.na, nbk, device().cus), nw = m6w_waves(nbk);
             MkGroup *g = nullptr;
             for (MkGroup &x : bt.mkg)
                 if (x.m6_wn == wn && x.m6_nw == nw && x.m6_keep == (nbk <= nw)) g = &x;

@@ -72,3 +72,30 @@ def test_several_products_in_a_launch(hip, orc):
     hip.run_jobs(specs)
     for dY, w in zip(outs, want):
         assert np.array_equal(bits(hip.download(dY, np.zeros_like(w))), bits(w))
+
+
+@pytest.mark.parametrize("shapes", [
+    [(2048, 1, 5 + j % 11) for j in range(40)],                       # several row groups per workgroup, chunks rounded to 8
+    [(1000 + 16 * j, 3, 20 + j) for j in range(20)],                  # ... at two tiles of activations
+    [(160, 4, 8), (96, 4, 15), (16, 4, 1), (7, 9, 3)],                # a decode launch beside it
+    [(16, 4, 5), (300, 4, 2), (250, 2, 4)],                           # few products of 5: all in the decode launch
+    [(64, 9, 6), (64, 9, 1)], [(64, 9, 9), (64, 9, 1)],               # rows longer than its waves
+    [(40, 2, 9), (40, 2, 33), (40, 2, 2)],                            # every kind
+], ids=["chunks", "tiles", "beside", "left", "long6", "long9", "mixed"])
+def test_batches(hip, orc, shapes):
+    specs, want, outs, keep = [], [], [], []
+    for j, (rows, nbk, na) in enumerate(shapes):
+        st = np.array([900 + j], np.uint64)
+        W = orc.mtest_blocks(O.Q6_K, st, rows, 256 * nbk)
+        acts = orc.quantize_act(O.Q6_K, orc.mtest_acts(st, na * 256 * nbk).reshape(na, 256 * nbk))
+        want.append(orc.matvec_multi(O.Q6_K, W, 256 * nbk, rows, acts))
+        dW, dA, dY = hip.upload(W), hip.upload(acts), hip.upload(np.full((na, rows), -7.0, np.float32))
+        keep += [dW, dA]
+        outs.append(dY)
+        specs.append(dict(type=O.Q6_K, rows=rows, cols=256 * nbk, W=dW, act=dA, astride=acts.strides[0], nb=na, y=dY, ystride=rows))
+    plan = hip.plan(specs)
+    plan.run()
+    hip.synchronize()
+    plan.close()
+    for dY, w in zip(outs, want):
+        assert np.array_equal(bits(hip.download(dY, np.zeros_like(w))), bits(w))
