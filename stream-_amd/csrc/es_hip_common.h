@@ -149,7 +149,8 @@ hipError_t mbx_launch(int type, bool gather, int nbk_max, const MkJob *jobs, int
                       int order, hipStream_t s);
 // Q6_K batches with one wave per superblock (es_hip_m6w.hip): the same jobs without a gather, workgroups of nw <= M6W_WAVES
 // waves over rows_per_wg groups of 16 rows x 16 wn activations (wn 1, 2 or 4; all activation tiles of a row chunk on one XCD:
-// 8 * ceil(chunks / 8) * ntok_tiles ids per job, tile0 a multiple of 8). keep: every job has at most nw superblocks per row.
+// 8 * ceil(chunks / 8) * ntok_tiles ids per job, tile0 a multiple of 8). keep: every job has at most nw superblocks per row;
+// without it nw >= wn.
 constexpr int M6W_WAVES = 8;
 hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob &single, int grid, int order, hipStream_t s);
 // gather: some job of the launch reads its activation rows through arow (a separate kernel build; the others need not);

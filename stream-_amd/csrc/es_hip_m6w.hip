@@ -6,7 +6,8 @@
 // A workgroup of up to 8 waves takes 16 rows x 16 WN activations at a time; wave w the superblocks w, w + waves, ... of
 // these rows. Only the last line above is sequential: every wave forms its superblock's integers for the whole tile and
 // leaves them in LDS as floats, and after one barrier each (4 rows, activation) has a thread that runs the reference's chain
-// over the superblocks at hand. A product of few rows and many superblocks (a 2048 x 8192 down projection: 16 workgroups of
+// over the superblocks at hand (rows of 1 to 3 superblocks have fewer threads than chains at 32 or 64 activations and run them
+// in turns: 8192 x 768 at 64 activations 8.6 us against 9.6 with narrower tiles, which unpack every superblock twice). A product of few rows and many superblocks (a 2048 x 8192 down projection: 16 workgroups of
 // 128 rows running 32 superblocks one after another, 94.9 us at 64 activations) so has its superblocks in flight on
 // different waves; with at most as many superblocks as waves a wave keeps its activation operands in registers over all
 // row groups of its workgroup, and no operand passes through LDS. Measured (tiled kernel before -> this one): 2048 x 8192 at
@@ -106,9 +107,7 @@ __global__ __launch_bounds__(512) void m6w_kernel(const MkJob *__restrict__ jobs
     load_w(0);
     load_x(0);
 
-    const bool chain = tid < WN * 64;   // this thread's chain: activation tid / 4 of the tile, rows 4 (tid % 4) .. + 3
-    const int cq = tid >> 2, cr = 4 * (tid & 3), q = tok0 + cq;
-    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // (!KEEP)
     for (int it = 0; it < items; it++) {
         const int g = g0 + (KEEP ? it : it / nround), rd = KEEP ? 0 : it % nround;
         float *buf = lds6 + (it & 1) * nw * PERW, *mine = buf + wave * PERW;
@@ -139,8 +138,8 @@ __global__ __launch_bounds__(512) void m6w_kernel(const MkJob *__restrict__ jobs
         }
         if constexpr (!KEEP) load_x((it + 1) % nround);
         lds_sync();   // the item's terms are complete; the other buffer's chains (before this barrier) are done with it
-        if (chain) {
-            const int n = min(nw, nbk - rd * nw);
+        auto chain = [&](int c, float (&s)[4]) {   // chain c: activation c / 4 of the tile, rows 4 (c % 4) .. + 3
+            const int n = min(nw, nbk - rd * nw), cq = c >> 2, cr = 4 * (c & 3), q = tok0 + cq;
             const float *e = buf;
             for (int k = 0; k < n; k++, e += PERW) {
                 const float4 t = *reinterpret_cast<const float4 *>(e + cq * 16 + cr), d = *reinterpret_cast<const float4 *>(e + TOT + cr);
@@ -171,6 +170,14 @@ __global__ __launch_bounds__(512) void m6w_kernel(const MkJob *__restrict__ jobs
                 }
                 s[0] = s[1] = s[2] = s[3] = 0.0f;
             }
+        };
+        if constexpr (KEEP) {   // a row of fewer superblocks than the tile has 16 activations: fewer threads than chains
+            for (int c = tid; c < WN * 64; c += blockDim.x) {
+                float s0[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                chain(c, s0);
+            }
+        } else if (tid < WN * 64) {   // the sums live over the row's rounds, in the chain's one thread
+            chain(tid, s);
         }
     }
 }
@@ -193,7 +200,8 @@ hipError_t launch(int nw, bool keep, const MkJob *jobs, int njobs, const MkJob &
 }  // namespace
 
 hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob &single, int grid, int order, hipStream_t s) {
-    switch (nw >= 1 && nw <= M6W_WAVES ? wn : 0) {
+    // over several rounds every chain needs a thread of its own
+    switch (nw >= 1 && nw <= M6W_WAVES && (keep || nw >= wn) ? wn : 0) {
     case 1: return launch<1>(nw, keep, jobs, njobs, single, grid, order, s);
     case 2: return launch<2>(nw, keep, jobs, njobs, single, grid, order, s);
     case 4: return launch<4>(nw, keep, jobs, njobs, single, grid, order, s);

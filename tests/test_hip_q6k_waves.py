@@ -81,7 +81,8 @@ def test_several_products_in_a_launch(hip, orc):
     [(16, 4, 5), (300, 4, 2), (250, 2, 4)],                           # few products of 5: all in the decode launch
     [(64, 9, 6), (64, 9, 1)], [(64, 9, 9), (64, 9, 1)],               # rows longer than its waves
     [(40, 2, 9), (40, 2, 33), (40, 2, 2)],                            # every kind
-], ids=["chunks", "tiles", "beside", "left", "long6", "long9", "mixed"])
+    [(1024, 3, 33 + 5 * j) for j in range(8)],                        # four tiles of activations, three waves
+], ids=["chunks", "tiles", "beside", "left", "long6", "long9", "mixed", "threes"])
 def test_batches(hip, orc, shapes):
     specs, want, outs, keep = [], [], [], []
     for j, (rows, nbk, na) in enumerate(shapes):
@@ -99,3 +100,27 @@ def test_batches(hip, orc, shapes):
     plan.close()
     for dY, w in zip(outs, want):
         assert np.array_equal(bits(hip.download(dY, np.zeros_like(w))), bits(w))
+
+
+@pytest.mark.parametrize("nbk", [1, 2, 3, 4, 8, 9, 17])
+@pytest.mark.parametrize("rows", [4096, 8203])
+def test_several_tiles_of_activations(hip, orc, nbk, rows):
+    """at least 256 row groups, so that a workgroup takes 2 or 4 tiles of 16 activations: rows of fewer superblocks (so fewer
+    waves) than tiles, full and ragged tiles, several rounds per row; every output against the vector kernel, the first and last
+    activations of the tiles against the oracle"""
+    cols = 256 * nbk
+    st = np.array([nbk * 100 + rows], np.uint64)
+    W = orc.mtest_blocks(O.Q6_K, st, rows, cols)
+    every = orc.quantize_act(O.Q6_K, orc.mtest_acts(st, 128 * cols).reshape(128, cols))
+    r0, ys = (5 if rows > 4096 else 0), rows + 3
+    for na in (17, 31, 32, 33, 48, 49, 64, 65, 128):
+        acts = np.ascontiguousarray(every[:na])
+        y = run(hip, W, cols, rows, acts, r0, rows, ys)
+        prev = hip.set_q6k_mfma_min_batch(0)
+        try:
+            ref = run(hip, W, cols, rows, acts, r0, rows, ys)
+        finally:
+            hip.set_q6k_mfma_min_batch(prev)
+        assert np.array_equal(bits(y), bits(ref)), na
+    pick = [0, 15, 16, 31, 32, 47, 48, 63, 64, 127]
+    assert np.array_equal(bits(y[pick, r0:rows]), bits(orc.matvec_multi(O.Q6_K, W, cols, rows, np.ascontiguousarray(every[pick]))[:, r0:]))
