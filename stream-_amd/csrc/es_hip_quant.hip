@@ -540,6 +540,68 @@ bool pk_schedule(PkGroup &g, int cus) {
     return pk_schedule_form(g, cus);
 }
 
+// one tile's record: rows [r0 + 64 rt, ...) of product p, nt activations from t0 on
+esq::PkTile pk_tile(const PkGroup::Prod &p, int rt, int t0, int nt, bool t64) {
+    const int row0 = p.r0 + esq::MK_ROWS * rt;
+    esq::PkTile r{};
+    r.w = p.W + (size_t)row0 * p.row_bytes;
+    r.act = p.act;
+    r.y = p.y + (size_t)t0 * p.ystride + row0;
+    r.astride = p.astride;
+    r.ystride4 = 4u * p.ystride;
+    r.row_bytes = p.row_bytes;
+    r.nbk = p.nbk;
+    r.t64 = t64 ? 1 : 0;
+    r.tok0 = t0;
+    r.na = p.na;
+    r.rows = std::min(esq::MK_ROWS, p.r1 - row0);
+    r.ntok = nt;
+    return r;
+}
+
+// whether product p of a launch in the two-workgroup form takes 64-wide tiles
+bool pk_narrow(const PkGroup::Prod &p, double mean) { return p.na <= 64 || pk_cost(p.nbk, false) > mean; }
+
+// The schedule of products whose tiles all cost the same, as pk_schedule_form's sorts and heaps come out then: row tile o on
+// XCD o % 8, an XCD's tiles dealt in turn to its workgroups. Written down directly, since a batch that is not kept is planned
+// on every call, on the calling thread: an 8192 x 2048 product 36 -> 3.2 us at 64 activations and 84 -> 7.5 at 512, a layer's
+// two batches (2048/8192, Q5_K or Q4_K) 84 -> 10 and 225 -> 25. False: not such products. g.grid 0: some workgroup would get
+// more than PK_MAX_TILES tiles.
+bool pk_schedule_even(PkGroup &g, int G, double mean) {
+    const PkGroup::Prod &f = g.prods[0];
+    const bool t64 = !g.ws && pk_narrow(f, mean);
+    const int T = g.ws ? g.ws_tok : t64 ? 64 : 128, ntt = (f.na + T - 1) / T;
+    int nrt = 0;
+    for (const PkGroup::Prod &p : g.prods) {
+        if (p.nbk != f.nbk || (p.na + T - 1) / T != ntt || (!g.ws && pk_narrow(p, mean) != t64)) return false;
+        nrt += (p.r1 - p.r0 + esq::MK_ROWS - 1) / esq::MK_ROWS;
+    }
+    const int m = G / 8;   // workgroups of an XCD
+    g.grid = 0;
+    if (((long)(nrt + 7) / 8 * ntt + m - 1) / m > esq::PK_MAX_TILES) return true;
+    struct Rt { int p, rt; };
+    std::vector<Rt> rts;
+    rts.reserve(nrt);
+    for (int pi = 0; pi < (int)g.prods.size(); pi++)
+        for (int rt = 0; rt < (g.prods[pi].r1 - g.prods[pi].r0 + esq::MK_ROWS - 1) / esq::MK_ROWS; rt++) rts.push_back({pi, rt});
+    g.grid = G;
+    g.g64 = t64 ? G : 0;
+    g.tiles.clear();
+    g.tiles.reserve((size_t)nrt * ntt);
+    g.wgptr.assign(G + 1, 0);
+    for (int w = 0; w < G; w++) {
+        const int x = w % 8, have = (nrt - x + 7) / 8 * ntt;   // tiles of this workgroup's XCD
+        for (int k = w / 8; k < have; k += m) {
+            const Rt &o = rts[x + 8 * (k / ntt)];
+            const PkGroup::Prod &p = g.prods[o.p];
+            const int t0 = k % ntt * T;
+            g.tiles.push_back(pk_tile(p, o.rt, t0, std::min(T, p.na - t0), t64));
+        }
+        g.wgptr[w + 1] = (int)g.tiles.size();
+    }
+    return true;
+}
+
 bool pk_schedule_form(PkGroup &g, int cus) {
     const int G = (g.ws ? 1 : 2) * std::max(cus, 8) / 8 * 8;
     struct Tl { int p, rt, t0, nt; bool t64; double c; };
@@ -548,10 +610,11 @@ bool pk_schedule_form(PkGroup &g, int cus) {
     for (const PkGroup::Prod &p : g.prods)
         mean += (double)((p.r1 - p.r0 + esq::MK_ROWS - 1) / esq::MK_ROWS) * ((p.na + 127) / 128) * pk_cost(p.nbk, false);
     mean /= G;
+    if (pk_schedule_even(g, G, mean)) return g.grid > 0;
     for (int pi = 0; pi < (int)g.prods.size(); pi++) {
         const PkGroup::Prod &p = g.prods[pi];
         const int rts = (p.r1 - p.r0 + esq::MK_ROWS - 1) / esq::MK_ROWS;
-        const bool t64 = !g.ws && (p.na <= 64 || pk_cost(p.nbk, false) > mean);
+        const bool t64 = !g.ws && pk_narrow(p, mean);
         const int T = g.ws ? g.ws_tok : t64 ? 64 : 128;
         for (int rt = 0; rt < rts; rt++)
             for (int t0 = 0; t0 < p.na; t0 += T)
@@ -670,21 +733,7 @@ bool pk_schedule_form(PkGroup &g, int cus) {
     for (const auto &pt : placed) {
         const Tl &t = *pt.first;
         const PkGroup::Prod &p = g.prods[t.p];
-        const int row0 = p.r0 + esq::MK_ROWS * t.rt;
-        esq::PkTile r{};
-        r.w = p.W + (size_t)row0 * p.row_bytes;
-        r.act = p.act;
-        r.y = p.y + (size_t)t.t0 * p.ystride + row0;
-        r.astride = p.astride;
-        r.ystride4 = 4u * p.ystride;
-        r.row_bytes = p.row_bytes;
-        r.nbk = p.nbk;
-        r.t64 = t.t64 ? 1 : 0;
-        r.tok0 = t.t0;
-        r.na = p.na;
-        r.rows = std::min(esq::MK_ROWS, p.r1 - row0);
-        r.ntok = t.nt;
-        g.tiles.push_back(r);
+        g.tiles.push_back(pk_tile(p, t.rt, t.t0, t.nt, t.t64));
     }
     return true;
 }

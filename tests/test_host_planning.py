@@ -1,0 +1,114 @@
+"""The library's host side on the CPU, with its HIP calls answered by tests/_hip_stub.c in a child process: the tile schedules of
+the persistent launches of Q5_K, Q4_K and Q3_K batches, what planning one costs, and which calls allocate, copy or wait."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+pytestmark = pytest.mark.skipif(not os.path.isdir("/opt/rocm/include/hip"), reason="no HIP headers")
+
+COMMON = r"""
+import ctypes as C, json, os, sys, time
+import numpy as np
+sys.path.insert(0, os.path.join(ROOT, "stream-_amd"))
+import es_hip_quant as E
+L, S = E.Lib(), C.CDLL(STUB)
+assert L.available(), L.last_error()
+counts = (C.c_long * 5).in_dll(S, "counts")
+def reset():
+    for i in range(5): counts[i] = 0
+def job(t, rows, cols, na, k):   # (addresses are never read)
+    return dict(type=t, rows=rows, cols=cols, W=(k + 1) << 40, act=1 << 50, astride=cols // 256 * 292, nb=na, y=(k + 1) << 52, ystride=rows)
+"""
+
+
+@pytest.fixture(scope="module")
+def child(hiplib, tmp_path_factory):
+    so = tmp_path_factory.mktemp("stub") / "stub.so"
+    subprocess.run(["gcc", "-O2", "-w", "-shared", "-fPIC", "-I/opt/rocm/include", "-o", str(so), os.path.join(ROOT, "tests", "_hip_stub.c")],
+                   check=True)
+
+    def run(code):
+        r = subprocess.run([sys.executable, "-c", f"ROOT, STUB = {ROOT!r}, {str(so)!r}\n" + COMMON + code], capture_output=True, text=True,
+                           env=dict(os.environ, LD_PRELOAD=str(so)), timeout=300)
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+        return json.loads(r.stdout.splitlines()[-1])
+
+    return run
+
+
+SCHEDULE = r"""
+rec = np.dtype([("w", "<u8"), ("act", "<u8"), ("y", "<u8"), ("astride", "<u4"), ("ystride4", "<u4"), ("row_bytes", "<u4"), ("nbk", "<i4"),
+                ("t64", "<i4"), ("tok0", "<i4"), ("na", "<i4"), ("rows", "<i4"), ("ntok", "<i4"), ("pad", "<i4")])
+bad = []
+def check(t, shapes, on):
+    L.set_direct_persistent(on)
+    p = L.plan([job(t, r, c, na, k) for k, (r, c, na) in enumerate(shapes)])
+    n = C.c_size_t.in_dll(S, "copy_bytes").value
+    raw = C.string_at(C.c_void_p.in_dll(S, "copy_dst").value, n)
+    p.close()
+    for T in (64, 128):   # the launch's tile width and grid, from the table's own end
+        nt = sum((r + 63) // 64 * ((na + T - 1) // T) for r, _, na in shapes)
+        at = (nt * 64 + 255) // 256 * 256
+        for grid in (512, 256):
+            if at + 4 * (grid + 1) > n: continue
+            ptr = np.frombuffer(raw, "<i4", grid + 1, at)
+            if ptr[0] == 0 and ptr[-1] == nt and np.all(np.diff(ptr) >= 0): break
+        else: continue
+        break
+    else:
+        bad.append([t, shapes, on, "no table"]); return
+    tiles = np.frombuffer(raw, rec, nt)
+    bb = {E.Q3_K: 110, E.Q4_K: 144, E.Q5_K: 176}[t]
+    want = {((k + 1 << 40) + 64 * rt * c // 256 * bb, t0) for k, (r, c, na) in enumerate(shapes) for rt in range((r + 63) // 64)
+            for t0 in range(0, na, T)}
+    got = [(int(x["w"]), int(x["tok0"])) for x in tiles]
+    wg = np.repeat(np.arange(grid), np.diff(ptr))
+    xcd = {}
+    for x, w in zip(tiles, wg): xcd.setdefault(int(x["w"]), set()).add(int(w) % 8)
+    load = np.diff(ptr).reshape(-1, 8)   # [workgroup of the XCD][XCD]
+    rts = np.bincount([next(iter(v)) for v in xcd.values()], minlength=8)
+    ok = (sorted(got) == sorted(want) and all(len(v) == 1 for v in xcd.values()) and np.all(load.max(0) - load.min(0) <= 1) and
+          rts.max() - rts.min() <= 1)
+    for x in tiles:
+        k = (int(x["w"]) >> 40) - 1
+        r, c, na = shapes[k]
+        row0 = (int(x["w"]) - (k + 1 << 40)) // (c // 256 * bb)
+        ok = ok and x["y"] == (k + 1 << 52) + 4 * (int(x["tok0"]) * r + row0) and x["rows"] == min(64, r - row0)
+        ok = ok and x["ntok"] == min(T, na - x["tok0"]) and x["na"] == na and x["nbk"] == c // 256 and x["t64"] == (T == 64 and grid == 512)
+    if not ok: bad.append([t, shapes, on, T, grid])
+for t in (E.Q3_K, E.Q4_K, E.Q5_K):
+    for on in (1, 3) if t != E.Q5_K else (1,):
+        for r in (1, 64, 65, 500, 2048, 8192, 8200):
+            for na in (33, 64, 65, 128, 129, 512):
+                check(t, [(r, 2048, na)], on)
+                check(t, [(r, 2048, na), (2 * r + 7, 2048, na)], on)
+print(json.dumps(bad))
+"""
+
+
+def test_even_schedules(child):
+    """products whose tiles cost the same: every tile once, a row tile's tiles on one XCD, tiles dealt evenly"""
+    assert child(SCHEDULE) == []
+
+
+def test_planning_time(child):
+    """a persistent launch of 256 tiles is planned in a few times what the same products' one-workgroup-per-tile launch takes (the
+    sorts and heaps of the general schedule made it over 30 times), so a batch that is planned on every call is not bound by it"""
+    r = child(r"""
+out = []
+for on in (3, 1):
+    L.set_direct_persistent(on)
+    best = 1e9
+    for _ in range(200):
+        jobs, n = L.make_jobs([job(E.Q5_K, 8192, 2048, 64, k) for k in range(2)])
+        t0 = time.perf_counter()
+        for _ in range(10): L._L.es_hip_plan_destroy(L._L.es_hip_plan_create(jobs, n))
+        best = min(best, (time.perf_counter() - t0) * 1e5)
+    out.append(best)
+print(json.dumps(out))
+""")
+    assert r[1] < 8 * r[0] + 5, r
