@@ -1801,8 +1801,10 @@ int es_hip_matvec_multi_dev_noalloc(uint32_t type, const void *W, int cols, int 
         return bt.mv.empty() ? ES_HIP_OK : launch_single(bt.mv[0], s);
     size_t need = align256(bt.table_bytes) + bt.ws_bytes;
     const size_t ws_at = align256(bt.table_bytes);
-    if (type == ES_HIP_Q6_K && na >= 16)   // the limit holds whichever Q6_K kernel serves the call: the tiled one's pre-pass planes
-        need = std::max(need, align256((size_t)(cols / 256) * ((na + 63) / 64 * 64) * 256) + align256((size_t)(cols / 256) * ((na + 63) / 64 * 64) * 36));
+    if (type == ES_HIP_Q6_K && na >= 16) {   // the limit holds whichever Q6_K kernel serves the call: the tiled one's tables and planes
+        const size_t n = (size_t)(cols / 256) * (na <= 16 ? 16 : na <= 32 ? 32 : (na + 63) / 64 * 64);
+        need = std::max(need, align256(sizeof(esq::MmJob)) + align256(sizeof(esq::PrepJob)) + align256(n * 256) + align256(n * 36));
+    }
     if (need > NOALLOC_SCRATCH)
         return fail(ES_HIP_EINVAL, "this product needs %zu bytes of job tables and workspace, more than the %zu bytes of the "
                                    "no-allocation scratch (use es_hip_matvec_multi_dev)", need, NOALLOC_SCRATCH);

@@ -112,3 +112,29 @@ for on in (3, 1):
 print(json.dumps(out))
 """)
     assert r[1] < 8 * r[0] + 5, r
+
+
+NOALLOC = r"""
+def noalloc(t, rows, cols, na):
+    return L._L.es_hip_matvec_multi_dev_noalloc(t, 1 << 40, cols, 0, rows, 1 << 50, E.act_bytes(t, cols), na, 1 << 52, rows, None)
+"""
+
+
+def test_noalloc_q6k_limit(child):
+    """the no-allocation product's row limit for Q6_K is the tiled kernel's (tables and pre-pass planes of 16, 32 or a multiple of
+    64 activations in 32 MiB), whichever kernel serves the call"""
+    r = child(NOALLOC + r"""
+def ok(nbk, na):
+    n = nbk * (16 if na <= 16 else 32 if na <= 32 else (na + 63) // 64 * 64)
+    up = lambda v: (v + 255) // 256 * 256
+    return 512 + up(n * 256) + up(n * 36) <= 32 << 20
+bad = []
+for na in (16, 17, 32, 33, 64, 65, 128, 129, 512, 2048):
+    edge = next((b for b in range(1, 4097) if not ok(b, na)), 4097)
+    for nbk in {1, edge // 2, edge - 2, edge - 1, edge, edge + 1, 4096} - {0}:
+        if nbk <= 4096 and (noalloc(E.Q6_K, 64, 256 * nbk, na) == 0) != ok(nbk, na): bad.append([na, nbk])
+for na in (1, 5, 8, 15):   # no planes: every row length
+    if noalloc(E.Q6_K, 64, 1 << 20, na): bad.append([na])
+print(json.dumps(bad))
+""")
+    assert r == []

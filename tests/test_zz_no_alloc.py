@@ -128,3 +128,10 @@ def test_noalloc_refuses_graph_capture(hip, orc):
         b.close()
     y = run(hip, hip.matvec_multi_dev_noalloc, O.Q4_K, W, cols, rows, acts)
     assert np.array_equal(bits(y), bits(run(hip, hip.matvec_multi_dev, O.Q4_K, W, cols, rows, acts)))
+
+
+def test_noalloc_long_q6k_rows(hip, orc):
+    """rows whose pre-pass planes for 16 activations fit the scratch and for 64 would not"""
+    W, acts = make(orc, O.Q6_K, 24, 524288, 16, 91)
+    y = run(hip, hip.matvec_multi_dev_noalloc, O.Q6_K, W, 524288, 24, acts)
+    assert np.array_equal(bits(y), bits(orc.matvec_multi(O.Q6_K, W, 524288, 24, acts)))
