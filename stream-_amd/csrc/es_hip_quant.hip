@@ -1805,12 +1805,16 @@ int es_hip_matvec_multi_dev_noalloc(uint32_t type, const void *W, int cols, int 
         const size_t n = (size_t)(cols / 256) * (na <= 16 ? 16 : na <= 32 ? 32 : (na + 63) / 64 * 64);
         need = std::max(need, align256(sizeof(esq::MmJob)) + align256(sizeof(esq::PrepJob)) + align256(n * 256) + align256(n * 36));
     }
+    const bool by_value = table_free(bt);
     if (need > NOALLOC_SCRATCH)
         return fail(ES_HIP_EINVAL, "this product needs %zu bytes of job tables and workspace, more than the %zu bytes of the "
                                    "no-allocation scratch (use es_hip_matvec_multi_dev)", need, NOALLOC_SCRATCH);
+    // a product that travels with its launch touches the scratch only for its pre-pass planes
+    if (by_value && !bt.ws_bytes) return launch_batch(bt, nullptr, g_order.load(), s);
     uint8_t *dev = nullptr;
     if (int rc = scratch_address(&dev)) return rc;
     bind(bt, dev + ws_at);
+    if (by_value) return launch_batch(bt, nullptr, g_order.load(), s);
     // Every pre-pass writes all of its padded planes (zeros past na), so nothing in the scratch needs clearing; the
     // tables are copied from pageable memory, which the copy has consumed when it returns.
     const std::vector<uint8_t> img = table_image(bt);

@@ -138,3 +138,18 @@ for na in (1, 5, 8, 15):   # no planes: every row length
 print(json.dumps(bad))
 """)
     assert r == []
+
+
+def test_noalloc_by_value(child):
+    """a no-allocation product that is one job of one launch (and its pre-pass) travels as kernel arguments: nothing is copied, and
+    without a pre-pass nothing of the shared scratch is used; only tile schedules (Q3_K and Q4_K on the persistent kernel) are"""
+    r = child(NOALLOC + r"""
+out = []
+for t in (E.Q4_0, E.Q5_0, E.Q8_0, E.Q2_K, E.Q4_K, E.Q6_K):
+    for na in (1, 2, 5, 8, 15, 16, 31):
+        reset()
+        assert noalloc(t, 2048, 2048, na) == 0, L.last_error()
+        if counts[0] < 1 or counts[1] or counts[2] or counts[3]: out.append([t, na, list(counts)])
+print(json.dumps(out))
+""")
+    assert r == []

@@ -135,3 +135,30 @@ def test_noalloc_long_q6k_rows(hip, orc):
     W, acts = make(orc, O.Q6_K, 24, 524288, 16, 91)
     y = run(hip, hip.matvec_multi_dev_noalloc, O.Q6_K, W, 524288, 24, acts)
     assert np.array_equal(bits(y), bits(orc.matvec_multi(O.Q6_K, W, 524288, 24, acts)))
+
+
+def test_noalloc_small_q6k_on_two_streams(hip, orc):
+    """Q6_K products of 5 to 15 activations travel with their launches and share nothing: calls on two streams may overlap"""
+    import ctypes as C
+    import glob
+    hiprt = C.CDLL(sorted(glob.glob("/opt/rocm/lib/libamdhip64.so*"))[0])
+    streams = [C.c_void_p(), C.c_void_p()]
+    for s in streams:
+        assert hiprt.hipStreamCreate(C.byref(s)) == 0
+    try:
+        shapes, work = [(2048, 2048, 8), (1000, 1024, 5)], []
+        for k, (rows, cols, na) in enumerate(shapes):
+            W, acts = make(orc, O.Q6_K, rows, cols, na, 300 + k)
+            work.append((hip.upload(W), hip.upload(acts), hip.upload(np.full((20, na, rows), -5.0, np.float32)), acts.strides[0],
+                         orc.matvec_multi(O.Q6_K, W, cols, rows, acts)))
+        hip.synchronize()
+        for i in range(20):
+            for (rows, cols, na), (dW, dA, dY, astride, _), s in zip(shapes, work, streams):
+                hip.matvec_multi_dev_noalloc(O.Q6_K, dW, cols, 0, rows, dA, astride, na, int(dY) + 4 * i * na * rows, rows, stream=s.value)
+        hip.synchronize()
+        for (rows, cols, na), (_, _, dY, _, ref) in zip(shapes, work):
+            y = hip.download(dY, np.zeros((20, na, rows), np.float32))
+            assert all(np.array_equal(bits(y[i]), bits(ref)) for i in range(20)), (rows, cols, na)
+    finally:
+        for s in streams:
+            hiprt.hipStreamDestroy(s)
