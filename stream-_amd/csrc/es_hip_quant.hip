@@ -1796,7 +1796,13 @@ int es_hip_matvec_multi_dev_noalloc(uint32_t type, const void *W, int cols, int 
                                    "memory at the call, so it cannot be recorded into a graph");
     std::vector<Req> reqs{{type, W, act, y, nullptr, nullptr, r0, r1, cols, na, astride, ystride}};
     Batch bt;
-    if (int rc = plan_batch(reqs, bt)) return rc;
+    // Nothing is kept here, so a persistent launch's tile tables are planned and copied on every call. A Q5_K product takes one
+    // only where its tables are short and the per-tile launch has wider tiles to fill than activations (fewer than 64 of 128);
+    // else that launch goes by value. Per call back to back (us, persistent / per tile): 2048 x 8192 at 8 and 32 41.1 / 58.9,
+    // 42.0 / 59.5, at 128 and 512 42.6 / 43.3, 58.2 / 45.4; 8192 x 2048 at 8 and 32 15.6 / 17.5, 15.9 / 17.6, at 128 and 512 31.3 /
+    // 14.0, 47.8 / 30.9; 32768 x 2048 at 8 29.5 / 28.0 without the copy of 34 KB.
+    const bool pk = type != ES_HIP_Q5_K || (na < 64 && (long)r1 - r0 <= 64 * 128);
+    if (int rc = plan_batch(reqs, bt, pk)) return rc;
     if (bt.mm.empty() && bt.mqg.empty() && bt.mbg.empty() && bt.mkg.empty() && bt.pkg.empty())
         return bt.mv.empty() ? ES_HIP_OK : launch_single(bt.mv[0], s);
     size_t need = align256(bt.table_bytes) + bt.ws_bytes;

@@ -153,3 +153,17 @@ for t in (E.Q4_0, E.Q5_0, E.Q8_0, E.Q2_K, E.Q4_K, E.Q6_K):
 print(json.dumps(out))
 """)
     assert r == []
+
+
+def test_noalloc_q5k_tables(child):
+    """Q5_K products: tile tables are copied only where they are short and the per-tile launch is the slower one"""
+    r = child(NOALLOC + r"""
+out = []
+for rows in (64, 2048, 8192, 8256, 32768):
+    for na in (1, 8, 63, 64, 65, 128, 512):
+        reset()
+        assert noalloc(E.Q5_K, rows, 2048, na) == 0, L.last_error()
+        if counts[2] != (8 <= na < 64 and rows <= 8192) or C.c_size_t.in_dll(S, "copy_bytes").value > 16384: out.append([rows, na, list(counts)])
+print(json.dumps(out))
+""")
+    assert r == []

@@ -162,3 +162,13 @@ def test_noalloc_small_q6k_on_two_streams(hip, orc):
     finally:
         for s in streams:
             hiprt.hipStreamDestroy(s)
+
+
+@pytest.mark.parametrize("rows,cols,na", [(2048, 2048, 8), (8192, 1024, 63), (8256, 1024, 33), (2048, 2048, 64), (300, 4096, 200)])
+def test_noalloc_q5k(hip, orc, rows, cols, na):
+    """either side of the rule that sends a Q5_K product to the persistent launch"""
+    W, acts = make(orc, O.Q5_K, rows, cols, na, rows + na)
+    y = run(hip, hip.matvec_multi_dev_noalloc, O.Q5_K, W, cols, rows, acts)
+    assert np.array_equal(bits(y), bits(run(hip, hip.matvec_multi_dev, O.Q5_K, W, cols, rows, acts)))
+    pick = [0, na // 2, na - 1]
+    assert np.array_equal(bits(y[pick]), bits(orc.matvec_multi(O.Q5_K, W, cols, rows, acts[pick])))
