@@ -765,25 +765,35 @@ bool m6w_capable(const Req &q) {
     return (size_t)q.na * stride < ((size_t)1 << 32) - 65536 && (size_t)q.r1 * nbk * 210 < ((size_t)1 << 32);
 }
 // Which of a batch's Q6_K products take it: those of 16 activations or more, and those of fewer, each where the launch of all
-// of them is the faster one. The tiled kernel (es_hip_mm6.hip) runs a tile's superblocks one after another, 2.4 us each, a set
-// of 256 tiles of 128 rows x 64 activations at a time (2 us more each), behind a pre-pass (6 us); this one takes about 1.4 ns
-// per superblock of 16 rows x 16 wn activations, 2.3 with several superblocks per wave, and 5 us. Measured (us, this kernel /
-// tiled): 2048 x 8192 at 64, 128 and 512 activations 24 / 79, 41 / 78, 141 / 79; 8192 x 2048 13 / 26, 18 / 26, 50 / 48; 4096 x
-// 4096 21 / 44, 37 / 43, 129 / 47. Against the decode kernel's passes of 4 at 8 activations 8192 x 2048 9.3 / 14.1, 151936 x 1024
-// 57 / 66 (2048 x 8192 16.6 / 15.2), and slower at 4 (8.9 / 8.6). Batches of these (us, this kernel / decode kernel): 112 x
-// 2048 x 768 at 5, 8 and 12 69 / 63, 69 / 74, 69 / 108, 32 of them at 6 22.5 / 29; 16 x 8192 x 2048 86 / 76, 86 / 87, 87 / 128, two 13.4 /
-// 17.8, 13.7 / 20.8; 16 x 2048 x 8192 104 / 77, 106 / 88, 109 / 129, two 15.8 / 17.7. So a batch that fills the device anyway takes it
-// from a mean of 7 activations, 9 with rows longer than its waves, a small one always; where products of fewer activations
-// need a decode launch beside it, it must have half of the weights (8192 x 2048 at 8 and at 1 14.0 / 19.6; an expert layer with
-// a few experts at 5 and 6 123 / 115) and rows not too long (2048 x 8192 at 8 with 512 x 2048 at 2 21.6 / 19.9). 64 x 2048 x 768 at
-// 20 and 40 against the tiled kernel 36.6 / 43.5, 44.8 / 54.8. A product of one activation tile and many row tiles whose
-// activations fit the LDS keeps the tiled kernel's persistent form (151936 x 1024 at 16 and 64: 57 / 43, 61 / 58).
+// of them is the faster one. Measured with weights from HBM (us, this kernel / the other).
+// 16 or more, against the tiled kernel (es_hip_mm6.hip): that one runs a tile's superblocks one after another, 2.4 us each
+// (1.9 at up to 16 activations, whose tiles are narrower), a set of 256 tiles of 128 rows x 64 activations at a time (2 us
+// more each; a product's row tiles are dealt to the XCDs in eights, and each tile width is a launch of its own), behind a
+// pre-pass (6 us). This one takes 5 us and about 1.4 ns per superblock of 16 rows x 16 wn activations, 2.3 with several
+// superblocks per wave; 3, 5 or 7 waves take as long as 4, 6 or 8. 8192 x 2048 at 64, 128 and 512 activations 13 / 25, 18 /
+// 28, 48 / 50; 2048 x 8192 at 64, 256 and 512 24 / 82, 75 / 84, 145 / 84; 8192 x 768 at 64, 128 and 256 8.6 / 14.2, 12.4 /
+// 14.3, 17.9 / 15.4; 8192 x 1280 at 256 23.1 / 19.9; 16 x 2048 x 768 at 16 and 64 15.0 / 13.7, 18.1 / 16.6; 32768 x 1536 at
+// 16 24.0 / 20.5; 16 x 2048 x 768 at 16 to 60 29.6 / 36.3. It errs by less than a tenth (8192 x 1024 at 256 18.5 / 17.3,
+// taken; 32768 x 2048 at 64 29.0 / 31.4, not taken). A product of one activation tile and many row tiles whose activations
+// fit the LDS keeps the tiled kernel's persistent form (151936 x 1024 at 16 and 64: 57 / 43, 61 / 58).
+// Fewer than 16, against the decode kernel's passes of 4, which are faster below 5 (8192 x 2048 at 4: 8.9 / 8.6). A batch
+// that fills the device anyway takes this kernel from a mean of 7 activations, of 9 with rows longer than its waves (112 x
+// 2048 x 768 at 5, 8 and 12 70 / 72, 69 / 80, 69 / 113; 16 x 2048 x 8192 111 / 89, 111 / 101, 113 / 144; at its worst 16 x
+// 8192 x 768 at 8 44.8 / 42.9). A small one takes it from 5 (2048 x 768 at 5 and 8 4.3 / 13.0, 4.3 / 15.2; 8192 x 2048 9.7 /
+// 12.8, 9.7 / 14.6; 2048 x 6144 12.8 / 14.9, 13.0 / 16.9) unless its rows are so long that their rounds, one after another,
+// outlast the decode kernel's passes: up to 14 + 2 x mean superblocks (2048 x 7168 at 5 and 7 15.8 / 15.2, 16.0 / 16.7; 2048
+// x 8192 at 5, 8 and 9 17.2 / 13.5, 17.4 / 15.3, 17.5 / 19.0), or rows enough for every CU (4096 x 8192 at 6 17.4 / 17.9).
+// Where products of fewer than 5 activations need a decode launch beside it, that costs 6 to 8 us: it must have half of the
+// weights and a mean of 9 (7 with rows of fewer superblocks than waves: 16 x 2048 x 768 at 3 to 15 25.5 / 28.9), with very
+// long rows also rows enough (8192 x 2048 at 8 and 9 with 512 x 2048 at 2 17.3 / 15.9, 17.3 / 19.3; 2048 x 4096 at 9 16.2 /
+// 17.2; 2048 x 8192 at 12 25.5 / 21.9; 4096 x 8192 at 9 25.3 / 28.6), or be short (2048 x 768 at 5 10.7 / 13.5; 2048 x 2048
+// at 5 and 8 12.1 / 11.6, 12.3 / 13.3).
 struct M6wChoice { bool few = false, many = false; long gfew = 0, gmany = 0; };   // groups: rows / 16 of either kind
 M6wChoice m6w_choose(const std::vector<Req> &reqs, int cus) {
     M6wChoice c;
-    long sfew = 0, afew = 0, rest = 0, tiles = 0;   // superblocks below 16 (and times activations), those left to the decode kernel
-    int nbk_max = 0;
-    bool longr = false;
+    long sfew = 0, afew = 0, rest = 0;   // superblocks below 16 (and times activations), those left to the decode kernel
+    long tiles[3] = {0, 0, 0};           // the tiled kernel's launches, by tile width: tiles of up to 16, 32, 64 activations
+    int nbk_max[3] = {0, 0, 0}, nbk_few = 0;
     for (const Req &q : reqs) {
         if (q.type != ES_HIP_Q6_K || q.r1 <= q.r0 || q.na <= 0) continue;
         const long g = (q.r1 - q.r0 + 15) / 16, blocks = (long)(q.r1 - q.r0) * (q.cols / 256);
@@ -792,22 +802,33 @@ M6wChoice m6w_choose(const std::vector<Req> &reqs, int cus) {
         } else if (q.na < 16) {
             sfew += blocks;
             afew += blocks * q.na;
-            longr = longr || q.cols / 256 > esq::M6W_WAVES;
+            nbk_few = std::max(nbk_few, q.cols / 256);
             c.gfew += g;
         } else {
             c.gmany += g;
-            tiles += (long)((q.r1 - q.r0 + 127) / 128) * ((q.na + 63) / 64);
-            nbk_max = std::max(nbk_max, q.cols / 256);
+            const int w = q.na <= 16 ? 0 : q.na <= 32 ? 1 : 2;
+            tiles[w] += 8L * ((q.r1 - q.r0 + 1023) / 1024) * ((q.na + 63) / 64);   // (row tiles come in eights, one per XCD)
+            nbk_max[w] = std::max(nbk_max[w], q.cols / 256);
         }
     }
     double cost = 5.0;
     for (const Req &q : reqs)
         if (q.na >= 16 && m6w_capable(q)) {
             const int nbk = q.cols / 256, wn = m6w_tiles(c.gmany, q.na, nbk, cus);
-            cost += (double)((q.r1 - q.r0 + 15) / 16) * ((q.na + 16 * wn - 1) / (16 * wn)) * nbk * (nbk > esq::M6W_WAVES ? 2.3e-3 : 1.4e-3);
+            cost += (double)((q.r1 - q.r0 + 15) / 16) * ((q.na + 16 * wn - 1) / (16 * wn)) *
+                    (nbk > esq::M6W_WAVES ? 2.3e-3 * nbk : nbk > 1 ? 1.4e-3 * ((nbk + 1) & ~1) : 1.4e-3);
         }
-    c.many = cost < 6.0 + (2.0 + 2.4 * nbk_max) * ((tiles + cus - 1) / cus);
-    c.few = sfew > 0 && sfew >= rest && (afew >= (longr ? 9 : 7) * sfew || (sfew <= (longr ? 131072 : 262144) && !(rest && longr)));
+    double tiled = 6.0;
+    for (int w = 0; w < 3; w++) tiled += (2.0 + (w ? 2.4 : 1.9) * nbk_max[w]) * ((tiles[w] + cus - 1) / cus);
+    c.many = cost < tiled;
+    const bool longr = nbk_few > esq::M6W_WAVES, rows = sfew > 98304;   // rows enough for every CU
+    if (rest) {
+        const bool shortr = sfew <= 32768 && (nbk_few < 8 || (nbk_few == 8 && afew >= 7 * sfew));
+        c.few = sfew >= rest && (afew >= (nbk_few < 8 ? 7 : 9) * sfew ? nbk_few <= 24 || rows : shortr);
+    } else {
+        const bool small = sfew <= (longr ? 131072 : 262144) && (rows || (nbk_few - 14) * sfew <= 2 * afew);
+        c.few = sfew > 0 && (small || afew >= (longr ? 9 : 7) * sfew);
+    }
     return c;
 }
 bool m6w_eligible(const Req &q, const M6wChoice &c) {
@@ -816,9 +837,8 @@ bool m6w_eligible(const Req &q, const M6wChoice &c) {
     const int nbk = q.cols / 256, rt = (q.r1 - q.r0 + 127) / 128, bn = q.na <= 16 ? 16 : q.na <= 32 ? 32 : 64;
     return c.many && !(q.na <= 64 && rt >= 2 * device().cus && nbk <= esq::mm6_persistent_blocks(bn));
 }
-// Row groups per workgroup and the tile numbering: about one resident set of workgroups (16 waves per CU) for the launch, a
-// product's chunks a multiple of 8 (workgroup g runs on XCD g % 8: 112
-// products of 2048 rows in 5 chunks each left three XCDs idle, 115 us; in 8 chunks 69).
+// Row groups per workgroup and the tile numbering: about 8 waves per CU for the launch, a product's chunks a multiple of 8
+// (workgroup g runs on XCD g % 8: 112 products of 2048 rows in 5 chunks each left three XCDs idle, 115 us; in 8 chunks 69).
 void m6w_tiling(MkGroup &g, int cus) {
     long units = 0;
     for (const esq::MkJob &j : g.jobs) units += (long)((j.r1 - j.r0 + 15) / 16) * j.ntok_tiles;

@@ -1,5 +1,6 @@
 """The library's host side on the CPU, with its HIP calls answered by tests/_hip_stub.c in a child process: the tile schedules of
-the persistent launches of Q5_K, Q4_K and Q3_K batches, what planning one costs, and which calls allocate, copy or wait."""
+the persistent launches of Q5_K, Q4_K and Q3_K batches, what planning one costs, which calls allocate, copy or wait, and which kernel
+a Q6_K batch takes."""
 import json
 import os
 import subprocess
@@ -167,3 +168,33 @@ for rows in (64, 2048, 8192, 8256, 32768):
 print(json.dumps(out))
 """)
     assert r == []
+
+
+Q6K_WAVES = [   # batches faster on the kernel with one wave per superblock: (rows, superblocks, activations) of each product
+    [(2048, 3, 5)], [(8192, 8, 5)], [(2048, 24, 5)], [(2048, 28, 7)], [(2048, 32, 9)], [(4096, 32, 6)], [(2048, 3, 8)] * 112, [(8192, 3, 64)],
+    [(8192, 3, 128)], [(8192, 8, 128)], [(2048, 32, 64)], [(2048, 32, 256)], [(512, 3, 256)] * 16, [(2048, 3, 5), (512, 8, 2)],
+    [(2048, 8, 8), (512, 8, 2)], [(2048, 16, 9), (512, 8, 2)], [(4096, 32, 9), (512, 8, 2)], [(32768, 1, 512)], [(32768, 2, 512)],
+    [(2048, 3, n) for n in (17, 25, 33, 41, 50, 60)]]
+Q6K_OTHERS = [   # ... and faster on the decode or the tiled kernel
+    [(512, 28, 5)], [(512, 32, 5)], [(2048, 32, 8)], [(512, 32, 8)] * 4, [(2048, 48, 6)], [(8192, 32, 5)], [(8192, 3, 256)], [(8192, 5, 256)],
+    [(32768, 3, 16)], [(32768, 6, 16)], [(2048, 3, 16)] * 64, [(2048, 3, 64)] * 16, [(2048, 8, 5), (512, 8, 2)], [(8192, 8, 8), (512, 8, 2)],
+    [(2048, 32, 12), (512, 8, 2)], [(8192, 8, 4)], [(2048, 32, 512)]]
+
+
+def test_q6k_kernel_choice(child):
+    """measured batches take the faster kernel (with the choice off, the launches are those of the decode and tiled kernels)"""
+    r = child(r"""
+shapes = ((C.c_long * 3) * 64).in_dll(S, "shapes")
+def launches(batch, on):
+    L.set_q6k_persistent(on)
+    p = L.plan([job(E.Q6_K, r, 256 * b, na, k) for k, (r, b, na) in enumerate(batch)])
+    reset()
+    p.run()
+    n = counts[0]
+    assert 0 < n < 64
+    p.close()
+    return [list(shapes[i]) for i in range(n)]
+def waves(batch): return launches(batch, 1) != launches(batch, 0)
+print(json.dumps([[b for b in %r if not waves(b)], [b for b in %r if waves(b)]]))
+""" % (Q6K_WAVES, Q6K_OTHERS))
+    assert r == [[], []]
