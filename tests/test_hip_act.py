@@ -191,3 +191,24 @@ def test_rmsnorm_sum_order(hip, orc, cols):
     finite = [i for i in range(rows) if np.isfinite(want[i]).all()]
     g80 = hip.download(d80, np.zeros((rows, (cols // 32) * 36), np.uint8))
     assert np.array_equal(g80[finite], blocks(orc, want[finite], "q80"))
+
+
+def test_rmsnorm_refused_rows_are_staged(hip):
+    """a row whose parallel sum is refused is added in order from on-chip copies (about 9 times an ordinary row's time here), not
+    with a memory access before every addition (50 times)"""
+    import time
+    cols = 16384
+    x = np.stack([_hard_sum_rows(cols, np.random.default_rng(1))[-1], np.random.default_rng(2).standard_normal(cols).astype(np.float32)])
+    dx, dxn = hip.upload(x), hip.alloc(cols * 4)
+    times = []
+    for r in range(2):
+        best = 1e9
+        for _ in range(6):
+            hip.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(100):
+                hip.rmsnorm_prepare_dev(int(dx) + 4 * cols * r, 0, None, 1e-6, 1, cols, dxn, 0, None, 0, None, 0)
+            hip.synchronize()
+            best = min(best, time.perf_counter() - t0)
+        times.append(best)
+    assert times[0] < 20 * times[1], times
