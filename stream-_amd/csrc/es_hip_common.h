@@ -151,8 +151,9 @@ hipError_t mbx_launch(int type, bool gather, int nbk_max, const MkJob *jobs, int
 // waves over rows_per_wg groups of 16 rows x 16 wn activations (wn 1, 2 or 4; all activation tiles of a row chunk on one XCD:
 // 8 * ceil(chunks / 8) * ntok_tiles ids per job, tile0 a multiple of 8). keep: every job has at most nw superblocks per row;
 // without it nw >= wn.
-constexpr int M6W_WAVES = 8;
-hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob &single, int grid, int order, hipStream_t s);
+// jobs: the launch's job table on the device, or null: the njobs <= M6W_INLINE jobs at hjobs travel with the launch.
+constexpr int M6W_WAVES = 8, M6W_INLINE = 4;
+hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob *hjobs, int grid, int order, hipStream_t s);
 // gather: some job of the launch reads its activation rows through arow (a separate kernel build; the others need not);
 // tok: activations per workgroup tile, MK_TOK or 64 (ntok_tiles and the tile numbering then count tiles of 64)
 hipError_t mk_launch(int type, bool gather, int tok, const MkJob *jobs, int njobs, const MkJob &single, int grid, int order,

@@ -73,12 +73,32 @@ __device__ __forceinline__ void load_b6(const uint8_t *blk, int lg, B6 &b) {   /
     b.d = ldg<float>(blk);
 }
 
+// The kernel's arguments, as one block (its first and only parameter, at offset 0 of the argument segment).
+struct M6wArgs {
+    const MkJob *jobs;   // the launch's job table, or null: grid row i runs j[i], tiles numbered from 0
+    int njobs, pad;
+    MkJob j[M6W_INLINE];
+};
+// this workgroup's job; an in-argument one is read at the grid row's offset of the argument segment, in the round trip that
+// brings the arguments themselves (found by its tile numbers it came a round trip later, 0.1 us a launch)
+__device__ __forceinline__ MkJob m6w_job(const M6wArgs &A) {
+    static_assert(sizeof(MkJob) % 4 == 0 && offsetof(M6wArgs, j) % 4 == 0, "jobs are read as dwords");
+    constexpr int N = sizeof(MkJob) / 4;
+    if (A.jobs) return uniform_job(load_tile_job(A.jobs, A.njobs, blockIdx.x));
+    typedef const __attribute__((address_space(4))) uint32_t *ArgPtr;
+    const ArgPtr src = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(M6wArgs, j) / 4 + blockIdx.y * N;
+    uint32_t v[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = src[i];
+    return uniform_job(__builtin_bit_cast(MkJob, v));
+}
+
 // KEEP: at most as many superblocks as waves (one round per row group, activation operands loaded once).
 template <int WN, bool CONTRACT, bool KEEP>
-__global__ __launch_bounds__(512) void m6w_kernel(const MkJob *__restrict__ jobs, int njobs, MkJob single) {
+__global__ __launch_bounds__(512) void m6w_kernel(M6wArgs A) {
     extern __shared__ __align__(16) float lds6[];   // two buffers of [wave][16 WN activations][16 rows] tot | d | y.d
-    const MkJob J = uniform_job(jobs ? load_tile_job(jobs, njobs, blockIdx.x) : single);
-    // all activation tiles of a row chunk on one XCD (workgroup g runs on XCD g % 8)
+    const MkJob J = m6w_job(A);
+    // all activation tiles of a row chunk on one XCD (workgroup g runs on XCD g % 8; a grid row is a multiple of 8)
     const int tile = blockIdx.x - J.tile0, kq = tile >> 3;
     const int chunk = (tile & 7) + 8 * (kq / J.ntok_tiles), tok0 = (kq % J.ntok_tiles) * 16 * WN;
     const int ngroup = (J.r1 - J.r0 + 15) / 16, g0 = chunk * J.rows_per_wg, g1 = min(ngroup, g0 + J.rows_per_wg);
@@ -107,12 +127,12 @@ __global__ __launch_bounds__(512) void m6w_kernel(const MkJob *__restrict__ jobs
     load_w(0);
     load_x(0);
 
-    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // (!KEEP)
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int it = 0; it < items; it++) {
         const int g = g0 + (KEEP ? it : it / nround), rd = KEEP ? 0 : it % nround;
         float *buf = lds6 + (it & 1) * nw * PERW, *mine = buf + wave * PERW;
-        A6 A;
-        build_a6(raw, lg, A);
+        A6 a6;
+        build_a6(raw, lg, a6);
         if (lg == 0) mine[TOT + lr] = half_bits_to_float(raw.d);
         load_w(it + 1);
 #pragma unroll
@@ -120,13 +140,13 @@ __global__ __launch_bounds__(512) void m6w_kernel(const MkJob *__restrict__ jobs
             v8h m;
 #pragma unroll
             for (int e = 0; e < 8; e++) m[e] = static_cast<_Float16>(B[c].m[e]);
-            const v4f dc = __builtin_amdgcn_mfma_f32_16x16x32_f16(A.corr, m, v4f{0, 0, 0, 0}, 0, 0, 0);
-            v4i hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(A.hi[0], B[c].x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
-            v4i lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(A.lo[0], B[c].x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
+            const v4f dc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a6.corr, m, v4f{0, 0, 0, 0}, 0, 0, 0);
+            v4i hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a6.hi[0], B[c].x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
+            v4i lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a6.lo[0], B[c].x[0], v4i{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
             for (int ks = 1; ks < 4; ks++) {
-                hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(A.hi[ks], B[c].x[ks], hi, 0, 0, 0);
-                lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(A.lo[ks], B[c].x[ks], lo, 0, 0, 0);
+                hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a6.hi[ks], B[c].x[ks], hi, 0, 0, 0);
+                lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a6.lo[ks], B[c].x[ks], lo, 0, 0, 0);
             }
             float4 t;   // rows 4 lg .. + 3 of activation 16 c + lr
             t.x = static_cast<float>(((hi[0] << 8) + lo[0]) + (int)dc[0]);
@@ -171,7 +191,7 @@ __global__ __launch_bounds__(512) void m6w_kernel(const MkJob *__restrict__ jobs
                 s[0] = s[1] = s[2] = s[3] = 0.0f;
             }
         };
-        if constexpr (KEEP) {   // a row of fewer superblocks than the tile has 16 activations: fewer threads than chains
+        if constexpr (KEEP && WN > 1) {   // a row of fewer superblocks than the tile has 16 activations: fewer threads than chains
             for (int c = tid; c < WN * 64; c += blockDim.x) {
                 float s0[4] = {0.0f, 0.0f, 0.0f, 0.0f};
                 chain(c, s0);
@@ -183,7 +203,7 @@ __global__ __launch_bounds__(512) void m6w_kernel(const MkJob *__restrict__ jobs
 }
 
 template <int WN>
-hipError_t launch(int nw, bool keep, const MkJob *jobs, int njobs, const MkJob &single, int grid, int order, hipStream_t s) {
+hipError_t launch(int nw, bool keep, const M6wArgs &A, dim3 grid, int order, hipStream_t s) {
     const bool contract = order == ES_HIP_ORDER_X86_CONTRACT;
     const auto kern = contract ? (keep ? m6w_kernel<WN, true, true> : m6w_kernel<WN, true, false>)
                                : (keep ? m6w_kernel<WN, false, true> : m6w_kernel<WN, false, false>);
@@ -193,18 +213,30 @@ hipError_t launch(int nw, bool keep, const MkJob *jobs, int njobs, const MkJob &
                                            static_cast<int>(lds));
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), lds, s, jobs, njobs, single);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, A);
     return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob &single, int grid, int order, hipStream_t s) {
+hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob *hjobs, int grid, int order, hipStream_t s) {
     // over several rounds every chain needs a thread of its own
-    switch (nw >= 1 && nw <= M6W_WAVES && (keep || nw >= wn) ? wn : 0) {
-    case 1: return launch<1>(nw, keep, jobs, njobs, single, grid, order, s);
-    case 2: return launch<2>(nw, keep, jobs, njobs, single, grid, order, s);
-    case 4: return launch<4>(nw, keep, jobs, njobs, single, grid, order, s);
+    if (nw < 1 || nw > M6W_WAVES || (!keep && nw < wn) || njobs < 1 || (!jobs && njobs > M6W_INLINE)) return hipErrorInvalidValue;
+    M6wArgs A{jobs, njobs, 0, {}};
+    dim3 g(grid);
+    if (!jobs) {
+        int most = 0;   // workgroups of the longest job; a shorter one's past its rows have nothing to do
+        for (int i = 0; i < njobs; i++) {
+            A.j[i] = hjobs[i];
+            A.j[i].tile0 = 0;
+            most = max(most, (i + 1 < njobs ? hjobs[i + 1].tile0 : grid) - hjobs[i].tile0);
+        }
+        g = dim3(most, njobs);
+    }
+    switch (wn) {
+    case 1: return launch<1>(nw, keep, A, g, order, s);
+    case 2: return launch<2>(nw, keep, A, g, order, s);
+    case 4: return launch<4>(nw, keep, A, g, order, s);
     }
     return hipErrorInvalidValue;
 }

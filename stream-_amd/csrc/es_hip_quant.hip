@@ -1240,17 +1240,20 @@ std::vector<uint8_t> table_image(const Batch &bt) {
 
 // a decode launch whose jobs travel as its arguments
 bool mv_inline(const Group &g) { return g.jobs.size() <= (size_t)esq::MV_INLINE && g.L.nt != 0; }
+bool m6w_inline(const MkGroup &g) { return g.m6_wn && g.jobs.size() <= (size_t)esq::M6W_INLINE; }   // ... and a Q6_K one
 // no launch of the batch reads anything but its arguments
 bool table_free(const Batch &bt) {   // single jobs go by value, the persistent direct kernel always reads tables
     if (!bt.pkg.empty()) return false;
     for (const Group &g : bt.mv)
         if (!mv_inline(g)) return false;
+    for (const MkGroup &g : bt.mkg)
+        if (g.jobs.size() != 1 && !m6w_inline(g)) return false;
     auto single = [](const auto &groups) {
         for (const auto &g : groups)
             if (g.jobs.size() != 1) return false;
         return true;
     };
-    return single(bt.mmg) && single(bt.mqg) && single(bt.mbg) && single(bt.mkg);
+    return single(bt.mmg) && single(bt.mqg) && single(bt.mbg);
 }
 
 // launches in stream order: pre-passes, decode kernels, matrix-core kernel. tables: the uploaded image, or null to pass
@@ -1291,7 +1294,8 @@ int launch_batch(const Batch &bt, const uint8_t *tables, int order, hipStream_t 
     }
     for (const MkGroup &g : bt.mkg) {
         const esq::MkJob *dj = tables ? reinterpret_cast<const esq::MkJob *>(tables + g.off) : nullptr;
-        if ((e = g.m6_wn ? esq::m6w_launch(g.m6_wn, g.m6_nw, g.m6_keep, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)
+        if (m6w_inline(g)) dj = nullptr;   // the jobs go with the launch
+        if ((e = g.m6_wn ? esq::m6w_launch(g.m6_wn, g.m6_nw, g.m6_keep, dj, (int)g.jobs.size(), g.jobs.data(), g.grid, order, s)
                  : g.b32  ? esq::mbx_launch(g.type, g.gather, g.nbkm, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)
                  : g.nbkm && g.gated ? esq::mxg_launch(g.gather, g.nbkm, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)
                  : g.nbkm ? esq::mx_launch(g.type, g.gather, g.nbkm, dj, (int)g.jobs.size(), g.jobs[0], g.grid, order, s)

@@ -82,7 +82,9 @@ def test_several_products_in_a_launch(hip, orc):
     [(64, 9, 6), (64, 9, 1)], [(64, 9, 9), (64, 9, 1)],               # rows longer than its waves
     [(40, 2, 9), (40, 2, 33), (40, 2, 2)],                            # every kind
     [(1024, 3, 33 + 5 * j) for j in range(8)],                        # four tiles of activations, three waves
-], ids=["chunks", "tiles", "beside", "left", "long6", "long9", "mixed", "threes"])
+    [(300, 4, 8), (33, 4, 8), (2500, 4, 7), (16, 4, 5)],              # jobs of unequal length as kernel arguments
+    [(300, 4, 8), (33, 4, 8), (2500, 4, 7), (16, 4, 5), (50, 4, 8)],  # ... and one more than fit
+], ids=["chunks", "tiles", "beside", "left", "long6", "long9", "mixed", "threes", "four", "five"])
 def test_batches(hip, orc, shapes):
     specs, want, outs, keep = [], [], [], []
     for j, (rows, nbk, na) in enumerate(shapes):

@@ -198,3 +198,19 @@ def waves(batch): return launches(batch, 1) != launches(batch, 0)
 print(json.dumps([[b for b in %r if not waves(b)], [b for b in %r if waves(b)]]))
 """ % (Q6K_WAVES, Q6K_OTHERS))
     assert r == [[], []]
+
+
+def test_q6k_pairs_travel_with_their_launch(child):
+    """gate and up of a Q6_K FFN of 5 to 64 activations on the kernel with one wave per superblock: no allocation, no copy and no
+    wait, on the first call or a later one"""
+    r = child(r"""
+out = []
+for k, na in enumerate((5, 8, 15, 16, 33, 64)):
+    for call in range(2):
+        reset()
+        assert L._L.es_hip_dense_ffn_dev(E.Q6_K, 1 << 40, E.Q6_K, 2 << 40, E.Q6_K, 3 << 40, 2048, 4096, na, 1 << 50, 292 * 8, 1 << 51, 1 << 52,
+                                         1 << 53, 2048, None) == 0, L.last_error()
+        if counts[0] != 3 or counts[1] or counts[2] or counts[3]: out.append([na, call, list(counts)])
+print(json.dumps(out))
+""")
+    assert r == []
