@@ -2846,9 +2846,12 @@ int moe_ctx_layer(es_hip_moe_ctx *c, int N, const int *sel, const float *w, cons
             a.ff = ff;
             a.n = n;
             a.order = g_order.load();
-            // rows per workgroup: about one workgroup per CU, a multiple of 8 in 8 .. 128 that fits 48 KB of LDS
-            a.rt = std::min(128, std::max(8, (int)((long)n * N / device().cus) / 8 * 8));
-            while (a.rt > 8 && esq::moe_pairs_down_lds(a.k, ff, a.rt) > 48 * 1024) a.rt -= 8;
+            // rows per workgroup: a multiple of 8 up to 128 that fits 48 KB of LDS, and of those one with whole rounds of at most
+            // a workgroup per CU (at 12 tokens of 2048 rows 96 rows made 264 workgroups for 256 CUs, 84.1 us a layer; 104 make 240)
+            int cap = 128;
+            while (cap > 8 && esq::moe_pairs_down_lds(a.k, ff, cap) > 48 * 1024) cap -= 8;
+            const long cus = device().cus, least = (n + cap - 1) / cap, rounds = (N * least + cus - 1) / cus, per = rounds * cus / N;
+            a.rt = (int)((n + per - 1) / per + 7) / 8 * 8;   // (per >= least: workgroups of a token)
             if (esq::moe_pairs_down_lds(a.k, ff, a.rt) <= 48 * 1024) {
                 hipError_t e = esq::moe_pairs_gu_launch(a, P.L, R, s);
                 a.mv.row_bytes = (uint64_t)(ff / fd.be) * fd.bb;

@@ -8,7 +8,7 @@
 long counts[5];      /* launches, allocations, copies, waits, frees */
 void *copy_dst;      /* the last copy */
 size_t copy_bytes;
-long shapes[64][3];  /* launch i: grid x, block x, dynamic LDS bytes (modulo 64 launches) */
+long shapes[64][4];  /* launch i: grid x and y, block x, dynamic LDS bytes (modulo 64 launches) */
 
 static hipError_t get(void **p, size_t n) { counts[1]++; *p = malloc(n ? n : 1); return *p ? hipSuccess : hipErrorOutOfMemory; }
 static hipError_t copy(void *d, const void *s, size_t n) { counts[2]++; copy_dst = d; copy_bytes = n; memcpy(d, s, n); return hipSuccess; }
@@ -51,8 +51,9 @@ hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t l, hipStream_t s) {
     long *r = shapes[counts[0] % 64];
     (void)s;
     r[0] = g.x;
-    r[1] = b.x;
-    r[2] = (long)l;
+    r[1] = g.y;
+    r[2] = b.x;
+    r[3] = (long)l;
     return hipSuccess;
 }
 hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *l, hipStream_t *s) {

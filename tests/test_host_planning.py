@@ -1,6 +1,6 @@
 """The library's host side on the CPU, with its HIP calls answered by tests/_hip_stub.c in a child process: the tile schedules of
-the persistent launches of Q5_K, Q4_K and Q3_K batches, what planning one costs, which calls allocate, copy or wait, and which kernel
-a Q6_K batch takes."""
+the persistent launches of Q5_K, Q4_K and Q3_K batches, what planning one costs, which calls allocate, copy or wait, which kernel a
+Q6_K batch takes, and the launches of device-routed MoE layers."""
 import json
 import os
 import subprocess
@@ -184,7 +184,7 @@ Q6K_OTHERS = [   # ... and faster on the decode or the tiled kernel
 def test_q6k_kernel_choice(child):
     """measured batches take the faster kernel (with the choice off, the launches are those of the decode and tiled kernels)"""
     r = child(r"""
-shapes = ((C.c_long * 3) * 64).in_dll(S, "shapes")
+shapes = ((C.c_long * 4) * 64).in_dll(S, "shapes")
 def launches(batch, on):
     L.set_q6k_persistent(on)
     p = L.plan([job(E.Q6_K, r, 256 * b, na, k) for k, (r, b, na) in enumerate(batch)])
@@ -212,5 +212,32 @@ for k, na in enumerate((5, 8, 15, 16, 33, 64)):
                                          1 << 53, 2048, None) == 0, L.last_error()
         if counts[0] != 3 or counts[1] or counts[2] or counts[3]: out.append([na, call, list(counts)])
 print(json.dumps(out))
+""")
+    assert r == []
+
+
+MOE = r"""
+shapes = ((C.c_long * 4) * 64).in_dll(S, "shapes")
+def layer(types, n, ff, ne, k, N):   # the launches of a layer of N tokens
+    experts = [dict(gate=(1 << 40) + e * (1 << 28), up=(2 << 40) + e * (1 << 28), down=(3 << 40) + e * (1 << 28)) for e in range(ne)]
+    ctx = L.moe_ctx(E.MoeArgs(*types, n, ff, experts, np.zeros(1, np.int32), np.zeros((1, k), np.int32), np.zeros((1, k), np.float32)), N, k)
+    reset()
+    ctx.run(N, 1 << 50, 1 << 51, 1 << 52, E.act_bytes(types[0], n), 1 << 53, n)
+    r = [list(shapes[i]) for i in range(counts[0])]
+    ctx.close()
+    return r
+"""
+
+
+def test_moe_pair_workgroups(child):
+    """the pair form's second launch: whole rounds of at most one workgroup per CU while 128 rows a workgroup allow it"""
+    r = child(MOE + r"""
+bad = []
+for n in (1024, 1280, 2048):
+    for N in range(1, 17):
+        gu, down = layer((E.Q4_K, E.Q4_K, E.Q4_K), n, 512, 128, 4, N)
+        rows = -(-n // down[0])
+        if down[1] != N or down[0] * N > 256 or rows > 128: bad.append([n, N, down])
+print(json.dumps(bad))
 """)
     assert r == []
