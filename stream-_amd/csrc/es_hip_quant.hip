@@ -2783,16 +2783,30 @@ namespace {
 
 // The pair form of a layer (es_hip_mv.hip): the products of R choices, each on its own, without grouping and job tables. It
 // saves about 15 us of launches and reads an expert chosen c times c times (the repeats at about 10 TB/s, from the L2 and the
-// Infinity Cache), so it is taken while the repeats of a random routing stay under 128 MB. Measured per layer (us, grouped /
-// pairs): 128 experts of 3.06 MB, top 8: 1 token 33.9 / 23.7, 4 46.8 / 35.3, 8 63.2 / 49.9, 16 (141 MB) 86.5 / 76.3, 32 (440
-// MB) 110 / 130; 64 of 2.06 MB (Q2_K), top 8: 28.0 / 19.7, 44.8 / 31.3, 58.4 / 44.0 (at 16 its grouped form runs on the
-// expert-sized kernel); 16 of 1.8 MB, top 4: 25.3 / 16.3, 31.3 / 20.0, 36.1 / 23.9, 43.8 / 32.9.
+// Infinity Cache), so it is taken while the repeats of a random routing stay under 128 MB (with cheap down projections it
+// would still be ahead up to some 200). Measured per layer (us, grouped / pairs): 128 experts of 3.06 MB, top 8: 1 token 30.8
+// / 22.0, 4 44.9 / 34.2, 8 64.1 / 49.7, 12 76.1 / 64.9, 16 (139 MB) 84.7 / 75.5, 20 (206 MB) 94.6 / 99.6, 32 (441 MB) 107.3 /
+// 130.1; 64 of 2.06 MB (Q2_K), top 8: 1 27.5 / 19.7, 4 40.9 / 28.9, 8 56.7 / 42.7 (from 12 its grouped form runs on the
+// expert-sized kernel); 16 of 3.5 MB, top 4: 1 25.5 / 17.0, 4 33.4 / 22.4, 8 38.2 / 29.5, 12 (115 MB) 45.1 / 37.1.
+// Few choices per token meet that limit at many tokens, where the second launch binds instead: a choice is one wave's work,
+// so each of its row blocks costs a CU the time of one wave, 7 of 8 idle at one choice. It is taken up to 1000 blocks per CU
+// with a Q2_K or Q4_K down projection, whose blocks are cheap, else 400 (60 experts, top 2, n 1792, ff 768, Q6_K down, 20
+// tokens: 420 blocks 46.0 / 49.0; 64, top 2, n 1792, ff 256, 75: 525 49.7 / 62.4; 128 experts, top 1, n 1536, ff 1024, 21 and
+// 53 tokens: 504 38.5 / 41.9, 1272 63.4 / 95.8; 60 experts, top 4, n 2048, ff 1024, 16 tokens: 512 62.7 / 64.2; 12: 384 57.0
+// / 54.8; Q4_K down, 128 experts, top 2, n 2048, ff 512, 32 and 80 tokens: 512 46.9 / 37.4, 1280 64.6 / 74.5), and beyond it
+// where the grouped form is at its worst: 32-element gates (8 experts, top 1, n 2048, ff 512, Q4_0, 58 tokens: 928, half the
+// time) and means of more than 5 tokens per expert, which its decode kernel takes in passes of 4 (8 experts, top 1, n 1280,
+// ff 512, 46 tokens: 55.2 / 37.2).
 bool moe_pairs_ok(const es_hip_moe_ctx *c, int N, size_t expert_bytes) {
     const int R = N * c->k;
     if (!c->h_q8k || c->k > esq::MOE_PAIR_K || R > 256) return false;
     double unused = c->n_exp;
     for (int t = 0; t < N; t++) unused *= 1.0 - (double)c->k / c->n_exp;
-    return (R - (c->n_exp - unused)) * (double)expert_bytes <= 128e6;
+    if ((R - (c->n_exp - unused)) * (double)expert_bytes > 128e6) return false;
+    const double blocks = (double)c->n * (c->ff / 256) * N * ((c->k + 7) / 8) / device().cus;   // (8 waves take a choice each)
+    FmtInfo fg;
+    fmt_info(c->gt, fg);
+    return blocks <= (c->dt == ES_HIP_Q2_K || c->dt == ES_HIP_Q4_K ? 1000 : 400) || fg.be == 32 || R > 5 * c->n_exp;
 }
 
 // one layer from a routing in device memory, in stream order

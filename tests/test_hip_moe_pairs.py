@@ -41,7 +41,7 @@ def routing(rng, N, n_exp, k):
 
 @pytest.mark.parametrize("types", [(O.Q4_K, O.Q4_K, O.Q6_K), (O.Q2_K, O.Q2_K, O.Q2_K), (O.Q5_K, O.Q5_K, O.Q3_K),
                                    (O.Q6_K, O.Q6_K, O.Q5_K), (O.Q4_0, O.Q4_0, O.Q4_K)], ids=lambda t: "-".join(map(str, t)))
-@pytest.mark.parametrize("N,k,ff", [(1, 8, 768), (3, 1, 256), (2, 16, 512), (18, 2, 1024)])
+@pytest.mark.parametrize("N,k,ff", [(1, 8, 768), (3, 1, 256), (2, 16, 512), (18, 2, 1024), (29, 4, 256)])
 def test_pairs(hipo, orc, types, N, k, ff):
     n = 352 if types[0] == O.Q4_0 else 512
     rng = np.random.default_rng(N * 100 + k)

@@ -241,3 +241,24 @@ for n in (1024, 1280, 2048):
 print(json.dumps(bad))
 """)
     assert r == []
+
+
+MOE_PAIRS = [   # measured layers faster as pairs: gate/up and down type, n, ff, experts, choices, tokens
+    ("Q4_K", "Q6_K", 2048, 768, 128, 8, 1), ("Q4_K", "Q6_K", 2048, 768, 128, 8, 12), ("Q4_K", "Q4_K", 2048, 512, 128, 2, 32),
+    ("Q4_K", "Q4_K", 2048, 256, 16, 1, 91), ("Q5_K", "Q6_K", 1536, 1024, 128, 1, 12), ("Q4_K", "Q6_K", 1280, 512, 8, 1, 46),
+    ("Q4_0", "Q4_K", 2048, 512, 8, 1, 58), ("Q8_0", "Q6_K", 2048, 256, 16, 1, 60), ("Q4_K", "Q6_K", 2048, 1024, 60, 4, 12)]
+MOE_GROUPED = [   # ... and faster grouped
+    ("Q4_K", "Q6_K", 2048, 768, 128, 8, 20), ("Q5_K", "Q6_K", 1536, 1024, 128, 1, 21), ("Q5_K", "Q6_K", 1536, 1024, 128, 1, 53),
+    ("Q4_K", "Q6_K", 1792, 256, 64, 2, 75), ("Q4_K", "Q6_K", 1792, 768, 60, 2, 20), ("Q4_K", "Q6_K", 2048, 1024, 16, 1, 27), ("Q4_K", "Q4_K", 2048, 512, 128, 2, 80),
+    ("Q5_K", "Q6_K", 2048, 512, 60, 1, 75), ("Q4_K", "Q6_K", 2048, 1024, 60, 4, 16)]
+
+
+def test_moe_form(child):
+    """measured layers take the faster form (the pair form is two launches)"""
+    r = child(MOE + r"""
+def pairs(c):
+    t = [E.TYPES[c[0]], E.TYPES[c[0]], E.TYPES[c[1]]]
+    return len(layer(t, *c[2:])) == 2
+print(json.dumps([[c for c in %r if not pairs(c)], [c for c in %r if pairs(c)]]))
+""" % (MOE_PAIRS, MOE_GROUPED))
+    assert r == [[], []]
