@@ -779,45 +779,41 @@ __device__ __forceinline__ void mv_body(const MvJob &J, int order) {
     }
 }
 
-// The kernels' arguments, as one block (their first and only parameter, at offset 0 of the argument segment).
+// Launches of a few jobs: the jobs as arguments, one block (the kernel's first and only parameter, at offset 0 of the argument
+// segment), read at the grid row's offset in the round trip that brings the arguments themselves (a select among the four
+// records loaded them all: 0.6 us a launch).
 struct MvArgs {
-    const MvJob *jobs;   // the launch's job table, or null: grid row i runs j[i], tiles numbered from 0
-    int njobs, order;
-    MvJob j[MV_INLINE];
+    int order, pad;
+    MvJob j[MV_INLINE];   // grid row i runs j[i], tiles numbered from 0
 };
-// this workgroup's job. In-argument jobs are read at the grid row's offset of the argument segment, in the round trip that
-// brings the arguments themselves (a select among the four records loaded them all: 0.6 us a launch).
-__device__ __forceinline__ MvJob mv_job(const MvArgs &A) {
+__device__ __forceinline__ MvJob mv_job() {
     static_assert(sizeof(MvJob) % 4 == 0 && offsetof(MvArgs, j) % 4 == 0, "jobs are read as dwords");
     constexpr int N = sizeof(MvJob) / 4;
+    typedef const __attribute__((address_space(4))) uint32_t *ArgPtr;
+    const ArgPtr src = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(MvArgs, j) / 4 + blockIdx.y * N;
     uint32_t v[N];
-    if (A.jobs) {
-        const MvJob J = load_tile_job(A.jobs, A.njobs, blockIdx.x);
-        __builtin_memcpy(v, &J, sizeof J);
-    } else {
-        typedef const __attribute__((address_space(4))) uint32_t *ArgPtr;
-        const ArgPtr src = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(MvArgs, j) / 4 + blockIdx.y * N;
 #pragma unroll
-        for (int i = 0; i < N; i++) v[i] = src[i];
-    }
-    // scalar registers on both paths: the compiler otherwise merges the two records in vector registers (17 to 28 more of
-    // them, which cost the multi-activation bodies a wave per SIMD)
-#pragma unroll
-    for (int i = 0; i < N; i++) v[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)v[i]);
-    return __builtin_bit_cast(MvJob, v);
+    for (int i = 0; i < N; i++) v[i] = src[i];
+    return uniform_job(__builtin_bit_cast(MvJob, v));
 }
-
 template <int F, int NT, int W, bool SEGLOOP>
 __global__ __launch_bounds__(WAVE * W, ESQ_MIN_WAVES) void mv_kernel(MvArgs A) {
-    const MvJob J = mv_job(A);
+    const MvJob J = mv_job();
     mv_body<F, NT, W, SEGLOOP>(J, A.order);
+}
+// Launches of more jobs, from their table on the device. A kernel of its own: with both sources in one, whose arguments hold
+// four records, every launch took 0.5 us more (24 Q4_K products of 1024 and 2048 columns 16.1 -> 16.5 us).
+template <int F, int NT, int W, bool SEGLOOP>
+__global__ __launch_bounds__(WAVE * W, ESQ_MIN_WAVES) void mv_kernel_table(const MvJob *__restrict__ jobs, int njobs, int order) {
+    const MvJob J = load_tile_job(jobs, njobs, blockIdx.x);
+    mv_body<F, NT, W, SEGLOOP>(J, order);
 }
 
 // A launch whose jobs take different activations per pass (J.nt: 1, 2 or 4), e.g. an MoE layer's experts at 1 to 8
 // tokens each: every job runs the body compiled for its own pass width (a single expert's token no longer runs in a
 // four-wide pass with its fewer loads in flight).
 // Always from the table: its launches are long job lists, and its registers have no room for a second source of the job
-// (config 5's layer 139 -> 144 us with mv_job).
+// (config 5's layer 139 -> 144 us with one).
 template <int F, int W, bool SEGLOOP>
 __global__ __launch_bounds__(WAVE * W, ESQ_MIN_WAVES) void mv_kernel_mixed(const MvJob *__restrict__ jobs, int njobs, int order) {
     const MvJob J = load_tile_job(jobs, njobs, blockIdx.x);
@@ -956,51 +952,35 @@ __global__ __launch_bounds__(512) void moe_down_pairs(MoePairs A) {
 namespace esq {
 
 using MvFn = void (*)(MvArgs);
+using MvTableFn = void (*)(const MvJob *, int, int);
 
 // Only the (NT, W) pairs the planner uses are instantiated.
-template <int F, int NT> static MvFn pick_w(int w, bool seg_loop) {
-    switch (w) {
-    case 4: return seg_loop ? nullptr : mv_kernel<F, NT, 4, false>;
-    case 8: return seg_loop ? mv_kernel<F, NT, 8, true> : mv_kernel<F, NT, 8, false>;
+template <int F, int NT> static void pick_w(int w, bool seg_loop, MvFn &fn, MvTableFn &table) {
+    if (w == 4 && !seg_loop) {
+        fn = mv_kernel<F, NT, 4, false>;
+        table = mv_kernel_table<F, NT, 4, false>;
+    } else if (w == 8) {
+        fn = seg_loop ? mv_kernel<F, NT, 8, true> : mv_kernel<F, NT, 8, false>;
+        table = seg_loop ? mv_kernel_table<F, NT, 8, true> : mv_kernel_table<F, NT, 8, false>;
     }
-    return nullptr;
 }
-using MvMixedFn = void (*)(const MvJob *, int, int);
-template <int F> static MvMixedFn pick_mixed(int w, bool seg_loop) {   // per-job pass widths
-    if (w == 4) return seg_loop ? nullptr : mv_kernel_mixed<F, 4, false>;
-    if (w == 8) return seg_loop ? mv_kernel_mixed<F, 8, true> : mv_kernel_mixed<F, 8, false>;
-    return nullptr;
-}
-template <int F> static MvFn pick_nt(int nt, int w, bool seg_loop) {
+template <int F> static void pick_nt(int nt, int w, bool seg_loop, MvFn &fn, MvTableFn &table) {
     switch (nt) {
-    case 1: return pick_w<F, 1>(w, seg_loop);
-    case 2: return pick_w<F, 2>(w, seg_loop);
-    case 4: return pick_w<F, 4>(w, seg_loop);
+    case 0:   // per-job pass widths
+        if (w == 4 && !seg_loop) table = mv_kernel_mixed<F, 4, false>;
+        if (w == 8) table = seg_loop ? mv_kernel_mixed<F, 8, true> : mv_kernel_mixed<F, 8, false>;
+        break;
+    case 1: pick_w<F, 1>(w, seg_loop, fn, table); break;
+    case 2: pick_w<F, 2>(w, seg_loop, fn, table); break;
+    case 4: pick_w<F, 4>(w, seg_loop, fn, table); break;
     }
-    return nullptr;
 }
 
 hipError_t mv_launch(const MvLaunch &L, const MvJob *jobs, int njobs, const MvJob *hjobs, int order, hipStream_t s) {
     if (!jobs && (njobs < 1 || njobs > MV_INLINE)) return hipErrorInvalidValue;
-    MvArgs A{jobs, njobs, order, {}};
-    dim3 grid(L.grid);
-    if (!jobs) {
-        int most = 0;   // tiles of the longest job; a shorter one's workgroups past its rows have nothing to do
-        for (int i = 0; i < njobs; i++) {
-            A.j[i] = hjobs[i];
-            A.j[i].tile0 = 0;
-            const int tiles = (hjobs[i].r1 - hjobs[i].r0 + hjobs[i].rows_per_wg - 1) / hjobs[i].rows_per_wg;
-            most = tiles > most ? tiles : most;
-        }
-        grid = dim3(most, njobs);
-    }
     MvFn fn = nullptr;
-    MvMixedFn mixed = nullptr;
-    auto pick = [&](auto type) {
-        constexpr int F = decltype(type)::value;
-        if (L.nt) fn = pick_nt<F>(L.nt, L.waves, L.seg_loop);
-        else mixed = pick_mixed<F>(L.waves, L.seg_loop);
-    };
+    MvTableFn table = nullptr;
+    auto pick = [&](auto type) { pick_nt<decltype(type)::value>(L.nt, L.waves, L.seg_loop, fn, table); };
     switch (L.type) {
     case ES_HIP_Q4_0: pick(std::integral_constant<int, ES_HIP_Q4_0>{}); break;
     case ES_HIP_Q5_0: pick(std::integral_constant<int, ES_HIP_Q5_0>{}); break;
@@ -1011,17 +991,25 @@ hipError_t mv_launch(const MvLaunch &L, const MvJob *jobs, int njobs, const MvJo
     case ES_HIP_Q5_K: pick(std::integral_constant<int, ES_HIP_Q5_K>{}); break;
     case ES_HIP_Q6_K: pick(std::integral_constant<int, ES_HIP_Q6_K>{}); break;
     }
-    if ((!fn && !mixed) || (mixed && !jobs)) return hipErrorInvalidValue;
+    if (jobs ? !table : !fn) return hipErrorInvalidValue;
     if (L.lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(fn ? reinterpret_cast<const void *>(fn) : reinterpret_cast<const void *>(mixed),
+        hipError_t e = hipFuncSetAttribute(jobs ? reinterpret_cast<const void *>(table) : reinterpret_cast<const void *>(fn),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(L.lds));
         if (e != hipSuccess) return e;
     }
-    if (mixed) {
-        hipLaunchKernelGGL(mixed, grid, dim3(WAVE * L.waves), L.lds, s, jobs, njobs, order);
+    if (jobs) {
+        hipLaunchKernelGGL(table, dim3(L.grid), dim3(WAVE * L.waves), L.lds, s, jobs, njobs, order);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(fn, grid, dim3(WAVE * L.waves), L.lds, s, A);
+    MvArgs A{order, 0, {}};
+    int most = 0;   // tiles of the longest job; a shorter one's workgroups past its rows have nothing to do
+    for (int i = 0; i < njobs; i++) {
+        A.j[i] = hjobs[i];
+        A.j[i].tile0 = 0;
+        const int tiles = (hjobs[i].r1 - hjobs[i].r0 + hjobs[i].rows_per_wg - 1) / hjobs[i].rows_per_wg;
+        most = tiles > most ? tiles : most;
+    }
+    hipLaunchKernelGGL(fn, dim3(most, njobs), dim3(WAVE * L.waves), L.lds, s, A);
     return hipGetLastError();
 }
 
