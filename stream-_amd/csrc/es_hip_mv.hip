@@ -714,9 +714,14 @@ __device__ __forceinline__ void mv_body(const MvJob &J, int order) {
                         s = cmode == CH_LANES ? ldg<float>(J.lanes + lane_at) : ldg<float>(J.y + (size_t)(t0 + t) * J.ystride + ra + rl);
                 }
                 int bb = 0;
-                if constexpr (W32 && NT == 1) {   // rows of many blocks: the next eight terms' reads in flight under the chain
-                    const int full = nbk & ~7;    // (every read unconditional, the last group's repeated: a branch would wait
-                    if (full) {                   // for them all)
+                if constexpr (W32 && NT == 1) {
+                    // Rows of more than 48 blocks: the next eight terms' reads in flight under the chain (every read
+                    // unconditional, the last group's repeated: a branch would wait for them all). Shorter rows have too little
+                    // to run ahead (us, with / without: 64 Q4_0 products of 2048 x 1024 29.9 / 26.8, x 1056 36.8 / 36.3, x 1536
+                    // 39.0 / 39.1, x 3072 74.9 / 78.0; Q8_0 x 1024 32.5 / 31.0, x 3072 81.7 / 83.8; one Q4_0 x 1024 6.2 / 5.9, x
+                    // 2048 6.3 / 6.9).
+                    const int full = nbk > 48 ? nbk & ~7 : 0;
+                    if (full) {
                         float ta[8], tb[8], ua[8], ub[8];
                         auto fetch = [&](int b0, float (&fa)[8], float (&fb)[8]) {
 #pragma unroll
@@ -743,18 +748,17 @@ __device__ __forceinline__ void mv_body(const MvJob &J, int order) {
                             bb += 8;
                         }
                     }
-                } else {
-                    for (; bb + 8 <= nbk; bb += 8) {
-                        float ta[8], tb[8];
+                }
+                for (; bb + 8 <= nbk; bb += 8) {
+                    float ta[8], tb[8];
 #pragma unroll
-                        for (int q = 0; q < 8; q++) { ta[q] = e[(bb + q) * NT * CW + oa]; tb[q] = e[(bb + q) * NT * CW + ob]; }
-                        if (cmode == CH_MULADD) {
+                    for (int q = 0; q < 8; q++) { ta[q] = e[(bb + q) * NT * CW + oa]; tb[q] = e[(bb + q) * NT * CW + ob]; }
+                    if (cmode == CH_MULADD) {
 #pragma unroll
-                            for (int q = 0; q < 8; q++) s = s + ta[q] * tb[q];   // -ffp-contract=off: two roundings
-                        } else {
+                        for (int q = 0; q < 8; q++) s = s + ta[q] * tb[q];   // -ffp-contract=off: two roundings
+                    } else {
 #pragma unroll
-                            for (int q = 0; q < 8; q++) s = __builtin_fmaf(ta[q], tb[q], s);
-                        }
+                        for (int q = 0; q < 8; q++) s = __builtin_fmaf(ta[q], tb[q], s);
                     }
                 }
                 for (; bb < nbk; bb++) {
