@@ -753,6 +753,39 @@ int m6w_tiles(long groups, int na, int nbk, int cus) {
     while (wn > 1 && groups * ((na + 16 * wn - 1) / (16 * wn)) < cus) wn /= 2;
     return wn;
 }
+// Row groups (of 16) per workgroup of a launch of products of `groups` row groups and `tiles` activation tiles each: about 8
+// waves per CU for the launch, a product's chunks a multiple of 8 (workgroup g runs on XCD g % 8: 112 products of 2048 rows in
+// 5 chunks each left three XCDs idle, 115 us; in 8 chunks 69), and of the numbers up to twice that one whose rounds of
+// workgroups come to the fewest row groups: rounding up to whole chunks and whole eights leaves a last round nearly empty
+// (5 products of 6359 x 1280 at 77 activations 66.5 us, 43.8 now; 12 products of 3461 x 5632 at 11 in 288 workgroups of 10 row groups on
+// 256 CUs 172 us, in 192 of 14 135). sets: 8-chunk sets per product; returns those row groups times the workgroups side by side.
+struct M6wProd { int groups, tiles; };
+long m6w_sets(const std::vector<M6wProd> &prods, int nw, int cus, std::vector<int> *sets) {
+    long units = 0;
+    for (const M6wProd &q : prods) units += (long)q.groups * q.tiles;
+    const long slots = (long)cus * std::max(1, 8 / nw);
+    const long per0 = std::max<long>(1, (units + slots - 1) / slots);
+    long best = -1, bper = per0;
+    const long step = std::max<long>(1, per0 / 8);
+    for (long per = per0; per <= 2 * per0; per += step) {
+        long grid = 0, most = 0;
+        for (const M6wProd &q : prods) {
+            const long n = ((q.groups + per - 1) / per + 7) / 8;
+            grid += 8 * n * q.tiles;
+            most = std::max(most, (q.groups + 8 * n - 1) / (8 * n));
+        }
+        const long eff = most * ((grid + slots - 1) / slots * slots);
+        if (best < 0 || eff < best) {
+            best = eff;
+            bper = per;
+        }
+    }
+    if (sets) {
+        sets->clear();
+        for (const M6wProd &q : prods) sets->push_back((int)(((q.groups + bper - 1) / bper + 7) / 8));
+    }
+    return best;
+}
 std::atomic<int> g_m6w_on{1};
 // What that kernel can take: no gather, 32-bit offsets; of the default g_mm6_min = 16 (the automatic choice) products of 5
 // activations or more, else those of g_mm6_min.
@@ -773,21 +806,22 @@ bool m6w_capable(const Req &q) {
 // superblocks per wave; 3, 5 or 7 waves take as long as 4, 6 or 8. 8192 x 2048 at 64, 128 and 512 activations 13 / 25, 18 /
 // 28, 48 / 50; 2048 x 8192 at 64, 256 and 512 24 / 82, 75 / 84, 145 / 84; 8192 x 768 at 64, 128 and 256 8.6 / 14.2, 12.4 /
 // 14.3, 17.9 / 15.4; 8192 x 1280 at 256 23.1 / 19.9; 16 x 2048 x 768 at 16 and 64 15.0 / 13.7, 18.1 / 16.6; 32768 x 1536 at
-// 16 24.0 / 20.5; 16 x 2048 x 768 at 16 to 60 29.6 / 36.3. It errs by less than a tenth (8192 x 1024 at 256 18.5 / 17.3,
-// taken; 32768 x 2048 at 64 29.0 / 31.4, not taken). A product of one activation tile and many row tiles whose activations
-// fit the LDS keeps the tiled kernel's persistent form (151936 x 1024 at 16 and 64: 57 / 43, 61 / 58).
+// 16 24.0 / 20.5; 16 x 2048 x 768 at 16 to 60 29.6 / 36.3. Over 293 random batches, of 5 activations or more, five lost more
+// than a tenth (12 x 1138 x 6400 at 11 89 / 67, 41244 x 1792 at 16 40 / 31). A product of one activation tile and many row
+// tiles whose activations fit the LDS keeps the tiled kernel's persistent form (151936 x 1024 at 16 and 64: 57 / 43, 61 /
+// 58).
 // Fewer than 16, against the decode kernel's passes of 4, which are faster below 5 (8192 x 2048 at 4: 8.9 / 8.6). A batch
-// that fills the device anyway takes this kernel from a mean of 7 activations, of 9 with rows longer than its waves (112 x
-// 2048 x 768 at 5, 8 and 12 70 / 72, 69 / 80, 69 / 113; 16 x 2048 x 8192 111 / 89, 111 / 101, 113 / 144; at its worst 16 x
-// 8192 x 768 at 8 44.8 / 42.9). A small one takes it from 5 (2048 x 768 at 5 and 8 4.3 / 13.0, 4.3 / 15.2; 8192 x 2048 9.7 /
-// 12.8, 9.7 / 14.6; 2048 x 6144 12.8 / 14.9, 13.0 / 16.9) unless its rows are so long that their rounds, one after another,
-// outlast the decode kernel's passes: up to 14 + 2 x mean superblocks (2048 x 7168 at 5 and 7 15.8 / 15.2, 16.0 / 16.7; 2048
-// x 8192 at 5, 8 and 9 17.2 / 13.5, 17.4 / 15.3, 17.5 / 19.0), or rows enough for every CU (4096 x 8192 at 6 17.4 / 17.9).
-// Where products of fewer than 5 activations need a decode launch beside it, that costs 6 to 8 us: it must have half of the
-// weights and a mean of 9 (7 with rows of fewer superblocks than waves: 16 x 2048 x 768 at 3 to 15 25.5 / 28.9), with very
-// long rows also rows enough (8192 x 2048 at 8 and 9 with 512 x 2048 at 2 17.3 / 15.9, 17.3 / 19.3; 2048 x 4096 at 9 16.2 /
-// 17.2; 2048 x 8192 at 12 25.5 / 21.9; 4096 x 8192 at 9 25.3 / 28.6), or be short (2048 x 768 at 5 10.7 / 13.5; 2048 x 2048
-// at 5 and 8 12.1 / 11.6, 12.3 / 13.3).
+// that fills the device anyway takes this kernel from a mean of 7 activations, of 9 with rows of 5 superblocks, of 7 or more
+// (112 x 2048 x 768 at 5, 8 and 12 70 / 72, 69 / 80, 69 / 113; 12 x 4593 x 1280 at 8 50 / 41, 12 x 5809 x 1792 85 / 68, 12 x
+// 8879 x 2048 114 / 89; 12 x 5874 x 3072 at 9 129 / 141; 16 x 2048 x 8192 at 5, 8 and 12 111 / 89, 111 / 101, 113 / 144). A
+// small one takes it from 5 (2048 x 768 at 5 and 8 4.3 / 13.0, 4.3 / 15.2; 8192 x 2048 9.7 / 12.8, 9.7 / 14.6; 2048 x 6144
+// 12.8 / 14.9, 13.0 / 16.9) unless its rows are so long that their rounds, one after another, outlast the decode kernel's
+// passes: up to 14 + 2 x mean superblocks (2048 x 7168 at 5 and 7 15.8 / 15.2, 16.0 / 16.7; 2048 x 8192 at 5, 8 and 9 17.2 /
+// 13.5, 17.4 / 15.3, 17.5 / 19.0), or rows enough for every CU (4096 x 8192 at 6 17.4 / 17.9). Where products of fewer than 5
+// activations need a decode launch beside it, that costs 6 to 8 us: it must have half of the weights and a mean of 9 (7 with
+// rows of fewer superblocks than waves: 16 x 2048 x 768 at 3 to 15 25.5 / 28.9), with very long rows also rows enough (8192 x
+// 2048 at 8 and 9 with 512 x 2048 at 2 17.3 / 15.9, 17.3 / 19.3; 2048 x 4096 at 9 16.2 / 17.2; 2048 x 8192 at 12 25.5 / 21.9;
+// 4096 x 8192 at 9 25.3 / 28.6), or be short (2048 x 768 at 5 10.7 / 13.5; 2048 x 2048 at 5 and 8 12.1 / 11.6, 12.3 / 13.3).
 struct M6wChoice { bool few = false, many = false; long gfew = 0, gmany = 0; };   // groups: rows / 16 of either kind
 M6wChoice m6w_choose(const std::vector<Req> &reqs, int cus) {
     M6wChoice c;
@@ -812,12 +846,17 @@ M6wChoice m6w_choose(const std::vector<Req> &reqs, int cus) {
         }
     }
     double cost = 5.0;
+    std::map<std::pair<int, int>, std::vector<M6wProd>> launches;   // by superblocks per row and activation tiles
     for (const Req &q : reqs)
         if (q.na >= 16 && m6w_capable(q)) {
             const int nbk = q.cols / 256, wn = m6w_tiles(c.gmany, q.na, nbk, cus);
-            cost += (double)((q.r1 - q.r0 + 15) / 16) * ((q.na + 16 * wn - 1) / (16 * wn)) *
-                    (nbk > esq::M6W_WAVES ? 2.3e-3 * nbk : nbk > 1 ? 1.4e-3 * ((nbk + 1) & ~1) : 1.4e-3);
+            launches[{nbk, wn}].push_back({(q.r1 - q.r0 + 15) / 16, (q.na + 16 * wn - 1) / (16 * wn)});
         }
+    for (const auto &l : launches) {
+        const int nbk = l.first.first;
+        cost += m6w_sets(l.second, m6w_waves(nbk), cus, nullptr) *
+                (nbk > esq::M6W_WAVES ? 2.3e-3 * nbk : nbk > 1 ? 1.4e-3 * ((nbk + 1) & ~1) : 1.4e-3);
+    }
     double tiled = 6.0;
     for (int w = 0; w < 3; w++) tiled += (2.0 + (w ? 2.4 : 1.9) * nbk_max[w]) * ((tiles[w] + cus - 1) / cus);
     c.many = cost < tiled;
@@ -827,7 +866,7 @@ M6wChoice m6w_choose(const std::vector<Req> &reqs, int cus) {
         c.few = sfew >= rest && (afew >= (nbk_few < 8 ? 7 : 9) * sfew ? nbk_few <= 24 || rows : shortr);
     } else {
         const bool small = sfew <= (longr ? 131072 : 262144) && (rows || (nbk_few - 14) * sfew <= 2 * afew);
-        c.few = sfew > 0 && (small || afew >= (longr ? 9 : 7) * sfew);
+        c.few = sfew > 0 && (small || afew >= (longr || nbk_few == 5 || nbk_few > 6 ? 9 : 7) * sfew);
     }
     return c;
 }
@@ -837,19 +876,18 @@ bool m6w_eligible(const Req &q, const M6wChoice &c) {
     const int nbk = q.cols / 256, rt = (q.r1 - q.r0 + 127) / 128, bn = q.na <= 16 ? 16 : q.na <= 32 ? 32 : 64;
     return c.many && !(q.na <= 64 && rt >= 2 * device().cus && nbk <= esq::mm6_persistent_blocks(bn));
 }
-// Row groups per workgroup and the tile numbering: about 8 waves per CU for the launch, a product's chunks a multiple of 8
-// (workgroup g runs on XCD g % 8: 112 products of 2048 rows in 5 chunks each left three XCDs idle, 115 us; in 8 chunks 69).
+// the row groups per workgroup and the tile numbering
 void m6w_tiling(MkGroup &g, int cus) {
-    long units = 0;
-    for (const esq::MkJob &j : g.jobs) units += (long)((j.r1 - j.r0 + 15) / 16) * j.ntok_tiles;
-    const long slots = (long)cus * std::max(1, 8 / g.m6_nw);
-    const int per = (int)std::max<long>(1, (units + slots - 1) / slots);
+    std::vector<M6wProd> prods;
+    std::vector<int> sets;
+    for (const esq::MkJob &j : g.jobs) prods.push_back({(j.r1 - j.r0 + 15) / 16, j.ntok_tiles});
+    m6w_sets(prods, g.m6_nw, cus, &sets);
     g.grid = 0;
-    for (esq::MkJob &j : g.jobs) {
-        const int ngroup = (j.r1 - j.r0 + 15) / 16, sets = ((ngroup + per - 1) / per + 7) / 8;
-        j.rows_per_wg = (ngroup + 8 * sets - 1) / (8 * sets);
+    for (size_t i = 0; i < g.jobs.size(); i++) {
+        esq::MkJob &j = g.jobs[i];
+        j.rows_per_wg = (prods[i].groups + 8 * sets[i] - 1) / (8 * sets[i]);
         j.tile0 = g.grid;
-        g.grid += 8 * sets * j.ntok_tiles;
+        g.grid += 8 * sets[i] * j.ntok_tiles;
     }
 }
 

@@ -174,11 +174,11 @@ Q6K_WAVES = [   # batches faster on the kernel with one wave per superblock: (ro
     [(2048, 3, 5)], [(8192, 8, 5)], [(2048, 24, 5)], [(2048, 28, 7)], [(2048, 32, 9)], [(4096, 32, 6)], [(2048, 3, 8)] * 112, [(8192, 3, 64)],
     [(8192, 3, 128)], [(8192, 8, 128)], [(2048, 32, 64)], [(2048, 32, 256)], [(512, 3, 256)] * 16, [(2048, 3, 5), (512, 8, 2)],
     [(2048, 8, 8), (512, 8, 2)], [(2048, 16, 9), (512, 8, 2)], [(4096, 32, 9), (512, 8, 2)], [(32768, 1, 512)], [(32768, 2, 512)],
-    [(2048, 3, n) for n in (17, 25, 33, 41, 50, 60)]]
+    [(2048, 3, n) for n in (17, 25, 33, 41, 50, 60)], [(24158, 12, 9)], [(24050, 12, 9)] * 3, [(52000, 4, 8)] * 3, [(5004, 8, 9)] * 12]
 Q6K_OTHERS = [   # ... and faster on the decode or the tiled kernel
     [(512, 28, 5)], [(512, 32, 5)], [(2048, 32, 8)], [(512, 32, 8)] * 4, [(2048, 48, 6)], [(8192, 32, 5)], [(8192, 3, 256)], [(8192, 5, 256)],
     [(32768, 3, 16)], [(32768, 6, 16)], [(2048, 3, 16)] * 64, [(2048, 3, 64)] * 16, [(2048, 8, 5), (512, 8, 2)], [(8192, 8, 8), (512, 8, 2)],
-    [(2048, 32, 12), (512, 8, 2)], [(8192, 8, 4)], [(2048, 32, 512)]]
+    [(2048, 32, 12), (512, 8, 2)], [(8192, 8, 4)], [(2048, 32, 512)], [(159288, 5, 8)], [(4593, 5, 8)] * 12, [(5809, 7, 8)] * 12, [(8879, 8, 8)] * 12, [(711, 9, 33)] * 12]
 
 
 def test_q6k_kernel_choice(child):
@@ -198,6 +198,23 @@ def waves(batch): return launches(batch, 1) != launches(batch, 0)
 print(json.dumps([[b for b in %r if not waves(b)], [b for b in %r if waves(b)]]))
 """ % (Q6K_WAVES, Q6K_OTHERS))
     assert r == [[], []]
+
+
+def test_q6k_whole_rounds(child):
+    """that kernel's workgroups come in whole rounds of the CUs (256) where its waves fill one with a single workgroup: ragged
+    batches whose last round was nearly empty"""
+    r = child(r"""
+shapes = ((C.c_long * 4) * 64).in_dll(S, "shapes")
+out = []
+for n, rows, nbk, na in ((12, 3461, 22, 11), (5, 6359, 5, 77), (2, 10291, 8, 64), (3, 648, 9, 100)):
+    p = L.plan([job(E.Q6_K, rows, 256 * nbk, na, k) for k in range(n)])
+    reset()
+    p.run()
+    if counts[0] != 1 or shapes[0][0] > 256: out.append([n, rows, nbk, na, counts[0], list(shapes[0])])
+    p.close()
+print(json.dumps(out))
+""")
+    assert r == []
 
 
 def test_q6k_pairs_travel_with_their_launch(child):
