@@ -299,8 +299,8 @@ int es_hip_set_direct_mfma_min_batch(int n);
 /* The direct-activation kernel's minimum tile count per product (default 128; twice that for rows longer than 4096):
  * below it a product has too few workgroups to fill the device. Returns the previous value. */
 int es_hip_set_direct_mfma_min_tiles(int n);
-/* Q5_K products with at least n activations (default 8) run on the direct-activation matrix-core kernel; below it, or with it off (n <= 0), on the vector kernel. Results are identical on both. Returns
- * the previous value. */
+/* Q5_K products with at least n activations (default 8) run on the direct-activation matrix-core kernel; below it, or with
+ * it off (n <= 0), on the vector kernel. Results are identical on both. Returns the previous value. */
 int es_hip_set_q5k_mfma_min_batch(int n);
 /* Q3_K products with at least n activations (default 8) run on the direct-activation matrix-core kernel (two int8 planes of
  * the signed codes against the split scales); below it, or with it off (n <= 0), on the vector kernel. Results are

@@ -153,7 +153,8 @@ hipError_t mbx_launch(int type, bool gather, int nbk_max, const MkJob *jobs, int
 // without it nw >= wn.
 // jobs: the launch's job table on the device, or null: the njobs <= M6W_INLINE jobs at hjobs travel with the launch.
 constexpr int M6W_WAVES = 8, M6W_INLINE = 4;
-hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob *hjobs, int grid, int order, hipStream_t s);
+hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob *hjobs, int grid, int order,
+                      hipStream_t s);
 // gather: some job of the launch reads its activation rows through arow (a separate kernel build; the others need not);
 // tok: activations per workgroup tile, MK_TOK or 64 (ntok_tiles and the tile numbering then count tiles of 64)
 hipError_t mk_launch(int type, bool gather, int tok, const MkJob *jobs, int njobs, const MkJob &single, int grid, int order,
@@ -307,7 +308,7 @@ hipError_t moe_pairs_gu_launch(const MoePairs &a, const MvLaunch &L, int pairs, 
 size_t moe_pairs_down_lds(int k, int ff, int rt);
 hipError_t moe_pairs_down_launch(int type, const MoePairs &a, int ntok, hipStream_t s);
 
-constexpr int ACT_RMS_MAX_COLS = 16384;   // rmsnorm rows' squares are staged whole in LDS (128 KB of doubles)
+constexpr int ACT_RMS_MAX_COLS = 16384;   // rmsnorm rows lie in a workgroup's registers, 8192 values a pass, in at most two passes
 // Activation preparation (es_hip_act.hip): rows of fp32 values (plain, rmsnorm-ed, or the SwiGLU of gate|up rows) into
 // Q8_0 and / or Q8_K blocks (either output may be null). Float strides in floats, block strides in bytes.
 hipError_t act_prep_launch(const float *x, uint64_t xs, int rows, int cols, uint8_t *q80, uint64_t q80s, uint8_t *q8k,

@@ -7,13 +7,14 @@
 // these rows. Only the last line above is sequential: every wave forms its superblock's integers for the whole tile and
 // leaves them in LDS as floats, and after one barrier each (4 rows, activation) has a thread that runs the reference's chain
 // over the superblocks at hand (rows of 1 to 3 superblocks have fewer threads than chains at 32 or 64 activations and run them
-// in turns: 8192 x 768 at 64 activations 8.6 us against 9.6 with narrower tiles, which unpack every superblock twice). A product of few rows and many superblocks (a 2048 x 8192 down projection: 16 workgroups of
-// 128 rows running 32 superblocks one after another, 94.9 us at 64 activations) so has its superblocks in flight on
-// different waves; with at most as many superblocks as waves a wave keeps its activation operands in registers over all
-// row groups of its workgroup, and no operand passes through LDS. Measured (tiled kernel before -> this one): 2048 x 8192 at
-// 64 activations 94.9 us and 5 us of pre-pass -> 24 us, 8192 x 2048 29.5 -> 12.8 us. Bound by the scattered weight loads (16
-// rows x 64 bytes an instruction, every other superblock 2 bytes off a dword) and the vector work of the unpacking: at 16
-// activations it streams 2.3 TB/s of the head's weights, and a second item of weights in flight changed nothing.
+// in turns: 8192 x 768 at 64 activations 8.6 us against 9.6 with narrower tiles, which unpack every superblock twice). A
+// product of few rows and many superblocks (a 2048 x 8192 down projection: 16 workgroups of 128 rows running 32 superblocks
+// one after another, 94.9 us at 64 activations) so has its superblocks in flight on different waves; with at most as many
+// superblocks as waves a wave keeps its activation operands in registers over all row groups of its workgroup, and no operand
+// passes through LDS. Measured (tiled kernel before -> this one): 2048 x 8192 at 64 activations 94.9 us and 5 us of pre-pass
+// -> 24 us, 8192 x 2048 29.5 -> 12.8 us. Bound by the address unit: 16 rows x 64 bytes a load instruction, every other
+// superblock 2 bytes off a dword. On 2048 x 8192 at 64 it is busy for 85% of the launch, the vector units for 25% of it; at 16
+// activations the kernel streams 2.3 TB/s of the head's weights, and a second item of weights in flight changed nothing.
 //
 // Integers: q_u * sc lies in -8064..8001 and is split into two signed bytes, q_u * sc = 256 hi + lo, so two int8 planes
 // carry it exactly: sum q_u * sc * x = 256 D(hi) + D(lo). -32 corr goes through one f16 MFMA (-32 sc and the bsums are
@@ -219,7 +220,8 @@ hipError_t launch(int nw, bool keep, const M6wArgs &A, dim3 grid, int order, hip
 
 }  // namespace
 
-hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob *hjobs, int grid, int order, hipStream_t s) {
+hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, const MkJob *hjobs, int grid, int order,
+                      hipStream_t s) {
     // over several rounds every chain needs a thread of its own
     if (nw < 1 || nw > M6W_WAVES || (!keep && nw < wn) || njobs < 1 || (!jobs && njobs > M6W_INLINE)) return hipErrorInvalidValue;
     M6wArgs A{jobs, njobs, 0, {}};

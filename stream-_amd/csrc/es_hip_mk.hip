@@ -41,8 +41,9 @@
 //
 // Q5_K (src/es_quant.c:1153-1175): Q4_K's layout plus qh[32] after the scales, bit 2c (2c + 1) of qh[l] the fifth bit of
 // element l of sub-block 2c (2c + 1). q * sc (<= 1953) goes through the matrix cores as two int8 planes,
-// q * sc = 256 hi + lo, so dot = 256 D_hi + D_lo, exact (three planes before, 13 MFMAs a tile instead of 9). Its epilogue is the reference's scalar mv_q5_K (the x86 build has no AVX2
-// Q5_K kernel and no FMA in it): s += y.d * (d * dot - dmin * mins) with every product and sum rounded, in every order.
+// q * sc = 256 hi + lo, so dot = 256 D_hi + D_lo, exact (9 MFMAs a tile; in three planes, as before, 13). Its epilogue is the
+// reference's scalar mv_q5_K (the x86 build has no AVX2 Q5_K kernel and no FMA in it): s += y.d * (d * dot - dmin * mins) with
+// every product and sum rounded, in every order.
 //
 // Q3_K (src/es_quant.c:1120-1150, 1369-1395): 110-byte superblocks hmask[32] | qs[64] | scales[12] | d, 2-byte aligned,
 // read with unaligned 16-byte loads (the header as bytes 94..109: qs[62..63], the scales and d, so no load passes the

@@ -165,7 +165,6 @@ __global__ __launch_bounds__(64 * RW * TW) void mm_q6k_kernel(const MmJob *__res
     const uint32_t mo = G::M_OFF + (wt + lr) * 32 + 16 * (lg & 1), dof = G::D_OFF + (wt + lr) * 4;
     const int qo = lg >> 1, lh = lg & 1;
     const uint32_t rowoff = (wr + lr) * 208, ddoff = G::D_W + (wr + 4 * lg) * 2;
-    const uint32_t sel = 0x0c000c00u + (uint32_t)lg * 0x00010001u;   // byte lg of a word into both 16-bit halves
 
     float s[WN][4];
 #pragma unroll

@@ -512,8 +512,9 @@ double pk_cost(int nbk, bool t64) { return nbk * (t64 ? 0.6 : 1.0) + 1.0; }
 // while every CU gets at most one of those, and from four per CU; in between the two-workgroup form packs better (8192 x
 // 2048 twice, us, two-workgroup / 64 / 128 wide: T = 64 13.6 / 12.6 / 16.7, 128 19.6 / 20.7 / 18.0, 256 30.7 / 36.8 / 31.4;
 // 2048 x 8192: T = 64 36.3 / 31.2 / 41.3, 512 37.7 / 34.2 / 42.9, 1024 58.0 / 64.2 / 53.0; 4096 x 4096: T = 256 21.9 / 19.7 /
-// 25.0, 512 31.3 / 34.4 / 28.1). Q5_K has no two-workgroup form: against its per-tile launches (three planes, before) 8192
-// x 2048 twice T = 8 19.3 -> 13.2, 512 67.3 -> 61.7; 2048 x 8192 T = 333 45.7 -> 41.8.
+// 25.0, 512 31.3 / 34.4 / 28.1). Q5_K has no two-workgroup form: its per-tile launches take (us, per tile / this) 8192 x 2048
+// twice T = 8 18.7 / 14.0, 512 59.2 / 58.4; 2048 x 8192 T = 8 59.5 / 39.5, 333 45.5 / 40.6; the shortest lose a little (1024 x
+// 1024 twice T = 64 8.4 / 8.7).
 bool pk_ws(PkGroup &g, int cus) {
     const int on = g_pk_on.load();
     if (g.type == ES_HIP_Q3_K || on == 3) return false;
@@ -757,8 +758,8 @@ int m6w_tiles(long groups, int na, int nbk, int cus) {
 // waves per CU for the launch, a product's chunks a multiple of 8 (workgroup g runs on XCD g % 8: 112 products of 2048 rows in
 // 5 chunks each left three XCDs idle, 115 us; in 8 chunks 69), and of the numbers up to twice that one whose rounds of
 // workgroups come to the fewest row groups: rounding up to whole chunks and whole eights leaves a last round nearly empty
-// (5 products of 6359 x 1280 at 77 activations 66.5 us, 43.8 now; 12 products of 3461 x 5632 at 11 in 288 workgroups of 10 row groups on
-// 256 CUs 172 us, in 192 of 14 135). sets: 8-chunk sets per product; returns those row groups times the workgroups side by side.
+// (5 products of 6359 x 1280 at 77 activations 66.5 us, 43.8 now; 12 products of 3461 x 5632 at 11 in 288 workgroups of 10 row
+// groups on 256 CUs 172 us, in 192 of 14 135). sets: 8-chunk sets per product; returns those row groups times the workgroups side by side.
 struct M6wProd { int groups, tiles; };
 long m6w_sets(const std::vector<M6wProd> &prods, int nw, int cus, std::vector<int> *sets) {
     long units = 0;
@@ -1757,9 +1758,10 @@ int es_hip_synchronize(void) {
 }
 
 // ---- products on device memory ----------------------------------------------------------------------------------------
-// Plan and launch a batch in stream order: decode launches of a few jobs and other launches of one by value (with a
-// stream-ordered allocation for their pre-pass workspace, if any); anything else (long job lists) with a stream-ordered allocation for the job tables and the pre-pass workspace, freed in stream order. The
-// tables are copied from pageable memory, which the copy has consumed when it returns.
+// Plan and launch a batch in stream order: decode and one-wave-a-superblock Q6_K launches of a few jobs and other launches of
+// one by value (with a stream-ordered allocation for their pre-pass workspace, if any); anything else (long job lists) with a
+// stream-ordered allocation for the job tables and the pre-pass workspace, freed in stream order. The tables are copied from
+// pageable memory, which the copy has consumed when it returns.
 static int run_async(const std::vector<Req> &reqs, hipStream_t s, int order = -1) {
     if (has_long(reqs))
         return run_in_pieces(reqs, s, order >= 0 ? order : g_order.load(),
