@@ -74,20 +74,15 @@ __device__ __forceinline__ void load_b6(const uint8_t *blk, int lg, B6 &b) {   /
     b.d = ldg<float>(blk);
 }
 
-// The kernel's arguments, as one block (its first and only parameter, at offset 0 of the argument segment).
-struct M6wArgs {
-    const MkJob *jobs;   // the launch's job table, or null: grid row i runs j[i], tiles numbered from 0
-    int njobs, pad;
-    MkJob j[M6W_INLINE];
-};
-// this workgroup's job; an in-argument one is read at the grid row's offset of the argument segment, in the round trip that
-// brings the arguments themselves (found by its tile numbers it came a round trip later, 0.1 us a launch)
-__device__ __forceinline__ MkJob m6w_job(const M6wArgs &A) {
-    static_assert(sizeof(MkJob) % 4 == 0 && offsetof(M6wArgs, j) % 4 == 0, "jobs are read as dwords");
+// Launches of a few jobs: the jobs as arguments, one block (the kernel's first and only parameter, at offset 0 of the argument
+// segment). A job is read at the grid row's offset of the segment, in the round trip that brings the arguments themselves (found
+// by its tile numbers it came a round trip later, 0.1 us a launch).
+struct M6wArgs { MkJob j[M6W_INLINE]; };   // grid row i runs j[i], tiles numbered from 0
+__device__ __forceinline__ MkJob m6w_job() {
+    static_assert(sizeof(MkJob) % 4 == 0 && offsetof(M6wArgs, j) == 0, "jobs are read as dwords");
     constexpr int N = sizeof(MkJob) / 4;
-    if (A.jobs) return uniform_job(load_tile_job(A.jobs, A.njobs, blockIdx.x));
     typedef const __attribute__((address_space(4))) uint32_t *ArgPtr;
-    const ArgPtr src = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(M6wArgs, j) / 4 + blockIdx.y * N;
+    const ArgPtr src = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr() + blockIdx.y * N;
     uint32_t v[N];
 #pragma unroll
     for (int i = 0; i < N; i++) v[i] = src[i];
@@ -96,9 +91,8 @@ __device__ __forceinline__ MkJob m6w_job(const M6wArgs &A) {
 
 // KEEP: at most as many superblocks as waves (one round per row group, activation operands loaded once).
 template <int WN, bool CONTRACT, bool KEEP>
-__global__ __launch_bounds__(512) void m6w_kernel(M6wArgs A) {
+__device__ __forceinline__ void m6w_body(const MkJob &J) {
     extern __shared__ __align__(16) float lds6[];   // two buffers of [wave][16 WN activations][16 rows] tot | d | y.d
-    const MkJob J = m6w_job(A);
     // all activation tiles of a row chunk on one XCD (workgroup g runs on XCD g % 8; a grid row is a multiple of 8)
     const int tile = blockIdx.x - J.tile0, kq = tile >> 3;
     const int chunk = (tile & 7) + 8 * (kq / J.ntok_tiles), tok0 = (kq % J.ntok_tiles) * 16 * WN;
@@ -203,18 +197,36 @@ __global__ __launch_bounds__(512) void m6w_kernel(M6wArgs A) {
     }
 }
 
+template <int WN, bool CONTRACT, bool KEEP>
+__global__ __launch_bounds__(512) void m6w_kernel(M6wArgs) {
+    const MkJob J = m6w_job();
+    m6w_body<WN, CONTRACT, KEEP>(J);
+}
+// Launches of more jobs, from their table on the device. A kernel of its own: with both sources in one every launch took 0.1 to
+// 0.5 us more (2048 x 768 at 8 activations 3.71 -> 3.93 us, 2048 x 8192 at 64 22.1 -> 22.4, 64 x 2048 x 768 at 12 45.2 -> 45.7).
+template <int WN, bool CONTRACT, bool KEEP>
+__global__ __launch_bounds__(512) void m6w_kernel_table(const MkJob *__restrict__ jobs, int njobs) {
+    const MkJob J = uniform_job(load_tile_job(jobs, njobs, blockIdx.x));
+    m6w_body<WN, CONTRACT, KEEP>(J);
+}
+
 template <int WN>
-hipError_t launch(int nw, bool keep, const M6wArgs &A, dim3 grid, int order, hipStream_t s) {
+hipError_t launch(int nw, bool keep, const MkJob *jobs, int njobs, const M6wArgs &A, dim3 grid, int order, hipStream_t s) {
     const bool contract = order == ES_HIP_ORDER_X86_CONTRACT;
     const auto kern = contract ? (keep ? m6w_kernel<WN, true, true> : m6w_kernel<WN, true, false>)
                                : (keep ? m6w_kernel<WN, false, true> : m6w_kernel<WN, false, false>);
+    const auto table = contract ? (keep ? m6w_kernel_table<WN, true, true> : m6w_kernel_table<WN, true, false>)
+                                : (keep ? m6w_kernel_table<WN, false, true> : m6w_kernel_table<WN, false, false>);
     const size_t lds = (size_t)2 * nw * (WN * 256 + 16 + 16 * WN) * sizeof(float);   // at most 70 KB
     if (lds > 60 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           static_cast<int>(lds));
+        hipError_t e = hipFuncSetAttribute(jobs ? reinterpret_cast<const void *>(table) : reinterpret_cast<const void *>(kern),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, A);
+    if (jobs)
+        hipLaunchKernelGGL(table, grid, dim3(64 * nw), lds, s, jobs, njobs);
+    else
+        hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, A);
     return hipGetLastError();
 }
 
@@ -224,7 +236,7 @@ hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, c
                       hipStream_t s) {
     // over several rounds every chain needs a thread of its own
     if (nw < 1 || nw > M6W_WAVES || (!keep && nw < wn) || njobs < 1 || (!jobs && njobs > M6W_INLINE)) return hipErrorInvalidValue;
-    M6wArgs A{jobs, njobs, 0, {}};
+    M6wArgs A{};
     dim3 g(grid);
     if (!jobs) {
         int most = 0;   // workgroups of the longest job; a shorter one's past its rows have nothing to do
@@ -236,9 +248,9 @@ hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, c
         g = dim3(most, njobs);
     }
     switch (wn) {
-    case 1: return launch<1>(nw, keep, A, g, order, s);
-    case 2: return launch<2>(nw, keep, A, g, order, s);
-    case 4: return launch<4>(nw, keep, A, g, order, s);
+    case 1: return launch<1>(nw, keep, jobs, njobs, A, g, order, s);
+    case 2: return launch<2>(nw, keep, jobs, njobs, A, g, order, s);
+    case 4: return launch<4>(nw, keep, jobs, njobs, A, g, order, s);
     }
     return hipErrorInvalidValue;
 }
