@@ -13,7 +13,7 @@
 // superblocks as waves a wave keeps its activation operands in registers over all row groups of its workgroup, and no operand
 // passes through LDS. Measured (tiled kernel before -> this one): 2048 x 8192 at 64 activations 94.9 us and 5 us of pre-pass
 // -> 24 us, 8192 x 2048 29.5 -> 12.8 us. Bound by the address unit: 16 rows x 64 bytes a load instruction, every other
-// superblock 2 bytes off a dword. On 2048 x 8192 at 64 it is busy for 85% of the launch, the vector units for 25% of it; at 16
+// superblock 2 bytes off a dword. On 2048 x 8192 at 64 it is busy for 88% of the launch, the vector units for 26% of it; at 16
 // activations the kernel streams 2.3 TB/s of the head's weights, and a second item of weights in flight changed nothing.
 //
 // Integers: q_u * sc lies in -8064..8001 and is split into two signed bytes, q_u * sc = 256 hi + lo, so two int8 planes
