@@ -84,7 +84,9 @@ def test_several_products_in_a_launch(hip, orc):
     [(1024, 3, 33 + 5 * j) for j in range(8)],                        # four tiles of activations, three waves
     [(300, 4, 8), (33, 4, 8), (2500, 4, 7), (16, 4, 5)],              # jobs of unequal length as kernel arguments
     [(300, 4, 8), (33, 4, 8), (2500, 4, 7), (16, 4, 5), (50, 4, 8)],  # ... and one more than fit
-], ids=["chunks", "tiles", "beside", "left", "long6", "long9", "mixed", "threes", "four", "five"])
+    [(2100, 8, 6), (512, 8, 6), (500, 8, 6)],                         # a long job over several rows of the grid
+    [(2700, 4, 70), (64, 4, 70), (40, 4, 64), (1300, 4, 33)],         # ... with several tiles of activations
+], ids=["chunks", "tiles", "beside", "left", "long6", "long9", "mixed", "threes", "four", "five", "rows", "rowtiles"])
 def test_batches(hip, orc, shapes):
     specs, want, outs, keep = [], [], [], []
     for j, (rows, nbk, na) in enumerate(shapes):

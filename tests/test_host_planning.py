@@ -233,6 +233,24 @@ print(json.dumps(out))
     assert r == []
 
 
+def test_q6k_grid_rows(child):
+    """jobs of unequal length as kernel arguments: at most a quarter of the launch's workgroups without a tile"""
+    r = child(r"""
+shapes = ((C.c_long * 4) * 64).in_dll(S, "shapes")
+out = []
+for rows, nbk, na in (((2048, 512, 512), 8, 6), ((4096, 1024, 1024), 8, 8), ((2048, 256), 8, 8), ((300, 33, 2500, 16), 4, 8), ((3584, 3584), 8, 6)):
+    p = L.plan([job(E.Q6_K, r, 256 * nbk, na, k) for k, r in enumerate(rows)])
+    reset()
+    p.run()
+    least = sum((r + 15) // 16 for r in rows)   # row groups; the largest batch here takes two a workgroup
+    x, y = shapes[0][0], shapes[0][1]
+    if counts[0] != 1 or x % 8 or y > 8 or x * y > 1.25 * least + 8 * len(rows) or 2 * x * y < least: out.append([rows, nbk, na, counts[0], list(shapes[0])])
+    p.close()
+print(json.dumps(out))
+""")
+    assert r == []
+
+
 MOE = r"""
 shapes = ((C.c_long * 4) * 64).in_dll(S, "shapes")
 def layer(types, n, ff, ne, k, N):   # the launches of a layer of N tokens
