@@ -77,8 +77,7 @@ __device__ __forceinline__ void load_b6(const uint8_t *blk, int lg, B6 &b) {   /
 // Launches of a few jobs: the jobs as arguments, one block (the kernel's first and only parameter, at offset 0 of the argument
 // segment). A job is read at the grid row's offset of the segment, in the round trip that brings the arguments themselves (found
 // by its tile numbers it came a round trip later, 0.1 us a launch).
-constexpr int M6W_ROWS = 8;
-struct M6wArgs { MkJob j[M6W_ROWS]; };   // grid row i runs the gridDim.x tiles of j[i] from -j[i].tile0 on
+struct M6wArgs { MkJob j[GRID_ROWS]; };   // grid row i runs the gridDim.x tiles of j[i] from -j[i].tile0 on
 __device__ __forceinline__ MkJob m6w_job() {
     static_assert(sizeof(MkJob) % 4 == 0 && offsetof(M6wArgs, j) == 0, "jobs are read as dwords");
     constexpr int N = sizeof(MkJob) / 4;
@@ -240,22 +239,9 @@ hipError_t m6w_launch(int wn, int nw, bool keep, const MkJob *jobs, int njobs, c
     M6wArgs A{};
     dim3 g(grid);
     if (!jobs) {
-        // Grid rows of a common width (a multiple of 8, as every job's tiles are), a long job over several of them: of the widths
-        // that cut one job evenly, the one that leaves the fewest workgroups without a tile. One row per job made q, k and v of
-        // 2048, 512 and 512 rows x 2048 at 6 activations 384 workgroups for 192 with work, 7.8 us; in six rows of 32
-        // 5.3.
-        int tiles[M6W_INLINE], width = 0, least = 0;
+        int tiles[M6W_INLINE];   // (multiples of 8)
         for (int i = 0; i < njobs; i++) tiles[i] = (i + 1 < njobs ? hjobs[i + 1].tile0 : grid) - hjobs[i].tile0;
-        for (int i = 0; i < njobs; i++)
-            for (int k = 1; k <= M6W_ROWS; k++) {
-                const int w = ((tiles[i] + k - 1) / k + 7) / 8 * 8;
-                int rows = 0;
-                for (int q = 0; q < njobs; q++) rows += (tiles[q] + w - 1) / w;
-                if (rows <= M6W_ROWS && (!width || rows * w < least)) {
-                    width = w;
-                    least = rows * w;
-                }
-            }
+        const int width = grid_row_width(tiles, njobs, 8);
         int row = 0;
         for (int i = 0; i < njobs; i++)
             for (int t = 0; t < tiles[i]; t += width) {

@@ -788,7 +788,7 @@ __device__ __forceinline__ void mv_body(const MvJob &J, int order) {
 // records loaded them all: 0.6 us a launch).
 struct MvArgs {
     int order, pad;
-    MvJob j[MV_INLINE];   // grid row i runs j[i], tiles numbered from 0
+    MvJob j[GRID_ROWS];   // grid row i runs the gridDim.x tiles of j[i] from -j[i].tile0 on
 };
 __device__ __forceinline__ MvJob mv_job() {
     static_assert(sizeof(MvJob) % 4 == 0 && offsetof(MvArgs, j) % 4 == 0, "jobs are read as dwords");
@@ -1006,14 +1006,15 @@ hipError_t mv_launch(const MvLaunch &L, const MvJob *jobs, int njobs, const MvJo
         return hipGetLastError();
     }
     MvArgs A{order, 0, {}};
-    int most = 0;   // tiles of the longest job; a shorter one's workgroups past its rows have nothing to do
-    for (int i = 0; i < njobs; i++) {
-        A.j[i] = hjobs[i];
-        A.j[i].tile0 = 0;
-        const int tiles = (hjobs[i].r1 - hjobs[i].r0 + hjobs[i].rows_per_wg - 1) / hjobs[i].rows_per_wg;
-        most = tiles > most ? tiles : most;
-    }
-    hipLaunchKernelGGL(fn, dim3(most, njobs), dim3(WAVE * L.waves), L.lds, s, A);
+    int tiles[MV_INLINE], row = 0;
+    for (int i = 0; i < njobs; i++) tiles[i] = max(1, (hjobs[i].r1 - hjobs[i].r0 + hjobs[i].rows_per_wg - 1) / hjobs[i].rows_per_wg);
+    const int width = grid_row_width(tiles, njobs, 1);
+    for (int i = 0; i < njobs; i++)   // (workgroups past a job's rows have nothing to do)
+        for (int t = 0; t < tiles[i]; t += width) {
+            A.j[row] = hjobs[i];
+            A.j[row++].tile0 = -t;
+        }
+    hipLaunchKernelGGL(fn, dim3(width, row), dim3(WAVE * L.waves), L.lds, s, A);
     return hipGetLastError();
 }
 

@@ -251,6 +251,25 @@ print(json.dumps(out))
     assert r == []
 
 
+def test_decode_grid_rows(child):
+    """... and in decode launches: q, k and v of a layer"""
+    r = child(r"""
+shapes = ((C.c_long * 4) * 64).in_dll(S, "shapes")
+out = []
+for t, na in ((E.Q6_K, 1), (E.Q3_K, 4), (E.Q4_K, 1), (E.Q2_K, 1)):
+    grids = []
+    for rows in ((4096, 1024, 1024), (4096,), (1024,)):
+        p = L.plan([job(t, r, 4096, na, k) for k, r in enumerate(rows)])
+        reset()
+        p.run()
+        grids.append(shapes[0][0] * shapes[0][1])
+        p.close()
+    if counts[0] != 1 or grids[0] > 1.1 * (grids[1] + 2 * grids[2]): out.append([t, na, grids])
+print(json.dumps(out))
+""")
+    assert r == []
+
+
 MOE = r"""
 shapes = ((C.c_long * 4) * 64).in_dll(S, "shapes")
 def layer(types, n, ff, ne, k, N):   # the launches of a layer of N tokens
